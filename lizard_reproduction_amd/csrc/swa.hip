@@ -835,6 +835,390 @@ __global__ __launch_bounds__(64 * SWA_WALK_WAVES, 1) void swa_bwd_walk_kernel(
   }
 }
 
+// ----------------------------------------------------------------------------
+// backward in one pass for wider windows and d up to 128: a ring of waves, each
+// holding one 32-key block
+//
+// The workgroup's R waves walk the 32-row query blocks i of a segment s0 .. s1
+// - 1 of one (b, h).  Key block j belongs to wave j mod R for the NS steps i =
+// j .. j + NS - 1 whose queries' windows meet it (NS = (W + 30) / 32 + 1 < R):
+// its v rows stay in that wave's registers as MFMA operands and its dk, dv in
+// its accumulators, so only k (R slots of 32 rows), q, dy and ds go through
+// LDS.  In step i a wave has the role rho = (i - wave) mod R:
+//   rho < NS        scores key block i - rho.  Phase 1: S = q k^T, dP = dy v^T
+//                   (lane = key, registers = queries), p, and its keys' part of
+//                   delta = sum_t p dp, summed over the lanes (the fp32 form of
+//                   the two kernels above).  Phase 2: delta from the parts in
+//                   key order; ds = p (dp - delta); dv += p^T dY and dk += ds^T Q
+//                   with p and ds straight from the accumulator registers; ds^T
+//                   to LDS as bf16 [key][query].
+//   rho >= NS       dq tiles of query block i - 1 from its ds^T and the k slots:
+//                   tiles 0, 1, .. by rho = NS + 1, NS + 2, .. in phase 1, the
+//                   rest by rho = NS, NS + 1, .. in phase 2.  In phase 1 rho = NS
+//                   stores the dk, dv of the key block that has just left the
+//                   window and rho = R - 1 loads the v rows of the next one; in
+//                   phase 2 rho = R - 1 adds the terms of T.
+// Each score is formed once (5 products per pair; the two kernels form 9) and
+// every operand read once, but for the halo: the segment's first queries read
+// the NS - 1 key blocks before it, and the steps s1 .. s1 + NS - 2 run for the
+// dk, dv of its last key blocks only.  Two barriers per step; the next block's
+// k, q, dy rows are loaded a step ahead.
+// What bounds it: the chain of a step (7,000 cycles at d = 128: operands from
+// LDS, 32 dependent MFMAs and ~300 VALU instructions per wave, two barriers),
+// the tile loads landing inside it.  B=4 H=32 L=4096 d=128 W=128 backward 635 ->
+// 250 us (3.77 TB/s of its 940 MB), d=64 216 -> 173 us.
+// ----------------------------------------------------------------------------
+template <int DP, int R>
+struct SwaRing {
+  static constexpr int P = lds_pitch(DP);             // k, q, dy tiles [32][P]
+  static constexpr int TB = 32 * P * 2;
+  static constexpr int PS = 40;                       // ds^T tiles [32 keys][PS]: 80-byte rows
+                                                      // spread 8-byte writes over all banks
+  static constexpr int OFF_K = 0;                     // R k slots
+  static constexpr int OFF_Q = OFF_K + R * TB;        // two q buffers
+  static constexpr int OFF_DY = OFF_Q + 2 * TB;       // two dy buffers
+  static constexpr int OFF_DS = OFF_DY + 2 * TB;      // two sets of R ds^T slots
+  static constexpr int OFF_LSE = OFF_DS + 2 * R * 32 * PS * 2;   // [2][32] f32, log2 units
+  static constexpr int OFF_RED = OFF_LSE + 2 * 32 * 4;       // [R][32] f32 parts of delta
+  static constexpr int LDS = OFF_RED + R * 32 * 4;
+  static_assert(LDS <= 160 * 1024, "LDS budget");
+};
+
+// The largest NS a ring of R waves takes: two waves left for dq, stores and loads.
+constexpr int swa_ring_max_ns(int R) { return R - 2; }
+// The lane number, formed anew where it is used: the compiler cannot carry it,
+// or addresses made from it, over from an earlier use.
+__device__ __forceinline__ int fresh_lane() {
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+// s_waitcnt vmcnt(0) (gfx9 encoding; expcnt and lgkmcnt unconstrained)
+constexpr int WAIT_VM0 = 0x0F70;
+inline int swa_ring_ns(int W) { return (int)(((long long)W + 30) / 32 + 1); }
+
+// t[r] summed over the 32 lanes of a lane half: afterwards a lane holds the sum
+// of register r = lane mod 16.  Mirror and quad permutations pair each lane with
+// one that keeps the other half of the registers, halving the registers a lane
+// carries at every step (15 exchanges, no LDS).
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int N, int CTRL>
+__device__ __forceinline__ void lane_halve(float (&t)[16], bool upper) {
+#pragma unroll
+  for (int r = 0; r < N; ++r) {
+    const float keep = upper ? t[r + N] : t[r], give = upper ? t[r] : t[r + N];
+    t[r] = keep + dpp_move<CTRL>(give);
+  }
+}
+__device__ __forceinline__ float lane_sum16(float (&t)[16], int lane) {
+  lane_halve<8, 0x140>(t, lane & 8);   // row_mirror: lane ^ 15
+  lane_halve<4, 0x141>(t, lane & 4);   // row_half_mirror: lane ^ 7
+  lane_halve<2, 0x1B>(t, lane & 2);    // quad_perm [3,2,1,0]: lane ^ 3
+  lane_halve<1, 0xB1>(t, lane & 1);    // quad_perm [1,0,3,2]: lane ^ 1
+  const unsigned x = __float_as_uint(t[0]);
+  const auto sw = __builtin_amdgcn_permlane16_swap(x, x, false, false);   // + lane ^ 16
+  return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+
+// x[r] -= (v of lane r of this lane's 16-lane row), by DPP row broadcasts
+template <int R0 = 0>
+__device__ __forceinline__ void sub_row_bcast(f32x16& x, float v) {
+  if constexpr (R0 < 16) {
+    x[R0] -= dpp_move<0x150 + R0>(v);   // row_newbcast:R0
+    sub_row_bcast<R0 + 1>(x, v);
+  }
+}
+
+template <int DP, int R, typename OutT, bool VEC>
+__global__ __launch_bounds__(64 * R, 1) void swa_bwd_ring_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
+    const float* __restrict__ meta, int n_meta, const float* __restrict__ lse,
+    const bf16* __restrict__ dy, OutT* __restrict__ dq, OutT* __restrict__ dk,
+    OutT* __restrict__ dv, float* __restrict__ dmeta_part, int BH, int L, int d, int W,
+    float scale, int NB, int nseg, int NS, int per, int nx, int KG) {
+  using C = SwaRing<DP, R>;
+  constexpr int P = C::P, PS = C::PS, NDT = DP / 32, NT = 64 * R, ITEMS = 32 * DP / 8;
+  static_assert(ITEMS <= NT, "one item per thread and tile");
+  extern __shared__ __align__(16) char smem[];
+  auto kslot = [&](int s) { return reinterpret_cast<bf16*>(smem + C::OFF_K + s * C::TB); };
+  auto qbuf = [&](int i) { return reinterpret_cast<bf16*>(smem + C::OFF_Q + (i & 1) * C::TB); };
+  auto dybuf = [&](int i) { return reinterpret_cast<bf16*>(smem + C::OFF_DY + (i & 1) * C::TB); };
+  auto dsslot = [&](int i, int s) {
+    return reinterpret_cast<bf16*>(smem + C::OFF_DS) + ((i & 1) * R + s) * 32 * PS;
+  };
+  auto lsebuf = [&](int i) { return reinterpret_cast<float*>(smem + C::OFF_LSE) + (i & 1) * 32; };
+  float* red = reinterpret_cast<float*>(smem + C::OFF_RED);
+
+  const int lb = xcd_block(blockIdx.x, per, nx);
+  if (lb >= BH * nseg) return;
+  const int bh = lb / nseg, seg = lb % nseg;
+  const int nsub = (L + 31) / 32;
+  const int s0 = seg * NB, s1 = min(nsub, s0 + NB);
+  const int send = min(nsub, s1 + NS - 1);   // steps s0 .. send - 1
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane0 = threadIdx.x & 63;
+  const size_t base = (size_t)bh * L * d, kvbase = (size_t)(bh / KG) * L * d;
+  const bool vec = VEC || (d & 7) == 0;
+  const float c = scale * LOG2E;
+  const rsrc_t lse_r = make_rsrc(lse + (size_t)bh * L, (size_t)L * 4);
+
+  // one 16-byte item per thread (the first ITEMS) of a 32-row tile; rows
+  // outside [0, L) read zero
+  auto load_tile = [&](uint4& r, const bf16* src, int i, int tid) {
+    // threads past the tile, and blocks past the last step's (i < 0), read
+    // zeros: no branch around the loads
+    const int row = i >= 0 && (ITEMS == NT || tid < ITEMS) ? 32 * i + tid / (DP / 8) : -1;
+    r = gload8(src, row, (tid % (DP / 8)) * 8, L, d, vec);
+  };
+  auto store_tile = [&](const uint4& r, bf16* tile, int tid) {
+    if (ITEMS == NT || wave < ITEMS / 64)
+      *reinterpret_cast<uint4*>(tile + (tid / (DP / 8)) * P + (tid % (DP / 8)) * 8) = r;
+  };
+  auto load_lse = [&](int i, int tid) {   // every thread, row tid % 32: no branch around the load
+    const int r = 32 * i + (tid & 31);
+    return bload_f32(lse_r, r >= 0 && r < L ? (uint32_t)r * 4u : OOB);
+  };
+
+  uint4 pk, pq, pd;
+  float pl;
+  auto load_next = [&](int i, int tid) __attribute__((always_inline)) {
+    const int at = i < send ? i : -1;
+    load_tile(pk, k + kvbase, at, tid);
+    load_tile(pq, q + base, at, tid);
+    load_tile(pd, dy + base, at, tid);
+    pl = load_lse(at, tid);
+  };
+
+  bf16x8 vreg[DP / 16];
+  f32x16 dka[NDT], dva[NDT];
+#pragma unroll
+  for (int t = 0; t < NDT; ++t) {
+    dka[t] = zero16();
+    dva[t] = zero16();
+  }
+  if (threadIdx.x < R * 32) red[threadIdx.x] = 0.f;
+
+  // the first step's blocks: k of key blocks s0 - NS + 1 .. s0 (zero rows
+  // before the sequence), q, dy, lse of block s0, the v rows of its keys
+  int slot0 = s0 % R;            // ring slot (and wave) of key block i
+  int rho = slot0 - wave;        // role in step i
+  if (rho < 0) rho += R;
+  {
+    const int tid = threadIdx.x;
+    uint4 kr[swa_ring_max_ns(R)];
+#pragma unroll
+    for (int u = 0; u < swa_ring_max_ns(R); ++u)
+      if (u < NS) load_tile(kr[u], k + kvbase, s0 - u, tid);
+    load_tile(pq, q + base, s0, tid);
+    load_tile(pd, dy + base, s0, tid);
+    pl = load_lse(s0, tid);
+    if (rho < NS) own_rows<DP>(v + kvbase, 32 * (s0 - rho) + (lane0 & 31), L, d, lane0 >> 5, vec, vreg);
+#pragma unroll
+    for (int u = 0; u < swa_ring_max_ns(R); ++u)
+      if (u < NS) {
+        const int s = slot0 - u;
+        store_tile(kr[u], kslot(s < 0 ? s + R : s), tid);
+      }
+    store_tile(pq, qbuf(s0), tid);
+    store_tile(pd, dybuf(s0), tid);
+    lsebuf(s0)[tid & 31] = pl * LOG2E;
+    load_next(s0 + 1, tid);
+  }
+  float mmax = -1e30f;
+  for (int j = 0; j < n_meta; ++j) mmax = fmaxf(mmax, meta[j] * LOG2E);
+  float tpart = 0.f;
+  const int nh = R - NS;   // waves without a key block
+  __syncthreads();
+
+  // dq tile t (columns 32 t) of query block i - 1 from its ds^T and the k slots,
+  // the operands read one product ahead
+  auto dq_tile = [&](int i, int t) __attribute__((always_inline)) {
+    if (i == s0 || i - 1 >= s1) return;
+    const int lane = fresh_lane();
+    const int n = min(NS, i);   // key blocks i - n .. i - 1, from the left
+    int sl = slot0 - n;
+    if (sl < 0) sl += R;
+    bf16x8 a[2], b[2];
+    auto fetch = [&](int kb) __attribute__((always_inline)) {
+      b[kb] = tr_operand(dsslot(i - 1, sl), PS, 16 * kb, 0, lane);
+      a[kb] = tr_operand(kslot(sl), P, 16 * kb, 32 * t, lane);
+      __builtin_amdgcn_sched_barrier(0x0006);
+    };
+    f32x16 g = zero16();
+    fetch(0);
+#pragma unroll 1
+    for (int u = n; u > 0; --u) {
+      fetch(1);
+      g = mfma(a[0], b[0], g);
+      sl = sl + 1 == R ? 0 : sl + 1;
+      if (u > 1) fetch(0);
+      g = mfma(a[1], b[1], g);
+    }
+    store_acc_row<OutT>(dq + base, 32 * (i - 1) + (lane & 31), 32 * t, L, d, vec, g, scale,
+                        lane >> 5);
+  };
+
+  for (int i = s0;; ++i) {
+    // ---- phase 1 ---------------------------------------------------------------
+    // this step's lane addresses, formed anew: kept across the loop they took
+    // more registers than there are, and a spilled address's reload waits for
+    // the tile loads in flight
+    const int lane = fresh_lane(), col = lane & 31, h = lane >> 5, tid = 64 * wave + lane;
+    const int j = i - rho;   // this wave's key block (rho < NS), or the last one it had
+    const bool own = j >= s0 && j < s1;
+    // block i + 1 to LDS (its k slot is past the reach of this step's dq: NS <=
+    // R - 2), block i + 2 on its way.  Everything still in flight was issued in
+    // the step before; waiting for all of it here, before new loads and stores
+    // go out, lets no later wait in the step (the compiler's are exact only in
+    // straight code) catch this step's own.
+    __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    store_tile(pk, kslot(slot0 + 1 == R ? 0 : slot0 + 1), tid);
+    store_tile(pq, qbuf(i + 1), tid);
+    store_tile(pd, dybuf(i + 1), tid);
+    lsebuf(i + 1)[tid & 31] = pl * LOG2E;
+    load_next(i + 2, tid);
+    // a key block that has left the window, or that the sequence's end cut short
+    if (own && (rho == NS || (i == send && rho > 0 && rho < NS))) {
+#pragma unroll
+      for (int t = 0; t < NDT; ++t) {
+        store_acc_row<OutT>(dk + base, 32 * j + col, 32 * t, L, d, vec, dka[t], scale, h);
+        store_acc_row<OutT>(dv + base, 32 * j + col, 32 * t, L, d, vec, dva[t], 1.f, h);
+        dka[t] = zero16();
+        dva[t] = zero16();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (rho == R - 1 && i + 1 < send)
+      own_rows<DP>(v + kvbase, 32 * (i + 1) + col, L, d, h, vec, vreg);
+    f32x16 p, dp;
+    if (rho >= NS) {
+      if (rho > NS && rho - NS - 1 < NDT) dq_tile(i, rho - NS - 1);
+      if (i == send)   // no phase 2 follows
+        for (int t = rho - NS + nh - 1; t < NDT; t += nh) dq_tile(i, t);
+    } else if (i < send) {
+      float part = 0.f;
+      if (j >= 0) {
+        const bf16* q_l = qbuf(i);
+        const bf16* dy_l = dybuf(i);
+        const bf16* k_l = kslot(wave);
+        // two independent chains, their LDS operands read a product or
+        // two ahead (as the registers allow)
+        p = zero16();
+        dp = zero16();
+        constexpr int NK = DP / 16, PD = R > 8 || DP > 64 ? 1 : 2;
+        bf16x8 qa[PD + 1], ka[PD + 1], ya[PD + 1];
+        auto fetch = [&](int kb) __attribute__((always_inline)) {
+          const int x = kb % (PD + 1);
+          qa[x] = row_operand(q_l, P, col, 16 * kb, h);
+          ka[x] = row_operand(k_l, P, col, 16 * kb, h);
+          ya[x] = row_operand(dy_l, P, col, 16 * kb, h);
+        };
+#pragma unroll
+        for (int kb = 0; kb < PD; ++kb) fetch(kb);
+#pragma unroll
+        for (int kb = 0; kb < NK; ++kb) {
+          if (kb + PD < NK) fetch(kb + PD);
+          __builtin_amdgcn_sched_barrier(0x0006);
+          p = mfma(qa[kb % (PD + 1)], ka[kb % (PD + 1)], p);
+          dp = mfma(ya[kb % (PD + 1)], vreg[kb], dp);
+        }
+        // only blocks that straddle the window's start or the diagonal are
+        // masked (uniform per wave)
+        const int q0 = 32 * i, k0 = 32 * j;
+        const bool full = k0 + 31 <= q0 && k0 >= q0 + 32 - W;
+        const float* ll = lsebuf(i);
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const f32x4 ls = *reinterpret_cast<const f32x4*>(ll + 8 * g4 + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            p[4 * g4 + e] = __builtin_amdgcn_exp2f(fmaf(p[4 * g4 + e], c, -ls[e]));
+        }
+        if (!full) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            p[r] = in_window(q0 + acc_row(r, h), k0 + col, W) ? p[r] : 0.f;
+        }
+        float t[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r] = p[r] * dp[r];
+        part = lane_sum16(t, lane);
+      }
+      if ((lane & 16) == 0) red[rho * 32 + acc_row(lane & 15, h)] = part;
+    }
+    if (i == send) break;
+    __syncthreads();
+    // ---- phase 2 ---------------------------------------------------------------
+    if (rho < NS) {
+      if (j >= 0) {
+        const int lane = fresh_lane(), col = lane & 31, h = lane >> 5;
+        bf16x8 pb[2], dsb[2];
+        bf16* ds_l = dsslot(i, wave);
+        // lane n of a 16-lane row sums the parts of register n's query (parts
+        // past NS are zero), and hands it to the row as it is used
+        float del = 0.f;
+#pragma unroll
+        for (int u = swa_ring_max_ns(R) - 1; u >= 0; --u) del += red[u * 32 + acc_row(lane & 15, h)];
+        sub_row_bcast(dp, del);
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          bf16x4 d4;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * g4 + e;
+            d4[e] = to_bf16(p[r] * dp[r]);
+            pb[r >> 3][r & 7] = to_bf16(p[r]);
+            dsb[r >> 3][r & 7] = d4[e];
+          }
+          *reinterpret_cast<bf16x4*>(ds_l + col * PS + 8 * g4 + 4 * h) = d4;
+        }
+        if (own) {
+          const bf16* q_l = qbuf(i);
+          const bf16* dy_l = dybuf(i);
+#pragma unroll
+          for (int t = 0; t < NDT; ++t)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+              dva[t] = mfma(tr_operand(dy_l, P, 16 * kb, 32 * t, lane), pb[kb], dva[t]);
+              dka[t] = mfma(tr_operand(q_l, P, 16 * kb, 32 * t, lane), dsb[kb], dka[t]);
+            }
+        }
+      }
+    } else {
+      for (int t = rho - NS + nh - 1; t < NDT; t += nh) dq_tile(i, t);
+    }
+    if (rho == R - 1 && n_meta > 0) {
+      const int col = fresh_lane() & 31, h = fresh_lane() >> 5;
+      float del = 0.f;
+#pragma unroll
+      for (int u = swa_ring_max_ns(R) - 1; u >= 0; --u) del += red[u * 32 + col];
+      if (h == 0 && i < s1 && 32 * i + col < L)
+        tpart += __builtin_amdgcn_exp2f(mmax - lsebuf(i)[col]) * del;
+    }
+    slot0 = slot0 + 1 == R ? 0 : slot0 + 1;
+    rho = rho + 1 == R ? 0 : rho + 1;
+    __syncthreads();
+  }
+
+  // ---- this workgroup's T: one part per wave, summed in wave order ------------
+  if (n_meta > 0) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) tpart += __shfl_xor(tpart, off);
+    __syncthreads();   // every reader of red is past it
+    if ((threadIdx.x & 63) == 0) red[wave] = tpart;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < R; ++w) t += red[w];
+      dmeta_part[lb] = t;
+    }
+  }
+}
+
 // dmeta_j = -e^{meta_j - m} sum_w T_w, the workgroups' T summed in a fixed
 // order by one wave (strided lane sums, then a butterfly).  The lane's sink
 // logit and its first 16 partials are loaded together, before any is used
@@ -961,6 +1345,52 @@ static hipError_t launch_swa_bwd_walk(const void* q, const void* k, const void* 
   return hipGetLastError();
 }
 
+// 32-row blocks per segment of the ring walk: the split of a row into nseg
+// segments with the fewest steps in sequence, rounds of workgroups (one per
+// CU) times a segment's steps (its blocks, the NS - 1 of its halo, and about
+// three steps' time to start).  At least four blocks per segment: the workspace
+// holds one dmeta term per 128 rows.
+static int swa_ring_blocks(int BH, int L, int NS) {
+  const int nsub = (L + 31) / 32, cus = device_geom().cus;
+  int best = nsub;
+  long long least = -1;
+  for (int nseg = 1; nseg <= (nsub + 3) / 4; ++nseg) {
+    const int nb = (nsub + nseg - 1) / nseg;
+    if (nb < 4 && nseg > 1) break;
+    const long long rounds = ((long long)BH * ((nsub + nb - 1) / nb) + cus - 1) / cus;
+    const long long cost = rounds * (nb + NS + 2);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = nb;
+    }
+    if ((long long)BH * nseg > 4LL * cus) break;   // more segments only add halos
+  }
+  return best;
+}
+
+template <int DP, int R, typename OutT, bool VEC>
+static hipError_t launch_swa_bwd_ring(const void* q, const void* k, const void* v,
+                                      const float* meta, int n_meta, const float* lse,
+                                      const void* dy, void* dq, void* dk, void* dv,
+                                      float* dmeta_part, float* dmeta, int BH, int L, int d, int W,
+                                      float scale, int KG, hipStream_t st) {
+  constexpr int lds = SwaRing<DP, R>::LDS;
+  if (hipError_t e = ensure_lds<swa_bwd_ring_kernel<DP, R, OutT, VEC>>(lds); e != hipSuccess)
+    return e;
+  const int NS = swa_ring_ns(W), NB = swa_ring_blocks(BH, L, NS);
+  const int nseg = ((L + 31) / 32 + NB - 1) / NB;
+  const int nx = device_geom().xcds, grid = xcd_grid(BH * nseg, nx), per = grid / nx;
+  hipLaunchKernelGGL((swa_bwd_ring_kernel<DP, R, OutT, VEC>), dim3(grid), dim3(64 * R), lds, st,
+                     (const bf16*)q, (const bf16*)k, (const bf16*)v, meta, n_meta, lse,
+                     (const bf16*)dy, (OutT*)dq, (OutT*)dk, (OutT*)dv, dmeta_part, BH, L, d, W,
+                     scale, NB, nseg, NS, per, nx, KG);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || n_meta == 0) return e;
+  hipLaunchKernelGGL(swa_dmeta_reduce_kernel, dim3(1), dim3(64), 0, st,
+                     (const float*)dmeta_part, BH * nseg, meta, n_meta, dmeta);
+  return hipGetLastError();
+}
+
 template <int DP, typename OutT, bool VEC>
 static hipError_t launch_swa_bwd_t(const void* q, const void* k, const void* v, const float* meta,
                                    int n_meta, const float* lse, const void* dy, void* dq,
@@ -973,19 +1403,39 @@ static hipError_t launch_swa_bwd_t(const void* q, const void* k, const void* v, 
       return launch_swa_bwd_walk<OutT, VEC>(q, k, v, meta, n_meta, lse, dy, dq, dk, dv, dmeta_part,
                                             dmeta, BH, L, d, W, scale, KG, st);
   }
+  // wider windows at 32 < d <= 64 and all windows at 64 < d <= 128: the ring
+  // walk, where its waves cover the window's key blocks (W <= 161, and W <= 289
+  // at d <= 64).  Against the two kernels below (B=4 H=32 L=4096, us): d = 64
+  // W = 96 152 against 225, W = 289 290 against 351; d = 128 W = 1 214 against
+  // 378, W = 161 276 against 713.  At d <= 32 they stay the faster ones: W = 16
+  // 102 against 86, W = 64 115 against 107.
+  if constexpr (DP == 64 || DP == 128) {
+    const int NS = swa_ring_ns(W);
+    if (NS <= swa_ring_max_ns(8))
+      return launch_swa_bwd_ring<DP, 8, OutT, VEC>(q, k, v, meta, n_meta, lse, dy, dq, dk, dv,
+                                                   dmeta_part, dmeta, BH, L, d, W, scale, KG, st);
+    if constexpr (DP <= 64) {
+      if (NS <= swa_ring_max_ns(12))
+        return launch_swa_bwd_ring<DP, 12, OutT, VEC>(q, k, v, meta, n_meta, lse, dy, dq, dk, dv,
+                                                      dmeta_part, dmeta, BH, L, d, W, scale, KG,
+                                                      st);
+    }
+  }
   int per, grid, nx;
   swa_grid(BH, L, &per, &grid, &nx);
   // the window's key tiles fit the LDS slots of the resident form when a
   // block's keys span at most SWA_RES tiles: klo >= Q0 - W - 62, khi <= Q0 +
-  // SWA_ROWS, so SWA_ROWS + W + 62 <= SWA_RES * SWA_TILE; and at d <= 64,
-  // where the slots leave the kernel's workgroups per CU in place
-  const bool res = DP <= 64 && SWA_ROWS + W + 62 <= SWA_RES * SWA_TILE;
+  // SWA_ROWS, so SWA_ROWS + W + 62 <= SWA_RES * SWA_TILE (at d <= 32; wider
+  // heads with such windows took a walk above)
+  constexpr bool CAN_RES = DP <= 32;
+  const bool res = CAN_RES && SWA_ROWS + W + 62 <= SWA_RES * SWA_TILE;
   hipError_t e;
   const size_t lds_q = 2 * (res ? SWA_RES : 1) * SwaCfg<DP>::TILE_BYTES +
                        4 * SWA_META_BLOCK * sizeof(float);
   if (res) {
-    if ((e = ensure_lds<swa_bwd_dq_kernel<DP, OutT, VEC, true>>((int)lds_q)) != hipSuccess) return e;
-    hipLaunchKernelGGL((swa_bwd_dq_kernel<DP, OutT, VEC, true>), dim3(grid), dim3(256), lds_q, st,
+    if ((e = ensure_lds<swa_bwd_dq_kernel<DP, OutT, VEC, CAN_RES>>((int)lds_q)) != hipSuccess)
+      return e;
+    hipLaunchKernelGGL((swa_bwd_dq_kernel<DP, OutT, VEC, CAN_RES>), dim3(grid), dim3(256), lds_q, st,
                        (const bf16*)q, (const bf16*)k, (const bf16*)v, meta, n_meta, lse,
                        (const bf16*)dy, (OutT*)dq, delta, dmeta_part, BH, L, d, W, scale, per, nx,
                        KG);

@@ -117,3 +117,24 @@ def test_swa_many_sinks_match_oracle(sinks, dim):
     compare(lambda q, k, v, m: kernels.swa(q, k, v, m, 48),
             lambda q, k, v, m: lo.swa_kernel_api(q, k, v, m, 48, dtype=torch.float32),
             inputs, grad, label=f"{sinks} sinks d={dim}")
+
+
+# The ring walk's edges: W = 161 is the widest window eight waves take and 162
+# the first of twelve (at d <= 64; at d = 128 the two kernels), 289 and 290
+# likewise for twelve; W = 97 and 98 meet four and five 32-key blocks.  Lengths
+# end inside a block, on one, inside the first segment's window, and cut the
+# last segment's halo short; few rows give segments of four blocks.
+@pytest.mark.parametrize("length, window, dim, heads, fp32", [
+    (700, 65, 64, 3, False), (700, 97, 64, 3, True), (703, 98, 128, 3, False),
+    (640, 161, 128, 2, False), (640, 162, 128, 2, False), (641, 162, 64, 2, False),
+    (450, 289, 40, 2, False), (450, 290, 64, 2, False), (300, 64, 128, 2, True),
+    (31, 128, 128, 2, False), (130, 1, 96, 2, False), (290, 128, 30, 3, False),
+    (300, 200, 20, 2, True), (1100, 128, 100, 64, False)])
+def test_swa_wide_window_backward_matches_oracle(length, window, dim, heads, fp32):
+    inputs = swa_inputs(length, batch=1, heads=heads, dim=dim, seed=window)
+    if fp32:
+        inputs = [t.float() for t in inputs[:3]] + [inputs[3]]
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(1))
+    compare(lambda q, k, v, m: kernels.swa(q, k, v, m, window),
+            lambda q, k, v, m: lo.swa_kernel_api(q, k, v, m, window, dtype=torch.float32),
+            inputs, grad, label=f"L={length} W={window} d={dim} H={heads}")
