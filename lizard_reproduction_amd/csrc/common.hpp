@@ -109,13 +109,13 @@ __device__ __forceinline__ bf16x4 load4(const bf16* __restrict__ p, int row, int
 }
 
 // Store 4 consecutive fp32 values as OutT (bf16 or float) at [row][c..c+4),
-// clipped to ncols.
+// clipped to ncols (rows `pitch` elements apart).
 template <typename OutT>
-__device__ __forceinline__ void store4(OutT* __restrict__ p, int row, int c, int ncols,
+__device__ __forceinline__ void store4(OutT* __restrict__ p, int row, int c, int ncols, int pitch,
                                        float a, float b, float cc, float d) {
   float v[4] = {a, b, cc, d};
-  OutT* q = p + (size_t)row * ncols + c;
-  if (c + 3 < ncols && (ncols & 3) == 0) {
+  OutT* q = p + (size_t)row * pitch + c;
+  if (c + 3 < ncols && (pitch & 3) == 0) {
     if constexpr (sizeof(OutT) == 2) {
       bf16x4 o;
 #pragma unroll
@@ -215,6 +215,14 @@ inline DevGeom device_geom() {
 __host__ __device__ constexpr int xcd_grid(int total, int X) { return X * ((total + X - 1) / X); }
 __device__ __forceinline__ int xcd_block(int i, int per, int X) {
   return (i % X) * per + i / X;
+}
+
+// The lane number, formed anew where it is used: the compiler cannot carry it,
+// or addresses made from it, over from an earlier use.
+__device__ __forceinline__ int fresh_lane() {
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
 }
 
 // Exchange with the other half of the wave (lane ^ 32).
@@ -343,6 +351,12 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, size_t bytes) {
                                            (int)(uint32_t)(bytes < OOB ? bytes : OOB), RSRC_WORD3);
 }
 
+// Bytes of nrows bf16 rows of ncols elements, `pitch` elements apart: to the
+// end of the last row, so that an offset of a row past it is out of range.
+__device__ __forceinline__ size_t pitched_bytes(int nrows, int ncols, int pitch) {
+  return ((size_t)(nrows - 1) * pitch + ncols) * 2;
+}
+
 // AUX: the load's cache policy (LOAD_NT: nontemporal, for data that nothing
 // reads again soon)
 constexpr int LOAD_NT = 2;
@@ -358,17 +372,18 @@ __device__ __forceinline__ float bload_f32(rsrc_t r, uint32_t off) {
 // Columns [c, c+8) of row `row` of a row-major [nrows x ncols] bf16 matrix
 // behind resource r, zero outside it (rows < 0 or >= nrows included).
 // Vector form (ncols % 8 == 0): an item is wholly inside or outside a row.
+// pitch: elements from one row to the next (at least ncols).
 template <int AUX = 0>
-__device__ __forceinline__ uint4 bload8_vec(rsrc_t r, int row, int c, int ncols) {
-  return bload16<AUX>(r, (row >= 0 && c < ncols) ? (uint32_t)(row * ncols + c) * 2u : OOB);
+__device__ __forceinline__ uint4 bload8_vec(rsrc_t r, int row, int c, int ncols, int pitch) {
+  return bload16<AUX>(r, (row >= 0 && c < ncols) ? (uint32_t)(row * pitch + c) * 2u : OOB);
 }
 
 // Element form for any ncols: eight 2-byte loads.
-__device__ __forceinline__ uint4 bload8_elem(rsrc_t r, int row, int c, int ncols) {
+__device__ __forceinline__ uint4 bload8_elem(rsrc_t r, int row, int c, int ncols, int pitch) {
   bf16x8 v;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const uint32_t off = (row >= 0 && c + e < ncols) ? (uint32_t)(row * ncols + c + e) * 2u : OOB;
+    const uint32_t off = (row >= 0 && c + e < ncols) ? (uint32_t)(row * pitch + c + e) * 2u : OOB;
     v[e] = __builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
   }
   return __builtin_bit_cast(uint4, v);
@@ -378,7 +393,7 @@ __device__ __forceinline__ uint4 bload8_elem(rsrc_t r, int row, int c, int ncols
 __device__ __forceinline__ uint4 gload8(const bf16* __restrict__ base, int row, int c, int nrows,
                                         int ncols, bool vec) {
   const rsrc_t r = make_rsrc(base, (size_t)nrows * ncols * 2);
-  return vec ? bload8_vec(r, row, c, ncols) : bload8_elem(r, row, c, ncols);
+  return vec ? bload8_vec(r, row, c, ncols, ncols) : bload8_elem(r, row, c, ncols, ncols);
 }
 
 // Row `row`, columns c0 .. c0+31 of a row-major [nrows x ncols] bf16 matrix
@@ -387,10 +402,11 @@ __device__ __forceinline__ uint4 gload8(const bf16* __restrict__ base, int row, 
 // matrix column c0 + acc_row(k, h)), times `scale`; rows past nrows are
 // dropped.  A permlane32 swap between the two lane halves first gives half h
 // the runs c0 + 16 j + 8 h + {0..7} (j = 0, 1), so each lane writes two
-// 16-byte pieces (vec: ncols % 8 == 0) rather than four 8-byte ones.
+// 16-byte pieces (vec: ncols % 8 == 0) rather than four 8-byte ones.  pitch:
+// elements from one row to the next.
 template <int AUX = 0>
-__device__ __forceinline__ void store_acc_row_bf16(rsrc_t r, int row, int c0, int ncols, bool vec,
-                                                   const f32x16& o, float scale, int h) {
+__device__ __forceinline__ void store_acc_row_bf16(rsrc_t r, int row, int c0, int ncols, int pitch,
+                                                   bool vec, const f32x16& o, float scale, int h) {
   uint32_t w[8];   // w[2g], w[2g+1]: rows 8g + 4h + {0..3} of the tile, as bf16 pairs
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -415,13 +431,13 @@ __device__ __forceinline__ void store_acc_row_bf16(rsrc_t r, int row, int c0, in
     if (vec) {
       const u32x4 v = {w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]};
       __builtin_amdgcn_raw_buffer_store_b128(
-          v, r, (row >= 0 && col < ncols) ? (uint32_t)(row * ncols + col) * 2u : OOB, 0, AUX);
+          v, r, (row >= 0 && col < ncols) ? (uint32_t)(row * pitch + col) * 2u : OOB, 0, AUX);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const uint16_t x = (uint16_t)(w[4 * j + (e >> 1)] >> (16 * (e & 1)));
         __builtin_amdgcn_raw_buffer_store_b16(
-            x, r, (row >= 0 && col + e < ncols) ? (uint32_t)(row * ncols + col + e) * 2u : OOB, 0,
+            x, r, (row >= 0 && col + e < ncols) ? (uint32_t)(row * pitch + col + e) * 2u : OOB, 0,
             AUX);
       }
     }
@@ -434,44 +450,53 @@ __device__ __forceinline__ void store_acc_row_bf16(rsrc_t r, int row, int c0, in
 // (the bf16 form swaps registers between lane halves); rows below 0 or at or
 // past nrows are skipped (bf16: dropped by the buffer range check).
 template <typename OutT>
-__device__ __forceinline__ void store_acc_row(OutT* __restrict__ base, int row, int c0, int nrows,
-                                              int ncols, bool vec, const f32x16& g, float scale,
-                                              int h) {
+__device__ __forceinline__ void store_acc_row_pitched(OutT* __restrict__ base, int row, int c0,
+                                                      int nrows, int ncols, int pitch, bool vec,
+                                                      const f32x16& g, float scale, int h) {
   if constexpr (sizeof(OutT) == 2) {
-    store_acc_row_bf16(make_rsrc(base, (size_t)nrows * ncols * 2), row, c0, ncols, vec, g, scale,
-                       h);
+    store_acc_row_bf16(make_rsrc(base, pitched_bytes(nrows, ncols, pitch)), row, c0, ncols, pitch,
+                       vec, g, scale, h);
   } else {
     if (row >= 0 && row < nrows) {
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4)
-        store4<OutT>(base, row, c0 + 8 * g4 + 4 * h, ncols, g[4 * g4] * scale,
+        store4<OutT>(base, row, c0 + 8 * g4 + 4 * h, ncols, pitch, g[4 * g4] * scale,
                      g[4 * g4 + 1] * scale, g[4 * g4 + 2] * scale, g[4 * g4 + 3] * scale);
     }
   }
+}
+
+// the same for rows that follow each other (pitch = ncols)
+template <typename OutT>
+__device__ __forceinline__ void store_acc_row(OutT* __restrict__ base, int row, int c0, int nrows,
+                                              int ncols, bool vec, const f32x16& g, float scale,
+                                              int h) {
+  store_acc_row_pitched<OutT>(base, row, c0, nrows, ncols, ncols, vec, g, scale, h);
 }
 
 // Items idx = threadIdx.x + NT i (i < N, idx < ITEMS) of a [rows x KP/8]
 // grid of 8-column items starting at row r0: item idx covers row
 // r0 + idx / (KP/8), columns 8 (idx % (KP/8)).  The uniform `vec` test sits
 // outside the unrolled loop, so the vector form is straight-line loads.
+// Rows are `pitch` elements apart.
 template <int KP, int NT, int N, int ITEMS, int AUX = 0>
 __device__ __forceinline__ void load_items(uint4 (&reg)[N], const bf16* __restrict__ base, int r0,
-                                           int nrows, int ncols, bool vec) {
+                                           int nrows, int ncols, bool vec, int pitch) {
   constexpr int K8 = KP / 8;
-  const rsrc_t r = make_rsrc(base, (size_t)nrows * ncols * 2);
+  const rsrc_t r = make_rsrc(base, pitched_bytes(nrows, ncols, pitch));
   if (vec) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int idx = threadIdx.x + NT * i;
       if (ITEMS % NT == 0 || idx < ITEMS)
-        reg[i] = bload8_vec<AUX>(r, r0 + idx / K8, (idx % K8) * 8, ncols);
+        reg[i] = bload8_vec<AUX>(r, r0 + idx / K8, (idx % K8) * 8, ncols, pitch);
     }
   } else {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int idx = threadIdx.x + NT * i;
       if (ITEMS % NT == 0 || idx < ITEMS)
-        reg[i] = bload8_elem(r, r0 + idx / K8, (idx % K8) * 8, ncols);
+        reg[i] = bload8_elem(r, r0 + idx / K8, (idx % K8) * 8, ncols, pitch);
     }
   }
 }

@@ -66,8 +66,8 @@ constexpr int B_THREADS = 64 * B_WAVES;
 // outside the matrix; items past the tile are skipped.
 template <int KP, int N>
 __device__ __forceinline__ void load_tile8(uint4 (&reg)[N], const bf16* __restrict__ base, int t0,
-                                           int L, int ncols, bool vec) {
-  load_items<KP, B_THREADS, N, GLA_C * KP / 8>(reg, base, t0, L, ncols, vec);
+                                           int L, int ncols, bool vec, int pitch) {
+  load_items<KP, B_THREADS, N, GLA_C * KP / 8>(reg, base, t0, L, ncols, vec, pitch);
 }
 
 template <int KP, int N>
@@ -135,6 +135,34 @@ struct BwdA : BwdCommon<FP, DP> {
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
 
+// dy of (b, h)
+__device__ __forceinline__ size_t dy_offset(const GlaRows& rows, int bh, int H, int L) {
+  if (rows.ldy == rows.ld && rows.hsy == L * rows.ld) return (size_t)bh * L * rows.ld;
+  return (size_t)(bh / H) * H * L * rows.ld + (size_t)(bh % H) * rows.hsy;
+}
+
+// The rows as the walk of FP features takes them: only the widest is launched on
+// columns of wider rows (GlaPart); for the others they follow each other, known
+// when compiled (as arguments, the pitches spilled 15 more scalar registers of
+// the F = D = 128 backward: 871 -> 874 us for the headline's fwd+bwd).
+template <int FP>
+__device__ __forceinline__ GlaRows walk_rows(const GlaRows& given, int L, int D) {
+  if constexpr (FP == 256)
+    return given;
+  else
+    return GlaRows{D, D, L * D};
+}
+
+// Columns [f, f + 4) of row `tok` of the fp32 [L, F] sums of (b, h) (at `off`)
+// that a D tile adds to, zero outside or with no sums yet (F % 4 == 0)
+__device__ __forceinline__ f32x4 part_in(const float* __restrict__ sums, size_t off, int tok, int f,
+                                         int L, int F) {
+  if (!sums) return f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint4 x = bload16(make_rsrc(sums + off, (size_t)L * F * 4),
+                          f < F ? (uint32_t)(tok * F + f) * 4u : OOB);
+  return __builtin_bit_cast(f32x4, x);
+}
+
 // qz[lane] = qs_lane (fq_lane . z) over features [f0, f0 + NF) (query = lane)
 template <int NF>
 __device__ __forceinline__ void qz_part(const bf16* fq_l, int pitch, const float* zs,
@@ -170,13 +198,15 @@ __device__ __forceinline__ void z_update(float* zn, const float* zs, const float
 // formed from this tile's features but read from den_out / delta_out, where
 // the caller has put those of the whole feature dimension; the kernel then
 // writes this tile's share of every gradient.
-template <int FP, int DP, typename OutT, bool VEC, bool EXT, bool FOLD = false>
+template <int FP, int DP, typename OutT, bool VEC, bool EXT, bool FOLD = false, bool PART = false>
 __device__ __forceinline__ void gla_bwd_dq_body(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy, OutT* __restrict__ dfq,
     float* __restrict__ den_out, float* __restrict__ delta_out, float* __restrict__ p_out,
-    const float* __restrict__ seg_state, int H, int L, int F, int D, int gate, int G,
-    int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam) {
+    const float* __restrict__ seg_state, int H, int L, int F, int D, GlaRows given, int gate, int G,
+    int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam,
+    GlaPart part) {
+  const GlaRows rows = walk_rows<FP>(given, L, D);
   using Cfg = BwdA<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT;
@@ -217,9 +247,10 @@ __device__ __forceinline__ void gla_bwd_dq_body(
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
-  const size_t offF = (size_t)bh * L * F, offD = (size_t)bh * L * D, offL = (size_t)bh * L;
+  const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
+  const size_t offDy = dy_offset(rows, bh, H, L);
   // fk and v of the kv head of this query head (KG query heads share one)
-  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * D;
+  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * rows.ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the forward state entering segment seg: its scanned record, or (FOLD) the
   // local records of segments 0 .. seg - 1 folded here (their total log
@@ -321,10 +352,10 @@ __device__ __forceinline__ void gla_bwd_dq_body(
   auto issue = [&](auto set, int n) __attribute__((always_inline)) {
     constexpr int S = decltype(set)::value;
     if (n < n1) {
-      load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF);
-      load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF);
-      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD);
-      load_tile8<DP>(rd[S], dy + offD, n * C, L, D, vecD);
+      load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF, F);
+      load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF, F);
+      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, rows.ld);
+      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, rows.ldy);
       if (wave == GW) {
         rg[S] = gate_at(lgb, n * C + lane, L);
         rgok[S] = n * C + lane < L;
@@ -512,12 +543,38 @@ __device__ __forceinline__ void gla_bwd_dq_body(
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * g4 + e;
             g[r] += qsd * (X[j][r] - z4[e] * delta);
-            ps += to_f32(f4[e]) * g[r];
+            if constexpr (!PART) ps += to_f32(f4[e]) * g[r];
+          }
+        }
+        if constexpr (PART) {
+          // the tiles' sums so far, loaded once X is used up (loaded above,
+          // beside X, they spilled the F = 256 walk: 114 against 92 us)
+          __builtin_amdgcn_sched_barrier(0);
+          const int ln = fresh_lane(), h = ln >> 5, q = hq * 32 + (ln & 31), tok = t0 + q;
+          f32x4 add[4];
+#pragma unroll
+          for (int g4 = 0; g4 < 4; ++g4)
+            add[g4] = part_in(part.dfq_in, offF, tok, ft * 32 + 8 * g4 + 4 * h, L, F);
+#pragma unroll
+          for (int g4 = 0; g4 < 4; ++g4) {
+            const bf16x4 f4 =
+                *reinterpret_cast<const bf16x4*>(fq_l + q * PF + ft * 32 + 8 * g4 + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              g[4 * g4 + e] += add[g4][e];
+              ps += to_f32(f4[e]) * g[4 * g4 + e];
+            }
           }
         }
         ps += xhalf(ps);
         if (h == 0) pp[ft * 64 + q] = tok < L ? ps : 0.f;
-        store_acc_row<OutT>(dfq + offF, tok, ft * 32, L, F, vecF, g, 1.f, h);
+        if (PART && part.dfq_out) {
+          const int ln = fresh_lane();
+          store_acc_row<float>(part.dfq_out + offF, t0 + hq * 32 + (ln & 31), ft * 32, L, F, vecF, g,
+                               1.f, ln >> 5);
+        } else {
+          store_acc_row<OutT>(dfq + offF, tok, ft * 32, L, F, vecF, g, 1.f, h);
+        }
       }
     }
     // S^T <- r S^T + V^T K~ for the owned tiles
@@ -551,16 +608,17 @@ __device__ __forceinline__ void gla_bwd_dq_body(
   }
 }
 
-template <int FP, int DP, typename OutT, bool VEC, bool EXT, bool FOLD = false>
+template <int FP, int DP, typename OutT, bool VEC, bool EXT, bool FOLD = false, bool PART = false>
 __global__ __launch_bounds__(B_THREADS, 1) void gla_bwd_dq_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy, OutT* __restrict__ dfq,
     float* __restrict__ den_out, float* __restrict__ delta_out, float* __restrict__ p_out,
-    const float* __restrict__ seg_state, int H, int L, int F, int D, int gate, int G,
-    int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam) {
-  gla_bwd_dq_body<FP, DP, OutT, VEC, EXT, FOLD>(fq, fk, v, log_gamma, dy, dfq, den_out, delta_out,
-                                                 p_out, seg_state, H, L, F, D, gate, G, cps, M,
-                                                 KG, xper, nxcd, nblk, seg_lam);
+    const float* __restrict__ seg_state, int H, int L, int F, int D, GlaRows rows, int gate, int G,
+    int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam,
+    GlaPart part) {
+  gla_bwd_dq_body<FP, DP, OutT, VEC, EXT, FOLD, PART>(
+      fq, fk, v, log_gamma, dy, dfq, den_out, delta_out, p_out, seg_state, H, L, F, D, rows, gate, G,
+      cps, M, KG, xper, nxcd, nblk, seg_lam, part);
 }
 
 // ============================================================================
@@ -650,7 +708,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ dy, const float* __restrict__ log_gamma,
     const float* __restrict__ den_in, const float* __restrict__ delta_in,
     float* __restrict__ seg_state, float* __restrict__ seg_logdecay, int H, int L, int F, int D,
-    int gate, int G, int cps) {
+    GlaRows given, int gate, int G, int cps) {
+  const GlaRows rows = walk_rows<FP>(given, L, D);
   using Cfg = BwdS<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT, NTILE = NFT * NDT, TPW = (NTILE + 3) / 4;
@@ -674,7 +733,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
-  const size_t offF = (size_t)bh * L * F, offD = (size_t)bh * L * D, offL = (size_t)bh * L;
+  const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
+  const size_t offDy = dy_offset(rows, bh, H, L);
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
 
   f32x16 dS[TPW];
@@ -685,8 +745,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
 
   uint4 rq[Cfg::NLF], rd[Cfg::NLD];
   TokScalars sc;
-  load_chunk<FP>(rq, fq + offF, (n1 - 1) * C, L, F, vecF);
-  load_chunk<DP>(rd, dy + offD, (n1 - 1) * C, L, D, vecD);
+  load_chunk<FP>(rq, fq + offF, (n1 - 1) * C, L, F, vecF, F);
+  load_chunk<DP>(rd, dy + offDy, (n1 - 1) * C, L, D, vecD, rows.ldy);
   sc = load_scalars(lgb, den_in, delta_in, nullptr, offL, (n1 - 1) * C + lane, L);
   store_chunk<FP>(rq, fq_l, PF);
   store_chunk<DP>(rd, dy_l, PD);
@@ -697,8 +757,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
   for (int n = n1 - 1; n >= n0; --n) {
     const bool more = n - 1 >= n0;
     if (more) {
-      load_chunk<FP>(rq, fq + offF, (n - 1) * C, L, F, vecF);
-      load_chunk<DP>(rd, dy + offD, (n - 1) * C, L, D, vecD);
+      load_chunk<FP>(rq, fq + offF, (n - 1) * C, L, F, vecF, F);
+      load_chunk<DP>(rd, dy + offDy, (n - 1) * C, L, D, vecD, rows.ldy);
       sc = load_scalars(lgb, den_in, delta_in, nullptr, offL, (n - 1) * C + lane, L);
     }
     // dz partials sum_i fq_i (qh_i delta_i)
@@ -813,7 +873,7 @@ struct BwdB : BwdCommon<FP, DP> {
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
 
-template <int FP, int DP, typename OutT, bool VEC, bool FOLD = false>
+template <int FP, int DP, typename OutT, bool VEC, bool FOLD = false, bool PART = false>
 __device__ __forceinline__ void gla_bwd_dkv_body(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy,
@@ -821,8 +881,9 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
     const float* __restrict__ p_in, OutT* __restrict__ dfk, OutT* __restrict__ dv,
     float* __restrict__ dG, float* __restrict__ csum, float* __restrict__ dlg_direct,
     const float* __restrict__ seg_state, int H,
-    int L, int F, int D, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
-    int nblk, const float* __restrict__ seg_lam, int rev) {
+    int L, int F, int D, GlaRows given, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
+    int nblk, const float* __restrict__ seg_lam, int rev, GlaPart part) {
+  const GlaRows rows = walk_rows<FP>(given, L, D);
   using Cfg = BwdB<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT, ZP = Cfg::ZP;
@@ -859,9 +920,10 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
-  const size_t offF = (size_t)bh * L * F, offD = (size_t)bh * L * D, offL = (size_t)bh * L;
+  const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
+  const size_t offDy = dy_offset(rows, bh, H, L);
   // fk and v of the kv head of this query head (KG query heads share one)
-  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * D;
+  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * rows.ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the gradient state entering segment seg from the right: its scanned
   // record, or (FOLD) the local records of segments G - 1 .. seg + 1 folded
@@ -938,10 +1000,10 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
   auto issue = [&](auto set, int n) __attribute__((always_inline)) {
     constexpr int S = decltype(set)::value;
     if (n >= n0) {
-      load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF);
-      load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF);
-      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD);
-      load_tile8<DP>(rd[S], dy + offD, n * C, L, D, vecD);
+      load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF, F);
+      load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF, F);
+      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, rows.ld);
+      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, rows.ldy);
       if (wave == SCW) sc[S] = load_scalars(lgb, den_in, delta_in, p_in, offL, n * C + lane, L);
     }
   };
@@ -1077,7 +1139,8 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
         for (int qb = 0; qb < 4; ++qb)   // keys 32-63 have no queries in blocks 0, 1
           if (hk == 0 || qb >= 2)
             g = mfma(tr_operand(dy_l, PD, 16 * qb, dt * 32, lane), fa[(hk * 4 + qb) * 64 + lane], g);
-        store_acc_row<OutT>(dv + offD, t0 + key, dt * 32, L, D, vecD, g, 1.f, h);
+        store_acc_row_pitched<OutT>(dv + (size_t)bh * L * rows.ld, t0 + key, dt * 32, L, D, rows.ld,
+                                    vecD, g, 1.f, h);
       }
     }
     // dS <- r_n dS + Q^T dy for the owned tiles, Q^ = bf16(qh fq): the owned
@@ -1128,16 +1191,22 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
           const int f0 = ft * 32 + 8 * g4 + 4 * h;
           const bf16x4 k4 = *reinterpret_cast<const bf16x4*>(fk_l + key * PF + f0);
           const f32x4 z4 = *reinterpret_cast<const f32x4*>(dzs + f0);
+          f32x4 add = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (PART) add = part_in(part.dfk_in, offF, tok, f0, L, F);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * g4 + e;
             g[r] += ksv * (x[r] - z4[e]);
+            if constexpr (PART) g[r] += add[e];
             pks += to_f32(k4[e]) * g[r];
           }
         }
         pks += xhalf(pks);
         if (h == 0) pk[ft * 64 + key] = pks;
-        store_acc_row<OutT>(dfk + offF, tok, ft * 32, L, F, vecF, g, 1.f, h);
+        if (PART && part.dfk_out)
+          store_acc_row<float>(part.dfk_out + offF, tok, ft * 32, L, F, vecF, g, 1.f, h);
+        else
+          store_acc_row<OutT>(dfk + offF, tok, ft * 32, L, F, vecF, g, 1.f, h);
       }
     }
     __syncthreads();
@@ -1179,7 +1248,7 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
   }
 }
 
-template <int FP, int DP, typename OutT, bool VEC, bool FOLD = false>
+template <int FP, int DP, typename OutT, bool VEC, bool FOLD = false, bool PART = false>
 __global__ __launch_bounds__(B_THREADS, (BwdB<FP, DP>::LB)) void gla_bwd_dkv_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy,
@@ -1187,33 +1256,33 @@ __global__ __launch_bounds__(B_THREADS, (BwdB<FP, DP>::LB)) void gla_bwd_dkv_ker
     const float* __restrict__ p_in, OutT* __restrict__ dfk, OutT* __restrict__ dv,
     float* __restrict__ dG, float* __restrict__ csum, float* __restrict__ dlg_direct,
     const float* __restrict__ seg_state, int H,
-    int L, int F, int D, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
-    int nblk, const float* __restrict__ seg_lam, int rev) {
-  gla_bwd_dkv_body<FP, DP, OutT, VEC, FOLD>(fq, fk, v, log_gamma, dy, den_in, delta_in, p_in, dfk,
-                                            dv, dG, csum, dlg_direct, seg_state, H, L, F, D, gate,
-                                            G, cps, M, KG, xper, nxcd, nblk, seg_lam, rev);
+    int L, int F, int D, GlaRows rows, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
+    int nblk, const float* __restrict__ seg_lam, int rev, GlaPart part) {
+  gla_bwd_dkv_body<FP, DP, OutT, VEC, FOLD, PART>(
+      fq, fk, v, log_gamma, dy, den_in, delta_in, p_in, dfk, dv, dG, csum, dlg_direct, seg_state, H,
+      L, F, D, rows, gate, G, cps, M, KG, xper, nxcd, nblk, seg_lam, rev, part);
 }
 
 // One segment per (b, h): the dq walk and then the dkv walk of the same
 // (b, h) in one workgroup.  The dkv walk starts on the chunks the dq walk
 // read last, still in the caches, and needs only this workgroup's own den,
 // delta and p rows (a workgroup-scope fence and barrier order them).
-template <int FP, int DP, typename OutT, bool VEC>
+template <int FP, int DP, typename OutT, bool VEC, bool PART = false>
 __global__ __launch_bounds__(B_THREADS, 1) void gla_bwd_fused_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy, OutT* __restrict__ dfq,
     OutT* __restrict__ dfk, OutT* __restrict__ dv, float* __restrict__ den,
     float* __restrict__ delta, float* __restrict__ p, float* __restrict__ dG,
     float* __restrict__ csum, float* __restrict__ dlg_direct, int H, int L, int F, int D,
-    int gate, int cps, int KG, int xper, int nxcd, int nblk) {
-  gla_bwd_dq_body<FP, DP, OutT, VEC, false>(fq, fk, v, log_gamma, dy, dfq, den, delta, p, nullptr,
-                                            H, L, F, D, gate, 1, cps, 1, KG, xper, nxcd, nblk,
-                                            nullptr);
+    GlaRows rows, int gate, int cps, int KG, int xper, int nxcd, int nblk, GlaPart part) {
+  gla_bwd_dq_body<FP, DP, OutT, VEC, false, false, PART>(
+      fq, fk, v, log_gamma, dy, dfq, den, delta, p, nullptr, H, L, F, D, rows, gate, 1, cps, 1, KG,
+      xper, nxcd, nblk, nullptr, part);
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   __syncthreads();
-  gla_bwd_dkv_body<FP, DP, OutT, VEC>(fq, fk, v, log_gamma, dy, den, delta, p, dfk, dv, dG, csum,
-                                      dlg_direct, nullptr, H, L, F, D, gate, 1, cps, 1, KG, xper,
-                                      nxcd, nblk, nullptr, 0);
+  gla_bwd_dkv_body<FP, DP, OutT, VEC, false, PART>(
+      fq, fk, v, log_gamma, dy, den, delta, p, dfk, dv, dG, csum, dlg_direct, nullptr, H, L, F, D,
+      rows, gate, 1, cps, 1, KG, xper, nxcd, nblk, nullptr, 0, part);
 }
 
 // ============================================================================
@@ -1277,6 +1346,13 @@ __global__ __launch_bounds__(64 * GATE_CHUNKS_PER_WG) void gla_gate_grad_kernel(
 // ============================================================================
 static int gate_rows(int B, int H, int gate) { return (gate & GATE_PER_HEAD) ? B * H : B; }
 
+// Whether the walks have a variant that adds to fp32 sums of dfq and dfk over
+// D tiles (GlaPart): the widest features, where D > 64 takes tiles of 64.
+template <int FP, bool VEC>
+constexpr bool gla_can_part() {
+  return VEC && FP == 256;
+}
+
 // den, delta, p, dG [BH][L]; forward and reverse segment records; chunk sums
 // of dG [BH][NT]
 size_t gla_bwd_workspace(int B, int H, int L, int F, int D, int gate) {
@@ -1307,9 +1383,9 @@ static hipError_t launch_gate_grad(const float* dG, const float* csum, const flo
 template <int FP, int DP, typename OutT, bool VEC>
 static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v, const float* lg,
                                    const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                                   int B, int H, int L, int F, int D, int gate, int KG,
-                                   const float* fwd_ws, float* ws, const float* ext_den,
-                                   const float* ext_delta, hipStream_t st) {
+                                   int B, int H, int L, int F, int D, GlaRows rows, int gate,
+                                   int KG, const float* fwd_ws, float* ws, const float* ext_den,
+                                   const float* ext_delta, const GlaPart* part, hipStream_t st) {
   const int BH = B * H;
   const size_t BHL = (size_t)BH * L;
   int G, cps;
@@ -1337,7 +1413,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
   hipError_t e;
   if (G > 1 && !fwd_ws) {
     e = launch_gla_fwd_states(fk, v, lg, own_fseg, own_fseg + (size_t)BH * G * SEG, BH, H, L, F,
-                              D, gate, G, cps, KG, fold, st);
+                              D, rows.ld, gate, G, cps, KG, fold, st);
     if (e != hipSuccess) return e;
   }
   // the walks take two segments per workgroup while that still gives one
@@ -1351,30 +1427,48 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
   // of workgroups (headline fwd+bwd 0.8808 -> 0.8628 ms, same bits).
   // a per-head gate in one segment: the reverse walk of (b, h) sees its whole
   // gate row and writes d log_gamma itself (no gate launch, no dG)
-  const bool direct_dlg = (gate & GATE_PER_HEAD) && G == 1;
+  const bool direct_dlg = (gate & GATE_PER_HEAD) && G == 1 && dlg;
+  // a D tile before the last leaves its share of dfq and dfk, and no gate gradient
+  auto gate_grad = [&]() {
+    return direct_dlg || !dlg ? hipSuccess
+                              : launch_gate_grad(dG, csum, lg, dlg, B, H, L, gate, st);
+  };
+  constexpr bool CAN_PART = gla_can_part<FP, VEC>();
+  const GlaPart pt = part ? *part : GlaPart{};
+  if (part && (!CAN_PART || ext)) return hipErrorInvalidValue;
   if (G == 1 && !ext) {
-    auto kf = gla_bwd_fused_kernel<FP, DP, OutT, VEC>;
     constexpr int LDS_F = LDS_A > LDS_B ? LDS_A : LDS_B;
-    if ((e = ensure_lds<gla_bwd_fused_kernel<FP, DP, OutT, VEC>>(LDS_F)) != hipSuccess) return e;
-    hipLaunchKernelGGL(kf, dim3(wg.grid), dim3(B_THREADS), LDS_F, st, (const bf16*)fq,
-                       (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (OutT*)dfq,
-                       (OutT*)dfk, (OutT*)dv, den, delta, p, dG, csum,
-                       direct_dlg ? dlg : nullptr, H, L, F, D, gate, cps, KG, wg.per, wg.nx,
-                       wg.nblk);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return direct_dlg ? hipSuccess : launch_gate_grad(dG, csum, lg, dlg, B, H, L, gate, st);
+    auto launch_f = [&](auto tag) {
+      constexpr auto kern = decltype(tag)::value;
+      if (hipError_t e2 = ensure_lds<kern>(LDS_F); e2 != hipSuccess) return e2;
+      hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_F, st, (const bf16*)fq,
+                         (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (OutT*)dfq,
+                         (OutT*)dfk, (OutT*)dv, den, delta, p, dG, csum,
+                         direct_dlg ? dlg : nullptr, H, L, F, D, rows, gate, cps, KG, wg.per, wg.nx,
+                         wg.nblk, pt);
+      return hipGetLastError();
+    };
+    if (part)
+      e = launch_f(KernTag<gla_bwd_fused_kernel<FP, DP, OutT, VEC, CAN_PART>>{});
+    else
+      e = launch_f(KernTag<gla_bwd_fused_kernel<FP, DP, OutT, VEC>>{});
+    return e != hipSuccess ? e : gate_grad();
   }
   auto launch_a = [&](auto tag) {
     constexpr auto kern = decltype(tag)::value;
     if (hipError_t e2 = ensure_lds<kern>(LDS_A); e2 != hipSuccess) return e2;
     hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_A, st, (const bf16*)fq,
                        (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (OutT*)dfq, den,
-                       delta, p, fseg, H, L, F, D, gate, G, cps, M, KG, wg.per, wg.nx,
-                       wg.nblk, flam);
+                       delta, p, fseg, H, L, F, D, rows, gate, G, cps, M, KG, wg.per, wg.nx,
+                       wg.nblk, flam, pt);
     return hipGetLastError();
   };
   if (ext)
     e = launch_a(KernTag<gla_bwd_dq_kernel<FP, DP, OutT, VEC, true>>{});
+  else if (part && fold)
+    e = launch_a(KernTag<gla_bwd_dq_kernel<FP, DP, OutT, VEC, false, CAN_FOLD, CAN_PART>>{});
+  else if (part)
+    e = launch_a(KernTag<gla_bwd_dq_kernel<FP, DP, OutT, VEC, false, false, CAN_PART>>{});
   else if (CAN_FOLD && fold)
     e = launch_a(KernTag<gla_bwd_dq_kernel<FP, DP, OutT, VEC, false, CAN_FOLD>>{});
   else
@@ -1386,7 +1480,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     if ((e = ensure_lds<gla_bwd_state_kernel<FP, DP, VEC>>(LDS_S)) != hipSuccess) return e;
     hipLaunchKernelGGL(ks, dim3(BH * (G - 1)), dim3(256), LDS_S, st,
                        (const bf16*)fq, (const bf16*)dy, lg, (const float*)den,
-                       (const float*)delta, rseg, rlam, H, L, F, D, gate, G, cps);
+                       (const float*)delta, rseg, rlam, H, L, F, D, rows, gate, G, cps);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!fold && (e = launch_gla_segment_scan(rseg, rlam, BH, G, SEG, true, st)) != hipSuccess)
       return e;
@@ -1403,30 +1497,35 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_B, st, (const bf16*)fq,
                        (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (const float*)den,
                        (const float*)delta, (const float*)p, (OutT*)dfk, (OutT*)dv, dG, csum,
-                       direct_dlg ? dlg : nullptr, (const float*)rseg, H, L, F, D, gate, G,
-                       cps, M, KG, wg.per, wg.nx, wg.nblk, (const float*)rlam, rev);
+                       direct_dlg ? dlg : nullptr, (const float*)rseg, H, L, F, D, rows, gate, G,
+                       cps, M, KG, wg.per, wg.nx, wg.nblk, (const float*)rlam, rev, pt);
     return hipGetLastError();
   };
-  if (CAN_FOLD && fold)
+  if (part && fold)
+    e = launch_b(KernTag<gla_bwd_dkv_kernel<FP, DP, OutT, VEC, CAN_FOLD, CAN_PART>>{});
+  else if (part)
+    e = launch_b(KernTag<gla_bwd_dkv_kernel<FP, DP, OutT, VEC, false, CAN_PART>>{});
+  else if (CAN_FOLD && fold)
     e = launch_b(KernTag<gla_bwd_dkv_kernel<FP, DP, OutT, VEC, CAN_FOLD>>{});
   else
     e = launch_b(KernTag<gla_bwd_dkv_kernel<FP, DP, OutT, VEC>>{});
-  if (e != hipSuccess) return e;
-  return direct_dlg ? hipSuccess : launch_gate_grad(dG, csum, lg, dlg, B, H, L, gate, st);
+  return e != hipSuccess ? e : gate_grad();
 }
 
 // ext_den / ext_delta: nullptr, or (one F tile of a split feature
 // dimension) den and delta [BH, L] of the whole feature dimension
 hipError_t launch_gla_bwd(const void* fq, const void* fk, const void* v, const float* lg,
                           const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                          bool grad_bf16, int B, int H, int L, int F, int D, int gate,
-                          int KG, const float* fwd_ws, float* ws, const float* ext_den,
-                          const float* ext_delta, hipStream_t st) {
+                          bool grad_bf16, int B, int H, int L, int F, int D, GlaRows rows,
+                          int gate, int KG, const float* fwd_ws, float* ws, const float* ext_den,
+                          const float* ext_delta, const GlaPart* part, hipStream_t st) {
   const int fp = gla_padded_dim(F), dp = gla_padded_dim(D);
-  const bool vec = F % 8 == 0 && D % 8 == 0;
+  if (fp < 256 && (rows.ld != D || rows.ldy != D || rows.hsy != L * D)) return hipErrorInvalidValue;
+  const bool vec = F % 8 == 0 && D % 8 == 0 && rows.ld % 8 == 0 && rows.ldy % 8 == 0 &&
+                   rows.hsy % 8 == 0;
 #define LZ_GLA_BWD_V(FPV, DPV, OUT, V)                                                          \
   launch_gla_bwd_t<FPV, DPV, OUT, V>(fq, fk, v, lg, dy, dfq, dfk, dv, dlg, B, H, L, F, D,      \
-                                     gate, KG, fwd_ws, ws, ext_den, ext_delta, st)
+                                     rows, gate, KG, fwd_ws, ws, ext_den, ext_delta, part, st)
 #define LZ_GLA_BWD(FPV, DPV)                                                                    \
   if (fp == FPV && dp == DPV)                                                                   \
     return grad_bf16 ? (vec ? LZ_GLA_BWD_V(FPV, DPV, bf16, true)                                \

@@ -27,18 +27,36 @@ struct GlaTiles {
 };
 GlaTiles gla_tiles(int F, int D);
 
+// Where the D-side rows of a walk lie, in elements: v, y and dv rows are `ld`
+// apart ([.., L, ld] slabs per head, the walk on D <= ld columns of them from
+// the pointers it is given: one D tile), dy rows `ldy` apart with heads `hsy`
+// apart.  Every batch entry spans H * L * ld elements.
+struct GlaRows {
+  int ld, ldy, hsy;
+};
+inline GlaRows gla_rows(int L, int ld) { return GlaRows{ld, ld, L * ld}; }
+
+// One of several D tiles' backward: dfq and dfk are sums over the tiles, kept
+// in fp32 [BH, L, F].  `in`: the sums so far to add (nullptr: the first tile);
+// `out`: where to leave them (nullptr: the last tile writes dfq, dfk and the
+// gate gradient).
+struct GlaPart {
+  const float *dfq_in, *dfk_in;
+  float *dfq_out, *dfk_out;
+};
+
 // The native walks (F, D within gla_dims_supported).  raw_den: see
 // gla_fwd_kernel's RAW; ext_den / ext_delta: see gla_bwd_dq_kernel's EXT.
 size_t gla_fwd_workspace(int B, int H, int L, int F, int D);
 size_t gla_bwd_workspace(int B, int H, int L, int F, int D, int gate);
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
-                          int B, int H, int L, int F, int D, int gate, int KG, float* ws,
-                          float* final_state, float* raw_den, hipStream_t st);
+                          int B, int H, int L, int F, int D, GlaRows rows, int gate, int KG,
+                          float* ws, float* final_state, float* raw_den, hipStream_t st);
 hipError_t launch_gla_bwd(const void* fq, const void* fk, const void* v, const float* lg,
                           const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                          bool grad_bf16, int B, int H, int L, int F, int D, int gate,
-                          int KG, const float* fwd_ws, float* ws, const float* ext_den,
-                          const float* ext_delta, hipStream_t st);
+                          bool grad_bf16, int B, int H, int L, int F, int D, GlaRows rows,
+                          int gate, int KG, const float* fwd_ws, float* ws, const float* ext_den,
+                          const float* ext_delta, const GlaPart* part, hipStream_t st);
 // Any F and D: the native walks, or tiles of them (gla_tiled.hip).
 size_t gla_fwd_workspace_any(int B, int H, int L, int F, int D);
 size_t gla_bwd_workspace_any(int B, int H, int L, int F, int D, int gate);
@@ -62,8 +80,8 @@ size_t gla_segment_floats(int BH, int G, int F, int D);
 // 8 * (idx % (KP/8)) .. +8.  Zero outside the matrix.
 template <int KP, int N, int AUX = 0>
 __device__ __forceinline__ void load_chunk(uint4 (&reg)[N], const bf16* __restrict__ base, int t0,
-                                           int L, int ncols, bool vec) {
-  load_items<KP, 256, N, 256 * N, AUX>(reg, base, t0, L, ncols, vec);
+                                           int L, int ncols, bool vec, int pitch) {
+  load_items<KP, 256, N, 256 * N, AUX>(reg, base, t0, L, ncols, vec, pitch);
 }
 
 template <int KP, int N>
@@ -455,7 +473,7 @@ inline bool gla_fold_segments(int G) { return G > 1 && G <= 4; }
 // segments; used by the forward and by the backward's forward walk.
 // fold: the walks fold the records (no scan).
 hipError_t launch_gla_fwd_states(const void* fk, const void* v, const float* lg, float* seg_state,
-                                 float* seg_logdecay, int BH, int H, int L, int F, int D,
+                                 float* seg_logdecay, int BH, int H, int L, int F, int D, int ld,
                                  int gate, int G, int cps, int KG, bool fold, hipStream_t st);
 hipError_t launch_gla_segment_scan(float* seg_state, const float* seg_logdecay, int BH, int G,
                                    int rec, bool reverse, hipStream_t st);

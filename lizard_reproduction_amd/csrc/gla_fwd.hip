@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, FP >= 256 ? 1 : 2) void gla_fwd_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, bf16* __restrict__ y,
     const float* __restrict__ seg_state, float* __restrict__ final_state, int H, int L, int F,
-    int D, int gate, int G, int cps, int M, int KG, float* __restrict__ raw_num,
+    int D, int ld, int gate, int G, int cps, int M, int KG, float* __restrict__ raw_num,
     float* __restrict__ raw_den, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam) {
   using Cfg = GlaFwd<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256, FP >= 256 ? 1 : 2) void gla_fwd_kernel(
   // fk and v belong to the kv head of this query head: KG query heads share one
   const bf16* fqb = fq + (size_t)bh * L * F;
   const bf16* fkb = fk + (size_t)(bh / KG) * L * F;
-  const bf16* vb = v + (size_t)(bh / KG) * L * D;
-  const rsrc_t yr = make_rsrc(y + (size_t)bh * L * D, (size_t)L * D * 2);
+  const bf16* vb = v + (size_t)(bh / KG) * L * ld;
+  const rsrc_t yr = make_rsrc(y + (size_t)bh * L * ld, pitched_bytes(L, D, ld));
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the state entering segment seg: its scanned record, or (FOLD) the local
   // records of segments 0 .. seg - 1 folded here (their total log decays at
@@ -175,9 +175,9 @@ __global__ __launch_bounds__(256, FP >= 256 ? 1 : 2) void gla_fwd_kernel(
 
   uint4 rq[Cfg::NLF], rk[Cfg::NLF], rv[Cfg::NLD];
   float rg;
-  load_chunk<FP, Cfg::NLF, AUX>(rq, fqb, n0 * C, L, F, vecF);
-  load_chunk<FP, Cfg::NLF, AUX>(rk, fkb, n0 * C, L, F, vecF);
-  load_chunk<DP, Cfg::NLD, AUX>(rv, vb, n0 * C, L, D, vecD);
+  load_chunk<FP, Cfg::NLF, AUX>(rq, fqb, n0 * C, L, F, vecF, F);
+  load_chunk<FP, Cfg::NLF, AUX>(rk, fkb, n0 * C, L, F, vecF, F);
+  load_chunk<DP, Cfg::NLD, AUX>(rv, vb, n0 * C, L, D, vecD, ld);
   rg = gate_at(lgb, n0 * C + lane, L);
   store_chunk<FP>(rq, fq_l, PF);
   store_chunk<FP>(rk, fk_l, PF);
@@ -189,9 +189,9 @@ __global__ __launch_bounds__(256, FP >= 256 ? 1 : 2) void gla_fwd_kernel(
     const int t0 = n * C;
     const bool more = n + 1 < n1;
     if (more) {   // next chunk in flight while this one computes
-      load_chunk<FP, Cfg::NLF, AUX>(rq, fqb, t0 + C, L, F, vecF);
-      load_chunk<FP, Cfg::NLF, AUX>(rk, fkb, t0 + C, L, F, vecF);
-      load_chunk<DP, Cfg::NLD, AUX>(rv, vb, t0 + C, L, D, vecD);
+      load_chunk<FP, Cfg::NLF, AUX>(rq, fqb, t0 + C, L, F, vecF, F);
+      load_chunk<FP, Cfg::NLF, AUX>(rk, fkb, t0 + C, L, F, vecF, F);
+      load_chunk<DP, Cfg::NLD, AUX>(rv, vb, t0 + C, L, D, vecD, ld);
       rg = gate_at(lgb, t0 + C + lane, L);
     }
     __builtin_amdgcn_s_setprio(0);
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256, FP >= 256 ? 1 : 2) void gla_fwd_kernel(
                                  1.f, h);
             if (dt == 0 && h == 0 && t0 + qi < L) raw_den[(size_t)bh * L + t0 + qi] = den;
           } else {
-            store_acc_row_bf16(yr, t0 + qi, dt * 32, D, vecD, o, recip_den(den), h);
+            store_acc_row_bf16(yr, t0 + qi, dt * 32, D, ld, vecD, o, recip_den(den), h);
           }
         }
 #pragma unroll
@@ -398,8 +398,8 @@ struct GlaFwdWide {
 // idx = tid + 512 i: row idx / (KP/8), 8 columns), and their LDS stores
 template <int KP, int N>
 __device__ __forceinline__ void load_chunk512(uint4 (&reg)[N], const bf16* __restrict__ base,
-                                              int t0, int L, int ncols, bool vec) {
-  load_items<KP, WIDE_THREADS, N, GLA_C * KP / 8>(reg, base, t0, L, ncols, vec);
+                                              int t0, int L, int ncols, bool vec, int pitch) {
+  load_items<KP, WIDE_THREADS, N, GLA_C * KP / 8>(reg, base, t0, L, ncols, vec, pitch);
 }
 
 template <int KP, int N>
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) void gla_fwd_wide_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, bf16* __restrict__ y,
     const float* __restrict__ seg_state, float* __restrict__ final_state, int H, int L, int F,
-    int D, int gate, int G, int cps, int M, int KG, float* __restrict__ raw_num,
+    int D, int ld, int gate, int G, int cps, int M, int KG, float* __restrict__ raw_num,
     float* __restrict__ raw_den, int xper, int nxcd, int nblk, const bf16* __restrict__ qrow,
     const bf16* __restrict__ wphi, const float* __restrict__ seg_lam) {
   static_assert(!(PHI && RAW), "the feature map is formed for whole-F walks only");
@@ -461,8 +461,8 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) void gla_fwd_wide_kernel(
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
   const bf16* fqb = fq + (size_t)bh * L * F;
   const bf16* fkb = fk + (size_t)(bh / KG) * L * F;   // fk, v: the kv head of this query head
-  const bf16* vb = v + (size_t)(bh / KG) * L * D;
-  const rsrc_t yr = make_rsrc(y + (size_t)bh * L * D, (size_t)L * D * 2);
+  const bf16* vb = v + (size_t)(bh / KG) * L * ld;
+  const rsrc_t yr = make_rsrc(y + (size_t)bh * L * ld, pitched_bytes(L, D, ld));
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the state entering segment seg: its scanned record, or (FOLD) the local
   // records of segments 0 .. seg - 1 folded here (their total log decays at
@@ -607,9 +607,9 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) void gla_fwd_wide_kernel(
   if constexpr (PHI)
     phi_load(n0 * C);
   else
-    load_chunk512<FP>(rq, fqb, n0 * C, L, F, vecF);
-  load_chunk512<FP>(rk, fkb, n0 * C, L, F, vecF);
-  load_chunk512<DP>(rv, vb, n0 * C, L, D, vecD);
+    load_chunk512<FP>(rq, fqb, n0 * C, L, F, vecF, F);
+  load_chunk512<FP>(rk, fkb, n0 * C, L, F, vecF, F);
+  load_chunk512<DP>(rv, vb, n0 * C, L, D, vecD, ld);
   rg = gate_at(lgb, n0 * C + lane, L);
 
   if constexpr (PHI) {
@@ -643,9 +643,9 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) void gla_fwd_wide_kernel(
       if constexpr (PHI)
         phi_load(t0 + C);
       else
-        load_chunk512<FP>(rq, fqb, t0 + C, L, F, vecF);
-      load_chunk512<FP>(rk, fkb, t0 + C, L, F, vecF);
-      load_chunk512<DP>(rv, vb, t0 + C, L, D, vecD);
+        load_chunk512<FP>(rq, fqb, t0 + C, L, F, vecF, F);
+      load_chunk512<FP>(rk, fkb, t0 + C, L, F, vecF, F);
+      load_chunk512<DP>(rv, vb, t0 + C, L, D, vecD, ld);
       rg = gate_at(lgb, t0 + C + lane, L);
     }
     // ---- phase 1 ------------------------------------------------------------
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(WIDE_THREADS, 1) void gla_fwd_wide_kernel(
                              h);
         if (dt == 0 && h == 0 && t0 + qi < L) raw_den[(size_t)bh * L + t0 + qi] = den;
       } else {
-        store_acc_row_bf16(yr, t0 + qi, dt * 32, D, vecD, o, recip_den(den), h);
+        store_acc_row_bf16(yr, t0 + qi, dt * 32, D, ld, vecD, o, recip_den(den), h);
       }
     }
 #pragma unroll
@@ -996,7 +996,7 @@ template <int FP, int DP, bool VEC, int FR, bool REV = false>
 __global__ __launch_bounds__(256, 2) void gla_fwd_state_kernel(
     const bf16* __restrict__ fk, const bf16* __restrict__ v, const float* __restrict__ log_gamma,
     float* __restrict__ seg_state, float* __restrict__ seg_logdecay, int H, int L, int F, int D,
-    int gate, int G, int cps, int KG) {
+    int ld, int gate, int G, int cps, int KG) {
   using Cfg = GlaState<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT;
@@ -1025,11 +1025,11 @@ __global__ __launch_bounds__(256, 2) void gla_fwd_state_kernel(
   const bf16* fkb = fk + (size_t)(bh / KG) * L * F + f0;
   const int fcols = F - f0;   // valid columns from f0 (<= 0: none, the slice is zero)
   const size_t fk_bytes = fcols > 0 ? ((size_t)L * F - f0) * 2 : 0;
-  const bf16* vb = v + (size_t)(bh / KG) * L * D;
+  const bf16* vb = v + (size_t)(bh / KG) * L * ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   auto load_fk = [&](uint4 (&reg)[Cfg::NLF], int t) {
     if constexpr (NFS == 1)
-      load_chunk<FP>(reg, fkb, t, L, F, vecF);
+      load_chunk<FP>(reg, fkb, t, L, F, vecF, F);
     else
       load_chunk_strided<FP>(reg, fkb, fk_bytes, t, F, fcols, vecF);
   };
@@ -1100,7 +1100,7 @@ __global__ __launch_bounds__(256, 2) void gla_fwd_state_kernel(
   const int nf = REV ? n1 - 1 : n0;   // the first chunk this pass reads
   float rg = gate_at(lgb, nf * C + lane, L);   // the gate first: waited for alone
   load_fk(rk, nf * C);
-  load_chunk<DP>(rv, vb, nf * C, L, D, vecD);
+  load_chunk<DP>(rv, vb, nf * C, L, D, vecD, ld);
   {
     const int pb = nf & 1;
     if (wave == 0)
@@ -1122,7 +1122,7 @@ __global__ __launch_bounds__(256, 2) void gla_fwd_state_kernel(
     const int tn = more ? (REV ? t0 - C : t0 + C) : L;
     rg = gate_at(lgb, tn + lane, L);
     load_fk(rk, tn);
-    load_chunk<DP>(rv, vb, tn, L, D, vecD);
+    load_chunk<DP>(rv, vb, tn, L, D, vecD, ld);
     __builtin_amdgcn_s_setprio(0);
     const float r_n = rdec[4 * pc];
     if (wave == 0) lam += rdec[4 * pc + 1];
@@ -1302,15 +1302,15 @@ constexpr size_t GLA_STATE_REV_BYTES = size_t(128) << 20;
 template <int FS, int FR, int DP, bool VEC>
 static hipError_t launch_state_slices(const void* fk, const void* v, const float* lg,
                                       float* seg_state, float* seg_logdecay, int BH, int H, int L,
-                                      int F, int D, int gate, int G, int cps, int KG, bool rev,
-                                      hipStream_t st) {
+                                      int F, int D, int ld, int gate, int G, int cps, int KG,
+                                      bool rev, hipStream_t st) {
   using Cfg = GlaState<FS, DP>;
   auto launch = [&](auto tag) {
     constexpr auto kern = decltype(tag)::value;
     if (hipError_t e = ensure_lds<kern>(Cfg::BYTES); e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(BH * (G - 1) * (FR / FS)), dim3(256), Cfg::BYTES, st,
                        (const bf16*)fk, (const bf16*)v, lg, seg_state, seg_logdecay, H, L, F, D,
-                       gate, G, cps, KG);
+                       ld, gate, G, cps, KG);
     return hipGetLastError();
   };
   if constexpr (FS == FR)
@@ -1329,7 +1329,7 @@ static int gla_state_slices(int workgroups, int FP) {
 template <int FP, int DP, bool VEC>
 static hipError_t launch_gla_fwd_states_t(const void* fk, const void* v, const float* lg,
                                           float* seg_state, float* seg_logdecay, int BH, int H,
-                                          int L, int F, int D, int gate, int G, int cps,
+                                          int L, int F, int D, int ld, int gate, int G, int cps,
                                           int KG, bool fold, hipStream_t st) {
   if (!(gate & GATE_PER_HEAD) && KG > 1) {   // one record per kv head (seg_owner)
     BH /= KG;
@@ -1344,22 +1344,22 @@ static hipError_t launch_gla_fwd_states_t(const void* fk, const void* v, const f
   if constexpr (FP == 256) {
     if (nfs == 4)
       e = launch_state_slices<64, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F,
-                                               D, gate, G, cps, KG, rev, st);
+                                               D, ld, gate, G, cps, KG, rev, st);
     else if (nfs == 2)
       e = launch_state_slices<128, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F,
-                                                D, gate, G, cps, KG, rev, st);
+                                                D, ld, gate, G, cps, KG, rev, st);
     else
       e = launch_state_slices<FP, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F,
-                                               D, gate, G, cps, KG, rev, st);
+                                               D, ld, gate, G, cps, KG, rev, st);
   } else if constexpr (FP == 128) {
     if (nfs == 2)
       e = launch_state_slices<64, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F,
-                                               D, gate, G, cps, KG, rev, st);
+                                               D, ld, gate, G, cps, KG, rev, st);
     else
       e = launch_state_slices<FP, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F,
-                                               D, gate, G, cps, KG, rev, st);
+                                               D, ld, gate, G, cps, KG, rev, st);
   } else {
-    e = launch_state_slices<FP, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F, D,
+    e = launch_state_slices<FP, FP, DP, VEC>(fk, v, lg, seg_state, seg_logdecay, BH, H, L, F, D, ld,
                                              gate, G, cps, KG, rev, st);
   }
   if (e != hipSuccess) return e;
@@ -1369,17 +1369,17 @@ static hipError_t launch_gla_fwd_states_t(const void* fk, const void* v, const f
 }
 
 hipError_t launch_gla_fwd_states(const void* fk, const void* v, const float* lg, float* seg_state,
-                                 float* seg_logdecay, int BH, int H, int L, int F, int D,
+                                 float* seg_logdecay, int BH, int H, int L, int F, int D, int ld,
                                  int gate, int G, int cps, int KG, bool fold, hipStream_t st) {
   const int fp = gla_padded_dim(F), dp = gla_padded_dim(D);
-  const bool vec = F % 8 == 0 && D % 8 == 0;
+  const bool vec = F % 8 == 0 && D % 8 == 0 && ld % 8 == 0;
 #define LZ_GLA_ST(FPV, DPV)                                                                   \
   if (fp == FPV && dp == DPV)                                                                 \
     return vec ? launch_gla_fwd_states_t<FPV, DPV, true>(fk, v, lg, seg_state, seg_logdecay,  \
-                                                         BH, H, L, F, D, gate, G,    \
+                                                         BH, H, L, F, D, ld, gate, G, \
                                                          cps, KG, fold, st)                   \
                : launch_gla_fwd_states_t<FPV, DPV, false>(fk, v, lg, seg_state, seg_logdecay, \
-                                                          BH, H, L, F, D, gate, G,   \
+                                                          BH, H, L, F, D, ld, gate, G, \
                                                           cps, KG, fold, st);
   LZ_GLA_ST(32, 32) LZ_GLA_ST(32, 64) LZ_GLA_ST(32, 128)
   LZ_GLA_ST(64, 32) LZ_GLA_ST(64, 64) LZ_GLA_ST(64, 128)
@@ -1392,7 +1392,7 @@ hipError_t launch_gla_fwd_states(const void* fk, const void* v, const float* lg,
 template <int FP, int DP, bool VEC, bool RAW>
 static hipError_t launch_gla_fwd_t(const void* fq, const void* fk, const void* v,
                                    const float* lg, void* y, int B, int H, int L, int F, int D,
-                                   int gate, int KG, float* ws, float* final_state,
+                                   int ld, int gate, int KG, float* ws, float* final_state,
                                    float* raw_den, hipStream_t st) {
   using Cfg = GlaFwd<FP, DP>;
   const int BH = B * H;
@@ -1404,7 +1404,7 @@ static hipError_t launch_gla_fwd_t(const void* fq, const void* fk, const void* v
   float* seg_lam = ws + (size_t)BH * G * Cfg::SEG;
   if (G > 1) {
     hipError_t e = launch_gla_fwd_states_t<FP, DP, VEC>(fk, v, lg, seg_state, seg_lam, BH, H, L,
-                                                        F, D, gate, G, cps, KG, fold, st);
+                                                        F, D, ld, gate, G, cps, KG, fold, st);
     if (e != hipSuccess) return e;
   }
   const int M = gla_walk_segments(BH, G, F);
@@ -1417,7 +1417,7 @@ static hipError_t launch_gla_fwd_t(const void* fq, const void* fk, const void* v
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(WIDE_THREADS), W::BYTES, st,
                          (const bf16*)fq, (const bf16*)fk, (const bf16*)v, lg, (bf16*)y,
-                         (const float*)seg_state, final_state, H, L, F, D, gate, G, cps, M, KG,
+                         (const float*)seg_state, final_state, H, L, F, D, ld, gate, G, cps, M, KG,
                          RAW ? (float*)y : nullptr, raw_den, wg.per, wg.nx, wg.nblk,
                          (const bf16*)nullptr, (const bf16*)nullptr, (const float*)seg_lam);
       return hipGetLastError();
@@ -1432,7 +1432,7 @@ static hipError_t launch_gla_fwd_t(const void* fq, const void* fk, const void* v
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(256), Cfg::BYTES, st, (const bf16*)fq,
                          (const bf16*)fk, (const bf16*)v, lg, (bf16*)y, (const float*)seg_state,
-                         final_state, H, L, F, D, gate, G, cps, M, KG,
+                         final_state, H, L, F, D, ld, gate, G, cps, M, KG,
                          RAW ? (float*)y : nullptr, raw_den, wg.per, wg.nx, wg.nblk,
                          (const float*)seg_lam);
       return hipGetLastError();
@@ -1509,15 +1509,15 @@ hipError_t gla_fwd_prepare() {
 // feature dimension) y is the fp32 numerator [BH, L, D] and raw_den the fp32
 // denominator [BH, L] of this tile (see gla_fwd_kernel's RAW).
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
-                          int B, int H, int L, int F, int D, int gate, int KG, float* ws,
-                          float* final_state, float* raw_den, hipStream_t st) {
-  const int fp = gla_padded_dim(F), dp = gla_padded_dim(D);
-  const bool vec = F % 8 == 0 && D % 8 == 0;
+                          int B, int H, int L, int F, int D, GlaRows rows, int gate, int KG,
+                          float* ws, float* final_state, float* raw_den, hipStream_t st) {
+  const int fp = gla_padded_dim(F), dp = gla_padded_dim(D), ld = rows.ld;
+  const bool vec = F % 8 == 0 && D % 8 == 0 && ld % 8 == 0;
 #define LZ_GLA_FWD_R(FPV, DPV, V)                                                               \
-  (raw_den ? launch_gla_fwd_t<FPV, DPV, V, true>(fq, fk, v, lg, y, B, H, L, F, D,               \
+  (raw_den ? launch_gla_fwd_t<FPV, DPV, V, true>(fq, fk, v, lg, y, B, H, L, F, D, ld,           \
                                                  gate, KG, ws, final_state, raw_den,   \
                                                  st)                                            \
-           : launch_gla_fwd_t<FPV, DPV, V, false>(fq, fk, v, lg, y, B, H, L, F, D,              \
+           : launch_gla_fwd_t<FPV, DPV, V, false>(fq, fk, v, lg, y, B, H, L, F, D, ld,          \
                                                   gate, KG, ws, final_state, nullptr,  \
                                                   st))
 #define LZ_GLA_FWD(FPV, DPV)                                                                    \
@@ -1548,7 +1548,7 @@ hipError_t launch_gla_fwd_phi(const void* q, const void* wq, const void* fk, con
   static_assert(gla_can_fold<FP, DP, true>(), "folding variant of the phi walk");
   if (G > 1) {
     hipError_t e = launch_gla_fwd_states_t<FP, DP, true>(fk, v, lg, ws, seg_lam, BH, H, L, F, D,
-                                                         gate, G, cps, KG, fold, st);
+                                                         D, gate, G, cps, KG, fold, st);
     if (e != hipSuccess) return e;
   }
   const int M = gla_walk_segments(BH, G, F);
@@ -1560,7 +1560,7 @@ hipError_t launch_gla_fwd_phi(const void* q, const void* wq, const void* fk, con
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(WIDE_THREADS), W::PHI_BYTES, st,
                        (const bf16*)nullptr, (const bf16*)fk, (const bf16*)v, lg, (bf16*)y,
-                       (const float*)ws, final_state, H, L, F, D, gate, G, cps, M, KG,
+                       (const float*)ws, final_state, H, L, F, D, D, gate, G, cps, M, KG,
                        (float*)nullptr, (float*)nullptr, wg.per, wg.nx, wg.nblk, (const bf16*)q,
                        (const bf16*)wq, (const float*)seg_lam);
     return hipGetLastError();

@@ -22,10 +22,15 @@
 //   (F tile, D tile) walk with that den and delta (EXT).  dfq and dfk of
 //   tile f are its columns, dv and d log_gamma sums over the tiles.
 //
-// Operand tiles are copied into contiguous workspace buffers (the walks read
-// contiguous [rows, width] slabs); partial results are summed in fp32 in a
-// fixed order (tiles in order, one launch each), so results stay
-// deterministic.
+// D tiles alone (F <= 256) need no copies: the walks read and write their
+// columns of v, y, dy and dv where they lie (GlaRows), and at F > 128 the
+// backward's walks add dfq and dfk over the tiles themselves (GlaPart: fp32
+// sums left by one tile's walk, added by the next, written by the last).  That
+// needs rows of whole 16-byte pieces (D % 8 == 0).  At F = 256 D = 128 (B=1 H=32
+// L=4096) the copies and sums had taken 837 us of a layer's training step beside
+// 480 us of walks; the walks with the sums in them take 550 us.  Otherwise operand tiles are copied into contiguous workspace
+// buffers and partial results are summed by launches of their own.  All sums are
+// fp32 in a fixed order (tiles in order), so results stay deterministic.
 #include <algorithm>
 
 #include "gla_common.hpp"
@@ -159,6 +164,16 @@ size_t max_over_tiles(const GlaTiles& t, int F, int D, Fn ws) {
   return std::max(m, ws(fl, dl));
 }
 
+// D tiles of whole 16-byte pieces are read and written where they lie.
+bool tiles_in_place(const GlaTiles& t, int D) { return t.nF == 1 && D % 8 == 0; }
+
+// ... and their backward's walks sum dfq and dfk themselves (the sums' rows
+// are behind one buffer resource each).
+bool tiles_sum_in_walk(const GlaTiles& t, int L, int F, int D) {
+  return tiles_in_place(t, D) && gla_padded_dim(F) == 256 && F % 8 == 0 &&
+         (size_t)L * F * 4 < OOB;
+}
+
 // The buffers of the tiled forward (workspace `ws`, or sizing when null).
 struct FwdBufs {
   bf16 *fqt, *fkt, *vt, *yt;
@@ -174,8 +189,10 @@ FwdBufs carve_fwd(Carve& c, const GlaTiles& t, int B, int H, int L, int F, int D
     return gla_fwd_workspace(B, H, L, f, d);
   });
   if (t.nF == 1) {
-    b.vt = c.take<bf16>(BHL * t.Dt);
-    b.yt = c.take<bf16>(BHL * t.Dt);
+    if (!tiles_in_place(t, D)) {
+      b.vt = c.take<bf16>(BHL * t.Dt);
+      b.yt = c.take<bf16>(BHL * t.Dt);
+    }
   } else {
     b.fqt = c.take<bf16>(BHL * t.Ft);
     b.fkt = c.take<bf16>(BHL * t.Ft);
@@ -207,7 +224,8 @@ hipError_t raw_forward(const GlaTiles& t, const FwdBufs& b, const void* fq, cons
         if ((e = copy_bf16(b.vt, dw, 0, (const bf16*)v, D, d * t.Dt, dw, BHLk, st))) return e;
         vt = b.vt;
       }
-      if ((e = launch_gla_fwd(b.fqt, b.fkt, vt, lg, b.numt, B, H, L, fw, dw, gph, KG, b.inner,
+      if ((e = launch_gla_fwd(b.fqt, b.fkt, vt, lg, b.numt, B, H, L, fw, dw, gla_rows(L, dw), gph,
+                              KG, b.inner,
                               nullptr, b.dent, st)))
         return e;
       if ((e = put_f32(b.num, D, d * t.Dt, b.numt, dw, 0, dw, BHL, f == 0, st))) return e;
@@ -232,8 +250,8 @@ hipError_t launch_gla_fwd_any(const void* fq, const void* fk, const void* v, con
                               void* ws, hipStream_t st) {
   const GlaTiles t = gla_tiles(F, D);
   if (t.native())
-    return launch_gla_fwd(fq, fk, v, lg, y, B, H, L, F, D, gph, KG, (float*)ws, nullptr, nullptr,
-                          st);
+    return launch_gla_fwd(fq, fk, v, lg, y, B, H, L, F, D, gla_rows(L, D), gph, KG, (float*)ws,
+                          nullptr, nullptr, st);
   Carve c{(char*)ws};
   const FwdBufs b = carve_fwd(c, t, B, H, L, F, D);
   const size_t BHL = (size_t)B * H * L, BHLk = BHL / KG;
@@ -244,9 +262,15 @@ hipError_t launch_gla_fwd_any(const void* fq, const void* fk, const void* v, con
       // every D tile reads fq and fk again: only the last may load them as
       // read no more (GATE_NO_REUSE)
       const int gd = d + 1 < t.nD ? gph & ~GATE_NO_REUSE : gph;
+      if (tiles_in_place(t, D)) {
+        if ((e = launch_gla_fwd(fq, fk, (const bf16*)v + d * t.Dt, lg, (bf16*)y + d * t.Dt, B, H, L,
+                                F, dw, gla_rows(L, D), gd, KG, b.inner, nullptr, nullptr, st)))
+          return e;
+        continue;
+      }
       if ((e = copy_bf16(b.vt, dw, 0, (const bf16*)v, D, d * t.Dt, dw, BHLk, st))) return e;
-      if ((e = launch_gla_fwd(fq, fk, b.vt, lg, b.yt, B, H, L, F, dw, gd, KG, b.inner, nullptr,
-                              nullptr, st)))
+      if ((e = launch_gla_fwd(fq, fk, b.vt, lg, b.yt, B, H, L, F, dw, gla_rows(L, dw), gd, KG,
+                              b.inner, nullptr, nullptr, st)))
         return e;
       if ((e = copy_bf16((bf16*)y, D, d * t.Dt, b.yt, dw, 0, dw, BHL, st))) return e;
     }
@@ -276,6 +300,15 @@ struct BwdBufs {
 BwdBufs carve_bwd(Carve& c, const GlaTiles& t, int B, int H, int L, int F, int D, int gph) {
   const size_t BHL = (size_t)B * H * L, NG = (gph & GATE_PER_HEAD) ? BHL : (size_t)B * L;
   BwdBufs b{};
+  b.inner_bytes = max_over_tiles(t, F, D, [&](int f, int d) {
+    return gla_bwd_workspace(B, H, L, f, d, gph);
+  });
+  if (tiles_sum_in_walk(t, L, F, D)) {
+    b.dfq_a = c.take<float>(BHL * F);
+    b.dfk_a = c.take<float>(BHL * F);
+    b.inner = c.take<float>((b.inner_bytes + 3) / 4);
+    return b;
+  }
   if (t.nF > 1) b.fwd = carve_fwd(c, t, B, H, L, F, D);
   b.vt = c.take<bf16>(BHL * t.Dt);
   b.dyt = c.take<bf16>(BHL * t.Dt);
@@ -288,9 +321,6 @@ BwdBufs carve_bwd(Carve& c, const GlaTiles& t, int B, int H, int L, int F, int D
   b.dfk_a = c.take<float>(BHL * F);
   if (t.nF > 1) b.dv_a = c.take<float>(BHL * D);
   b.dlg_a = c.take<float>(NG);
-  b.inner_bytes = max_over_tiles(t, F, D, [&](int f, int d) {
-    return gla_bwd_workspace(B, H, L, f, d, gph);
-  });
   b.inner = c.take<float>((b.inner_bytes + 3) / 4);
   return b;
 }
@@ -311,12 +341,28 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
                               const float* fwd_ws, void* ws, hipStream_t st) {
   const GlaTiles t = gla_tiles(F, D);
   if (t.native())
-    return launch_gla_bwd(fq, fk, v, lg, dy, dfq, dfk, dv, dlg, grad_bf16, B, H, L, F, D, gph,
-                          KG, fwd_ws, (float*)ws, nullptr, nullptr, st);
+    return launch_gla_bwd(fq, fk, v, lg, dy, dfq, dfk, dv, dlg, grad_bf16, B, H, L, F, D,
+                          gla_rows(L, D), gph, KG, fwd_ws, (float*)ws, nullptr, nullptr, nullptr,
+                          st);
   Carve c{(char*)ws};
   const BwdBufs b = carve_bwd(c, t, B, H, L, F, D, gph);
   const size_t BHL = (size_t)B * H * L, BHLk = BHL / KG, NG = (gph & GATE_PER_HEAD) ? BHL : (size_t)B * L;
   hipError_t e;
+  if (tiles_sum_in_walk(t, L, F, D)) {
+    const size_t es = grad_bf16 ? 2 : 4;
+    for (int d = 0; d < t.nD; ++d) {
+      const bool last = d + 1 == t.nD;
+      const size_t c0 = (size_t)d * t.Dt;
+      const GlaPart part = {d ? b.dfq_a : nullptr, d ? b.dfk_a : nullptr,
+                            last ? nullptr : b.dfq_a, last ? nullptr : b.dfk_a};
+      if ((e = launch_gla_bwd(fq, fk, (const bf16*)v + c0, lg, (const bf16*)dy + c0, dfq, dfk,
+                              (char*)dv + c0 * es, last ? dlg : nullptr, grad_bf16, B, H, L, F,
+                              width_of(d, t.nD, t.Dt, D), gla_rows(L, D), gph, KG, nullptr, b.inner,
+                              nullptr, nullptr, &part, st)))
+        return e;
+    }
+    return hipSuccess;
+  }
   if (t.nF > 1) {   // num, den of the whole feature dimension, then delta per D tile
     if ((e = raw_forward(t, b.fwd, fq, fk, v, lg, B, H, L, F, D, gph, KG, st))) return e;
     for (int d = 0; d < t.nD; ++d) {
@@ -349,7 +395,8 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
       const float* eden = t.nF > 1 ? b.fwd.den : nullptr;
       const float* edel = t.nF > 1 ? b.delta + (size_t)d * BHL : nullptr;
       if ((e = launch_gla_bwd(fqt, fkt, vt, lg, dyt, b.dfq_t, b.dfk_t, b.dv_t, b.dlg_t, false, B,
-                              H, L, fw, dw, gph, KG, nullptr, b.inner, eden, edel, st)))
+                              H, L, fw, dw, gla_rows(L, dw), gph, KG, nullptr, b.inner, eden, edel,
+                              nullptr, st)))
         return e;
       // dfq, dfk: this F tile's columns, summed over the D tiles
       if ((e = put_f32(b.dfq_a, F, f * t.Ft, b.dfq_t, fw, 0, fw, BHL, d == 0, st))) return e;

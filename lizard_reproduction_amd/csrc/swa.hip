@@ -46,7 +46,7 @@ struct SwaCfg {
 template <int DP>
 __device__ __forceinline__ void swa_load(uint4 (&reg)[SwaCfg<DP>::NL], const bf16* __restrict__ base,
                                          int r0, int L, int d, bool vec) {
-  load_items<DP, 256, SwaCfg<DP>::NL, 256 * SwaCfg<DP>::NL>(reg, base, r0, L, d, vec);
+  load_items<DP, 256, SwaCfg<DP>::NL, 256 * SwaCfg<DP>::NL>(reg, base, r0, L, d, vec, d);
 }
 
 template <int DP>
@@ -630,12 +630,12 @@ __global__ __launch_bounds__(64 * SWA_WALK_WAVES, 1) void swa_bwd_walk_kernel(
   // 8 (tid % 8)); rows outside [0, L) read zero
   auto load_tile = [&](uint4& r, const bf16* src, int r0) {
     uint4 t[1];
-    load_items<64, NT, 1, NT>(t, src, r0, L, d, vec);
+    load_items<64, NT, 1, NT>(t, src, r0, L, d, vec, d);
     r = t[0];
   };
   auto load_qd = [&](uint4& r, const bf16* src, int r0) {   // a q or dy tile
     uint4 t[1];
-    load_items<64, NT, 1, NT, NTQ ? LOAD_NT : 0>(t, src, r0, L, d, vec);
+    load_items<64, NT, 1, NT, NTQ ? LOAD_NT : 0>(t, src, r0, L, d, vec, d);
     r = t[0];
   };
   auto store_tile = [&](const uint4& r, bf16* tile) {
@@ -886,13 +886,6 @@ struct SwaRing {
 
 // The largest NS a ring of R waves takes: two waves left for dq, stores and loads.
 constexpr int swa_ring_max_ns(int R) { return R - 2; }
-// The lane number, formed anew where it is used: the compiler cannot carry it,
-// or addresses made from it, over from an earlier use.
-__device__ __forceinline__ int fresh_lane() {
-  int zero = 0;
-  asm volatile("" : "+v"(zero));
-  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
-}
 // s_waitcnt vmcnt(0) (gfx9 encoding; expcnt and lgkmcnt unconstrained)
 constexpr int WAIT_VM0 = 0x0F70;
 inline int swa_ring_ns(int W) { return (int)(((long long)W + 30) / 32 + 1); }

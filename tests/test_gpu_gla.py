@@ -292,3 +292,24 @@ def test_gla_tiled_constant_values_stay_constant():
     with torch.no_grad():
         y = kernels.gla(fq.cuda(), fk.cuda(), v.cuda(), F.logsigmoid(z).cuda())
     assert ((y.float() + 1.25).abs().max() / 1.25).item() <= OUT_TOL
+
+
+# D tiles read and written in place, dfq and dfk summed over them inside the
+# walks: two and three tiles (the last one narrower: D = 72 is 40 + 32, D = 136
+# is 48 + 48 + 40), one segment per (b, h) (B*H = 256), folded and scanned
+# segment records, ragged features, both gate kinds and gradient dtypes; D = 100
+# (rows of no whole 16-byte pieces) still copies its tiles
+@pytest.mark.parametrize("features, dim, length, batch, heads, per_head, fp32", [
+    (256, 128, 333, 1, 2, True, False), (256, 72, 150, 1, 2, False, True),
+    (232, 136, 200, 1, 3, True, True), (256, 128, 70, 8, 32, True, False),
+    (256, 96, 130, 8, 32, False, True), (160, 80, 300, 2, 50, False, False),
+    (256, 128, 1100, 1, 2, False, False), (250, 128, 90, 1, 2, True, False),
+    (256, 100, 150, 1, 2, True, False)])
+def test_gla_value_tiles_in_place_match_oracle(features, dim, length, batch, heads, per_head, fp32):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=dim)
+    if fp32:
+        inputs = [t.float() for t in inputs[:3]] + [inputs[3]]
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(1))
+    compare(gla_kernel(64), gla_reference, inputs, grad,
+            label=f"value tiles F={features} D={dim} L={length} BH={batch * heads}")
