@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define LZ_ABI_VERSION 15
+#define LZ_ABI_VERSION 16
 
 /*
  * gate_mode of the GLA entry points: a combination of
@@ -257,6 +257,22 @@ int lz_swa_fwd(const void* q, const void* k, const void* v, const float* meta, i
 int lz_swa_decode_step(const void* q, const void* k_cache, const void* v_cache,
                        const float* meta, int n_meta, void* y, int batch, int heads, int kv_heads,
                        int window, int dim, int pos, float scale, void* stream);
+
+/*
+ * The layer's SWA decode step: lz_swa_decode_step that also puts the token's key
+ * and value into the caches and blends the branches (src/lizard_attention.py:94).
+ *   k_new, v_new  bf16 [B, kv_heads, dim], the key (RoPE applied) and value of
+ *             position pos, written to slot pos % window of k_cache, v_cache
+ *   meta      [n_meta] and alpha [1], bf16 if params_bf16, else f32
+ *   y_gla     bf16 [B, H, dim];  out  [B, H, dim] (bf16 if out_bf16, else f32) =
+ *             y_gla + alpha * y, y the row lz_swa_decode_step gives
+ * Other arguments as lz_swa_decode_step.
+ */
+int lz_layer_decode_swa(const void* q, const void* k_new, const void* v_new, void* k_cache,
+                        void* v_cache, const void* meta, int n_meta, const void* alpha,
+                        int params_bf16, const void* y_gla, void* out, int out_bf16, int batch,
+                        int heads, int kv_heads, int window, int dim, int pos, float scale,
+                        void* stream);
 
 /* Workspace bytes lz_swa_bwd needs for these sizes. */
 size_t lz_swa_bwd_workspace_bytes(int batch, int heads, int length, int dim, int n_meta);

@@ -8,7 +8,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_lib", "liblizard_hip.so")
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -33,6 +33,8 @@ SIGNATURES = {
                         _I, _I, _I, _I, _I, _I, _I, _I, _P, _S, _P, _S, _P]),
     "lz_swa_fwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
     "lz_swa_decode_step": (_I, [_P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "lz_layer_decode_swa": (_I, [_P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I,
+                                 _I, _I, _F, _P]),
     "lz_swa_bwd_workspace_bytes": (_S, [_I, _I, _I, _I, _I]),
     "lz_swa_bwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I,
                         _I, _I, _I, _I, _I, _I, _F, _P, _S, _P]),

@@ -49,6 +49,11 @@ constexpr int SWA_DEC_MAX_W = 8192;
 hipError_t launch_swa_decode(const void* q, const void* k_cache, const void* v_cache,
                              const float* meta, int n_meta, void* y, int BH, int W, int d,
                              int pos, float scale, int KG, hipStream_t st);
+hipError_t launch_layer_decode_swa(const void* q, const void* k_new, const void* v_new,
+                                   void* k_cache, void* v_cache, const void* meta, int n_meta,
+                                   const void* alpha, bool params_bf16, const void* yg, void* out,
+                                   bool out_bf16, int BH, int W, int d, int pos, float scale,
+                                   int KG, hipStream_t st);
 hipError_t launch_swa_bwd(const void* q, const void* k, const void* v, const float* meta,
                           int n_meta, const float* lse, const void* dy, void* dq, void* dk,
                           void* dv, bool grad_bf16, float* delta, float* dmeta_part,
@@ -411,6 +416,27 @@ extern "C" int lz_swa_decode_step(const void* q, const void* k_cache, const void
                                           window, dim, pos, scale, heads / kv_heads,
                                           (hipStream_t)stream),
                     "swa_decode_step");
+}
+
+extern "C" int lz_layer_decode_swa(const void* q, const void* k_new, const void* v_new,
+                                   void* k_cache, void* v_cache, const void* meta, int n_meta,
+                                   const void* alpha, int params_bf16, const void* y_gla, void* out,
+                                   int out_bf16, int batch, int heads, int kv_heads, int window,
+                                   int dim, int pos, float scale, void* stream) {
+  if (int rc = check_swa(q, k_cache, v_cache, (const float*)meta, n_meta, batch, heads, 1, dim,
+                         window))
+    return rc;
+  if (int rc = check_kv_heads("layer_decode_swa", heads, kv_heads)) return rc;
+  if (!k_new || !v_new || !alpha || !y_gla || !out)
+    return fail(1, "layer_decode_swa: null pointer");
+  if (window > lz::SWA_DEC_MAX_W)
+    return fail(1, "layer_decode_swa: window %d > %d unsupported", window, lz::SWA_DEC_MAX_W);
+  if (pos < 0) return fail(1, "layer_decode_swa: pos must be >= 0, got %d", pos);
+  return hip_status(
+      lz::launch_layer_decode_swa(q, k_new, v_new, k_cache, v_cache, meta, n_meta, alpha,
+                                  params_bf16 != 0, y_gla, out, out_bf16 != 0, batch * heads,
+                                  window, dim, pos, scale, heads / kv_heads, (hipStream_t)stream),
+      "layer_decode_swa");
 }
 
 extern "C" size_t lz_swa_bwd_workspace_bytes(int batch, int heads, int length, int dim,

@@ -170,12 +170,23 @@ struct ProBwdArgs {
 template <typename T, int FT, int HT>
 __device__ void load_weight(const T* __restrict__ w, int f, bf16* hi, bf16* lo) {
   using C = Pro<T, FT, HT>;
-  for (int i = threadIdx.x; i < C::FP * C::HP; i += blockDim.x) {
-    const int r = i / C::HP, c = i % C::HP;
-    const float x = r < f ? static_cast<float>(w[r * C::HP + c]) : 0.f;
-    const bf16 h = to_bf16(x);
-    hi[r * C::WP + c] = h;
-    if constexpr (C::SPLIT) lo[r * C::WP + c] = to_bf16(x - to_f32(h));
+  const bool aligned = (reinterpret_cast<uintptr_t>(w) & 15) == 0;   // a view may start anywhere
+  // 8 columns per load: element by element, the 32 dependent round trips of a
+  // 128 x 64 weight were most of a one-token launch (decode: 16.0 -> 10.0 us)
+  for (int i = threadIdx.x; i < C::FP * (C::HP / 8); i += blockDim.x) {
+    const int r = i / (C::HP / 8), c = 8 * (i % (C::HP / 8));
+    float x[8] = {};
+    if (r < f) {
+      const T* src = w + r * C::HP + c;
+      if (aligned)
+        cvt8(load8r(src), x);
+      else
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = static_cast<float>(src[e]);
+    }
+    const bf16x8 h = to_bf8(x);
+    *reinterpret_cast<bf16x8*>(hi + r * C::WP + c) = h;
+    if constexpr (C::SPLIT) *reinterpret_cast<bf16x8*>(lo + r * C::WP + c) = low8(x, h);
   }
 }
 

@@ -1501,6 +1501,12 @@ hipError_t launch_swa_bwd(const void* q, const void* k, const void* v, const flo
 //   s_p = scale q . k_p, m = max(max_p s_p, max_j meta_j) -- the forward's
 //   row at position pos (src/kernels/swa.py:19-59), with e^{s_p - m} rounded to
 //   bf16 before it weights v, as the forward's P is.
+// APPEND (the layer's step): position pos's key and value come from k_new, v_new
+// [B*Hkv, d] instead of the caches, into whose slot the first query head of each
+// kv head writes them (no workgroup reads that slot: it holds position pos - W or
+// nothing), and the output is the layer's blend yg + alpha y, y rounded to bf16
+// and the product and sum rounded separately as the blend kernel does.  That takes
+// two copies into the caches and the blend launch out of a step.
 // One workgroup per (b, h): thread t scores keys t, t + 256, ... (16-byte
 // loads of its key rows when d % 8 == 0 and the cache is 16-byte aligned); the
 // block takes the max and the sum; then thread (g, c) sums column c over keys
@@ -1529,10 +1535,17 @@ __device__ __forceinline__ float decode_sum256(float* sh, float x) {
   return x;
 }
 
+struct SwaAppend {
+  const bf16 *k_new, *v_new, *yg;
+  const void* alpha;
+  bf16 *k_slot, *v_slot;      // the caches, to write
+  int params_bf16, out_bf16;  // types of meta and alpha, and of the output
+};
+
+template <bool APPEND>
 __global__ __launch_bounds__(256) void swa_decode_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
-    const float* __restrict__ meta, int n_meta, bf16* __restrict__ y, int W, int d, int pos,
-    float scale, int KG) {
+    const bf16* __restrict__ q, const bf16* kc, const bf16* vc, const void* __restrict__ meta_,
+    int n_meta, void* __restrict__ y, int W, int d, int pos, float scale, int KG, SwaAppend ap) {
   extern __shared__ __align__(16) char smem[];
   float* w = reinterpret_cast<float*>(smem);        // [W] bf16-rounded weights
   float* qs = w + W;                                // [d] query
@@ -1542,14 +1555,30 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
   const int n = min(pos + 1, W);
   const bf16* kb = kc + (size_t)(bh / KG) * W * d;
   const bf16* vb = vc + (size_t)(bh / KG) * W * d;
+  const bool mb = APPEND && ap.params_bf16;
+  auto meta = [&](int j) {
+    return mb ? to_f32(static_cast<const bf16*>(meta_)[j]) : static_cast<const float*>(meta_)[j];
+  };
+  // row of key i (position pos - n + 1 + i) of a cache, or the new row
+  auto row = [&](const bf16* cache, const bf16* fresh, int i) {
+    if (APPEND && i == n - 1) return fresh + (size_t)(bh / KG) * d;
+    return cache + (size_t)((pos - n + 1 + i) % W) * d;
+  };
   const bool vec = (d & 7) == 0 && (reinterpret_cast<uintptr_t>(kb) & 15) == 0;
   for (int c = tid; c < d; c += 256) qs[c] = to_f32(q[(size_t)bh * d + c]);
+  if (APPEND && bh % KG == 0)
+    for (int c = tid; c < d; c += 256) {
+      const size_t from = (size_t)(bh / KG) * d + c;
+      const size_t to = ((size_t)(bh / KG) * W + pos % W) * d + c;
+      ap.k_slot[to] = ap.k_new[from];
+      ap.v_slot[to] = ap.v_new[from];
+    }
   __syncthreads();
   float mx = -1e30f;
-  for (int j = 0; j < n_meta; ++j) mx = fmaxf(mx, meta[j]);
+  for (int j = 0; j < n_meta; ++j) mx = fmaxf(mx, meta(j));
   // scores, key i = tid, tid + 256, ... (position pos - n + 1 + i)
   for (int i = tid; i < n; i += 256) {
-    const bf16* kr = kb + (size_t)((pos - n + 1 + i) % W) * d;
+    const bf16* kr = row(kb, ap.k_new, i);
     float s = 0.f;
     if (vec) {
       for (int c = 0; c < d; c += 8) {
@@ -1573,21 +1602,34 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
   }
   l = decode_sum256(sh, l);   // also orders the weight writes before the reads below
   float ls = 0.f;
-  for (int j = 0; j < n_meta; ++j) ls += fexp(meta[j] - m);
+  for (int j = 0; j < n_meta; ++j) ls += fexp(meta(j) - m);
   const float inv = 1.f / (ls + l);
   const int NG = 256 / d, g = tid / d, c = tid - g * d;   // d <= 256: NG >= 1
   float acc = 0.f;
   if (g < NG) {
 #pragma unroll 4
     for (int i = g; i < n; i += NG)
-      acc += w[i] * to_f32(vb[(size_t)((pos - n + 1 + i) % W) * d + c]);
+      acc += w[i] * to_f32(row(vb, ap.v_new, i)[c]);
   }
   part[tid] = acc;
   __syncthreads();
   if (tid < d) {
     float t = part[tid];
     for (int j = 1; j < NG; ++j) t += part[j * d + tid];
-    y[(size_t)bh * d + tid] = to_bf16(t * inv);
+    const size_t at = (size_t)bh * d + tid;
+    const bf16 ys = to_bf16(t * inv);
+    if constexpr (APPEND) {
+#pragma clang fp contract(off)
+      const float al = mb ? to_f32(*static_cast<const bf16*>(ap.alpha))
+                          : *static_cast<const float*>(ap.alpha);
+      const float o = to_f32(ap.yg[at]) + al * to_f32(ys);
+      if (ap.out_bf16)
+        static_cast<bf16*>(y)[at] = to_bf16(o);
+      else
+        static_cast<float*>(y)[at] = o;
+    } else {
+      static_cast<bf16*>(y)[at] = ys;
+    }
   }
 }
 
@@ -1599,11 +1641,27 @@ hipError_t launch_swa_decode(const void* q, const void* k_cache, const void* v_c
                              const float* meta, int n_meta, void* y, int BH, int W, int d,
                              int pos, float scale, int KG, hipStream_t st) {
   const size_t lds = swa_decode_lds(W, d);
-  hipError_t e = ensure_lds<swa_decode_kernel>((int)swa_decode_lds(SWA_DEC_MAX_W, 256));
+  hipError_t e = ensure_lds<swa_decode_kernel<false>>((int)swa_decode_lds(SWA_DEC_MAX_W, 256));
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(swa_decode_kernel, dim3(BH), dim3(256), lds, st, (const bf16*)q,
-                     (const bf16*)k_cache, (const bf16*)v_cache, meta, n_meta, (bf16*)y, W, d,
-                     pos, scale, KG);
+  hipLaunchKernelGGL(swa_decode_kernel<false>, dim3(BH), dim3(256), lds, st, (const bf16*)q,
+                     (const bf16*)k_cache, (const bf16*)v_cache, (const void*)meta, n_meta, y, W,
+                     d, pos, scale, KG, SwaAppend{});
+  return hipGetLastError();
+}
+
+hipError_t launch_layer_decode_swa(const void* q, const void* k_new, const void* v_new,
+                                   void* k_cache, void* v_cache, const void* meta, int n_meta,
+                                   const void* alpha, bool params_bf16, const void* yg, void* out,
+                                   bool out_bf16, int BH, int W, int d, int pos, float scale,
+                                   int KG, hipStream_t st) {
+  const size_t lds = swa_decode_lds(W, d);
+  hipError_t e = ensure_lds<swa_decode_kernel<true>>((int)swa_decode_lds(SWA_DEC_MAX_W, 256));
+  if (e != hipSuccess) return e;
+  const SwaAppend ap = {(const bf16*)k_new, (const bf16*)v_new, (const bf16*)yg, alpha,
+                        (bf16*)k_cache, (bf16*)v_cache, params_bf16, out_bf16};
+  hipLaunchKernelGGL(swa_decode_kernel<true>, dim3(BH), dim3(256), lds, st, (const bf16*)q,
+                     (const bf16*)k_cache, (const bf16*)v_cache, meta, n_meta, out, W, d, pos,
+                     scale, KG, ap);
   return hipGetLastError();
 }
 

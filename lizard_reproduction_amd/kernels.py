@@ -14,14 +14,17 @@ the reference; results do not depend on them beyond rounding, and the HIP
 kernels always use their own tiles (64-token GLA chunks, 32-row SWA tiles).
 
 Every call goes through the C ABI of ``liblizard_hip.so`` on the current HIP
-stream; there is no CPU or PyTorch fallback.
+stream; there is no CPU or PyTorch fallback.  ``gla`` and ``swa`` make their
+autograd nodes and launches in C++ (``_ops``, csrc/torch_ops.cpp) after the checks
+here; the Python nodes below serve calls under ``torch.func`` transforms or
+``torch.jit`` tracing.
 """
 import functools
 import math
 
 import torch
 
-from . import _lib
+from . import _lib, _ops
 
 CHUNK = 64
 FWD_BLOCKS = (64, 64)
@@ -283,7 +286,9 @@ def gla_prefill(fq, fk, v, log_gamma, chunk=CHUNK, gate_logit=False):
     b, h, length, nf = fq.shape
     nd = v.shape[-1]
     y = torch.empty(b, h, length, nd, device=v.device, dtype=torch.bfloat16)
-    state = torch.zeros(b, h, nf * nd + nf, device=fq.device, dtype=torch.float32)
+    # the launch writes the whole state; with no token it is an empty prefix's
+    state = (torch.empty if y.numel() else torch.zeros)(b, h, nf * nd + nf, device=fq.device,
+                                                         dtype=torch.float32)
     if y.numel():
         lib = _lib.load()
         mode = _gate_mode(lg, gate_logit) | GLA_NO_REUSE   # inference: no backward
@@ -324,7 +329,10 @@ def gla_forward_phi(qp, wq, fk, v, lg, heads, gate_logit=False, final_state=Fals
             raise ValueError(f"gla_forward_phi: {name} must be contiguous bf16")
     lg = _f32(lg)
     y = torch.empty(b, heads, length, 64, device=qp.device, dtype=torch.bfloat16)
-    state = new_state(b, heads, 256, 64, qp.device) if final_state else None
+    state = None
+    if final_state:   # written whole by the launch, zeros for an empty prompt
+        state = (torch.empty if y.numel() else torch.zeros)(b, heads, 256 * 64 + 256,
+                                                             device=qp.device, dtype=torch.float32)
     if y.numel():
         mode = _gate_mode(lg, gate_logit)
         nbytes = _gla_fwd_ws(b, heads, length, 256, 64, mode & GATE_PER_HEAD, chunk)
@@ -395,6 +403,8 @@ def gla(fq, fk, v, log_gamma, chunk=CHUNK):
     Returns bf16 ``[B, H, L, D]``.
     """
     _check_gla(fq, fk, v, log_gamma, chunk)
+    if _ops.plain():
+        return _ops.load().gla(fq, fk, v, log_gamma, chunk)
     if not (torch.is_grad_enabled() and (fq.requires_grad or fk.requires_grad or
                                          v.requires_grad or log_gamma.requires_grad)):
         # nothing to differentiate: the same forward launch without the
@@ -547,6 +557,8 @@ def swa(q, k, v, meta, window, fwd_blocks=FWD_BLOCKS, bwd_blocks=BWD_BLOCKS):
     s_it = q_i . k_t / sqrt(d).  Returns bf16 ``[B, H, L, d]``.
     """
     _check_swa(q, k, v, meta, window, fwd_blocks, bwd_blocks)
+    if _ops.plain():
+        return _ops.load().swa(q, k, v, meta, window)
     if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or
                                          v.requires_grad or meta.requires_grad)):
         # nothing to differentiate: the forward launch without the autograd node

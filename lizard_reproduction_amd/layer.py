@@ -36,7 +36,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib, kernels
+from . import _lib, _ops, kernels
 
 BACKENDS = ("hip",)
 MAX_HEAD_DIM = 256       # lz_swa_*: dim <= 256
@@ -257,9 +257,12 @@ class LizardCache:
             self.v[:, :, p0 % window] = v[:, :, 0]
             return
         first = max(0, n - window)
-        slots = torch.arange(p0 + first, p0 + n, device=kr.device) % window
-        self.k[:, :, slots] = kr[:, :, first:]
-        self.v[:, :, slots] = v[:, :, first:]
+        while first < n:   # at most two runs of slots: to the ring's end, from its start
+            slot = (p0 + first) % window
+            run = min(n - first, window - slot)
+            self.k[:, :, slot:slot + run] = kr[:, :, first:first + run]
+            self.v[:, :, slot:slot + run] = v[:, :, first:first + run]
+            first += run
 
 
 class LizardAttention(nn.Module):
@@ -431,7 +434,6 @@ class LizardAttention(nn.Module):
         """``forward`` over a prompt [B, L, hidden] (no autograd) that also
         returns the decode cache after it: ``(out, cache)``."""
         x = hidden_states
-        cache = self.new_cache(x.shape[0], x.device)
         cos, sin = position_embeddings
         qp, kp, vp = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         if self._fused(qp, kp, vp, cos, sin) and self._phi_walk(qp, kp, vp, cos, sin):
@@ -446,10 +448,33 @@ class LizardAttention(nn.Module):
                                            self.meta_tokens.detach().float().contiguous(),
                                            self.window)
             out = self._out(y_gla, y_swa, x)
-        cache.state = state
+        shape = (x.shape[0], self.kv_heads, self.window, self.head_dim)
+        make = torch.empty if x.shape[1] >= self.window else torch.zeros   # the prompt fills it
+        cache = LizardCache(state, make(shape, device=x.device, dtype=torch.bfloat16),
+                            make(shape, device=x.device, dtype=torch.bfloat16), 0)
         cache.put(kr, v, 0)
         cache.pos = x.shape[1]
         return out, cache
+
+    def _step_native(self, x, projections, cos, sin, cache):
+        """Whether ``_ops.layer_step`` takes this step: the shapes the decode
+        kernels take, and a cache as ``prefill`` and ``new_cache`` make it.  Any
+        other step goes operator by operator, which casts or refuses it."""
+        b, hd, nf = x.shape[0], self.head_dim, 2 * self.phi_q.weight.shape[0]
+        ring = (b, self.kv_heads, self.window, hd)
+        return (b > 0 and _ops.plain() and self._fused(*projections, cos, sin)
+                and kernels.gla_native(nf, hd)
+                and tuple(cos.shape) == tuple(sin.shape)
+                and tuple(cos.shape) in ((1, hd), (1, 1, hd), (b, 1, hd))
+                and type(cache.pos) is int and cache.pos >= 0
+                and self.window <= kernels.SWA_DECODE_MAX_WINDOW
+                and tuple(cache.state.shape) == (b, self.heads, nf * hd + nf)
+                and cache.state.dtype is torch.float32 and cache.state.is_contiguous()
+                and all(tuple(t.shape) == ring and t.dtype is torch.bfloat16
+                        and t.is_contiguous() and t.device == x.device
+                        for t in (cache.k, cache.v))
+                and cache.state.device == x.device
+                and all(t.device == x.device for t in (cos, sin)))
 
     @torch.no_grad()
     def step(self, hidden_states, position_embeddings, cache):
@@ -460,7 +485,19 @@ class LizardAttention(nn.Module):
         if x.dim() != 3 or x.shape[1] != 1:
             raise ValueError(f"LizardAttention.step: hidden_states must be [B, 1, hidden], got "
                              f"{tuple(x.shape)}")
-        z, fq, fk, qr, kr, v = self._operands(x, position_embeddings)
+        kernels._refuse_capture("LizardAttention")
+        if x.device.type != "cuda":
+            raise ValueError("LizardAttention (hip backend) needs its input on a ROCm GPU")
+        cos, sin = position_embeddings
+        projections = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        if self._step_native(x, projections, cos, sin, cache):
+            y = _ops.load().layer_step(*projections, self.W_gamma(x), self.phi_q.weight,
+                                       self.phi_k.weight, cos, sin, self.meta_tokens,
+                                       self.alpha_blend, cache.state, cache.k, cache.v, cache.pos,
+                                       x.dtype == torch.bfloat16)
+            cache.pos += 1
+            return self.o_proj(y.to(x.dtype))
+        z, fq, fk, qr, kr, v = self._operands(x, position_embeddings, projections)
         cache.put(kr, v, cache.pos)
         y_gla = kernels.gla_decode_step(fq[:, :, 0], fk[:, :, 0], v[:, :, 0], z[:, 0].contiguous(),
                                         cache.state, gate_logit=True)

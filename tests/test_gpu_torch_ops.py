@@ -1,0 +1,164 @@
+"""The C++ autograd nodes and decode step (csrc/torch_ops.cpp) against the Python
+ones they stand in for: the same bits over the forms the operators accept, and
+the same behaviour under the features that act on an autograd node."""
+import types
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from lizard_reproduction_amd import _ops, kernels
+from lizard_reproduction_amd.layer import LizardAttention
+
+pytestmark = pytest.mark.gpu
+
+
+def _through_python(monkeypatch, fn):
+    with monkeypatch.context() as m:
+        m.setattr(_ops, "plain", lambda: False)
+        return fn()
+
+
+def _step(op, tensors, requires):
+    leaves = [t.detach().requires_grad_(r) for t, r in zip(tensors, requires)]
+    y = op(*leaves)
+    got = [y.detach()]
+    if any(requires):
+        g = torch.Generator(device="cuda").manual_seed(3)
+        y.backward(torch.randn(y.shape, device="cuda", generator=g).to(y.dtype))
+        got += [t.grad for t in leaves]
+    return got
+
+
+def _forms(t, form):
+    """The same values in another dtype or layout."""
+    if form == "strided":
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+    return t.to({"bf16": torch.bfloat16, "fp32": torch.float32, "fp16": torch.float16}[form])
+
+
+FORMS = [("bf16",) * 3, ("fp32",) * 3, ("bf16", "fp32", "fp16"), ("strided", "bf16", "strided")]
+
+
+@pytest.mark.parametrize("forms", FORMS)
+@pytest.mark.parametrize("requires", [(True,) * 4, (False,) * 4, (False, True, False, True)])
+@pytest.mark.parametrize("shape, features, dim, per_head", [
+    ((1, 2, 1), 16, 16, False), ((2, 3, 77), 24, 20, True), ((1, 2, 130), 256, 128, False),
+    ((1, 2, 0), 16, 16, True)])
+def test_gla_node_gives_the_python_nodes_bits(monkeypatch, forms, requires, shape, features, dim,
+                                              per_head):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    fq, fk = (torch.rand(*shape, features, device="cuda", generator=g) for _ in range(2))
+    v = torch.randn(*shape, dim, device="cuda", generator=g)
+    lg = F.logsigmoid(torch.randn(shape if per_head else (shape[0], shape[2]), device="cuda",
+                                  generator=g))
+    tensors = [_forms(t, f) for t, f in zip((fq, fk, v), forms)] + [lg]
+    ours = _step(kernels.gla, tensors, requires)
+    theirs = _through_python(monkeypatch, lambda: _step(kernels.gla, tensors, requires))
+    for a, b in zip(ours, theirs):
+        assert (a is None) == (b is None)
+        assert a is None or (a.dtype == b.dtype and torch.equal(a, b))
+
+
+@pytest.mark.parametrize("forms", FORMS)
+@pytest.mark.parametrize("requires", [(True,) * 4, (False,) * 4, (True, False, False, False)])
+@pytest.mark.parametrize("shape, window, sinks", [((1, 2, 1, 16), 4, 2), ((2, 3, 77, 64), 16, 0),
+                                                  ((1, 2, 150, 128), 100, 4)])
+def test_swa_node_gives_the_python_nodes_bits(monkeypatch, forms, requires, shape, window, sinks):
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(shape, device="cuda", generator=g) for _ in range(3))
+    meta = torch.randn(sinks, device="cuda", generator=g)
+    tensors = [_forms(t, f) for t, f in zip((q, k, v), forms)] + [meta]
+
+    def op(*a):
+        return kernels.swa(*a, window)
+    ours = _step(op, tensors, requires)
+    theirs = _through_python(monkeypatch, lambda: _step(op, tensors, requires))
+    for a, b in zip(ours, theirs):
+        assert (a is None) == (b is None)
+        assert a is None or (a.dtype == b.dtype and torch.equal(a, b))
+
+
+def _gla_leaves():
+    g = torch.Generator(device="cuda").manual_seed(1)
+    fq, fk = (torch.rand(1, 2, 70, 16, device="cuda", generator=g).bfloat16().requires_grad_()
+              for _ in range(2))
+    v = torch.randn(1, 2, 70, 16, device="cuda", generator=g).bfloat16().requires_grad_()
+    return fq, fk, v, F.logsigmoid(torch.randn(1, 70, device="cuda", generator=g)).requires_grad_()
+
+
+def test_saved_tensor_hooks_see_the_saved_operands():
+    leaves, packed = _gla_leaves(), []
+
+    def pack(t):
+        packed.append(tuple(t.shape))
+        return t.cpu()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        y = kernels.gla(*leaves)
+    plain = kernels.gla(*leaves)
+    dy = torch.ones_like(y)
+    assert packed == [tuple(t.shape) for t in leaves]
+    for a, b in zip(torch.autograd.grad(y, leaves, dy), torch.autograd.grad(plain, leaves, dy)):
+        assert torch.equal(a, b)
+
+
+def test_changed_operands_second_backward_and_transforms_are_refused():
+    fq, fk, v, lg = _gla_leaves()
+    y = kernels.gla(fq, fk, v, lg)
+    with torch.no_grad():
+        fk.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    y = kernels.gla(fq, fk, v, lg)
+    y.sum().backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        y.sum().backward()
+    # gradients of gradients have no graph
+    y = kernels.gla(fq, fk, v, lg)
+    dv, = torch.autograd.grad(y.float().sum(), v, create_graph=True)
+    assert not dv.requires_grad or dv.grad_fn is None
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(kernels.gla)(*(t.detach()[None] for t in (fq, fk, v, lg)))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: kernels.gla(fq, fk, t, lg).float().sum())(v.detach())
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        kernels.gla(fq, fk, torch.autograd.forward_ad.make_dual(v, torch.ones_like(v)), lg)
+
+
+@pytest.mark.parametrize("heads, kv, dtype, rope_batched, window, prompt", [
+    (4, 2, torch.bfloat16, False, 16, 40), (4, 4, torch.float32, True, 64, 10),
+    (2, 1, torch.bfloat16, True, 5, 0)])
+def test_native_layer_step_equals_the_step_by_operators(monkeypatch, heads, kv, dtype, rope_batched,
+                                                        window, prompt):
+    """Prompt (none, shorter and longer than the window), then steps through the
+    ring's wrap: outputs, state and caches bit for bit."""
+    torch.manual_seed(heads)
+    cfg = types.SimpleNamespace(hidden_size=64 * heads, num_attention_heads=heads,
+                                num_key_value_heads=kv)
+    layer = LizardAttention(cfg, 0, window=window, feature_dim=32).to("cuda", dtype)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0, 0.2)
+    b, steps = 3, 9
+    x = torch.randn(b, prompt + steps, 64 * heads, device="cuda").to(dtype)
+    angle = torch.rand(prompt + steps, 64, device="cuda") * 6
+    cos, sin = angle.cos().to(dtype), angle.sin().to(dtype)
+
+    def tables(lo, hi):
+        c, s = cos[lo:hi], sin[lo:hi]
+        return (c.expand(b, -1, -1), s.expand(b, -1, -1)) if rope_batched else (c, s)
+
+    def run():
+        if prompt:
+            with torch.no_grad():
+                y, cache = layer.prefill(x[:, :prompt], tables(0, prompt))
+            outs = [y]
+        else:
+            cache, outs = layer.new_cache(b), []
+        for t in range(prompt, prompt + steps):
+            outs.append(layer.step(x[:, t:t + 1], tables(t, t + 1), cache))
+        return outs + [cache.state, cache.k, cache.v]
+    ours = run()
+    theirs = _through_python(monkeypatch, run)
+    for a, c in zip(ours, theirs):
+        assert torch.equal(a, c)
