@@ -26,6 +26,8 @@
 // softmax statistics are per-lane scalars; P and dS then feed the next product
 // straight from the accumulator registers.  Consecutive workgroups of one
 // (b, h) are mapped to one XCD so that the tiles they share hit one L2.
+#include <initializer_list>
+
 #include "common.hpp"
 
 namespace lz {
@@ -1507,13 +1509,19 @@ hipError_t launch_swa_bwd(const void* q, const void* k, const void* v, const flo
 // nothing), and the output is the layer's blend yg + alpha y, y rounded to bf16
 // and the product and sum rounded separately as the blend kernel does.  That takes
 // two copies into the caches and the blend launch out of a step.
-// One workgroup per (b, h): thread t scores keys t, t + 256, ... (16-byte
-// loads of its key rows when d % 8 == 0 and the cache is 16-byte aligned); the
-// block takes the max and the sum; then thread (g, c) sums column c over keys
-// g, g + NG, ... (NG = 256 / d groups, v rows read coalesced) and the groups'
-// partial sums meet in LDS.
+// One workgroup per (b, h).  Where rows are 16-byte pieces (d = 32, 64, 128 or 256
+// and aligned operands), CG = d / 8 lanes share a key or value row, one load each:
+// the scores are lane-group sums, the block takes the max and the denominator, and
+// the weighted values are summed over a wave's lane groups and the four waves.
+// The loads of four passes' key rows and of the first value rows go out together,
+// so a window of 64 waits for memory once (per-thread key rows and a column per
+// thread waited 8 and 4 times: B=4, 32/8 heads, d=64, W=64 9.1 -> 6.6 us).
+// Otherwise (CG = 0) thread t scores keys t, t + 256, ... element by element; then
+// thread (g, c) sums column c over keys g, g + NG, ... (NG = 256 / d groups) and
+// the groups' partial sums meet in LDS.
 // ----------------------------------------------------------------------------
 constexpr int SWA_DEC_MAX_W = 8192;
+constexpr int SWA_DEC_PART = 4 * 256;   // one sum per wave and column, or one per thread
 
 __device__ __forceinline__ float decode_max256(float* sh, float x) {
 #pragma unroll
@@ -1542,15 +1550,15 @@ struct SwaAppend {
   int params_bf16, out_bf16;  // types of meta and alpha, and of the output
 };
 
-template <bool APPEND>
+template <int CG, bool APPEND>
 __global__ __launch_bounds__(256) void swa_decode_kernel(
     const bf16* __restrict__ q, const bf16* kc, const bf16* vc, const void* __restrict__ meta_,
     int n_meta, void* __restrict__ y, int W, int d, int pos, float scale, int KG, SwaAppend ap) {
   extern __shared__ __align__(16) char smem[];
   float* w = reinterpret_cast<float*>(smem);        // [W] bf16-rounded weights
   float* qs = w + W;                                // [d] query
-  float* part = qs + ((d + 3) & ~3);                // [256] column partial sums
-  float* sh = part + 256;                           // [4] block reductions
+  float* part = qs + ((d + 3) & ~3);                // column partial sums
+  float* sh = part + SWA_DEC_PART;                  // [4] block reductions
   const int bh = blockIdx.x, tid = threadIdx.x;
   const int n = min(pos + 1, W);
   const bf16* kb = kc + (size_t)(bh / KG) * W * d;
@@ -1564,8 +1572,6 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
     if (APPEND && i == n - 1) return fresh + (size_t)(bh / KG) * d;
     return cache + (size_t)((pos - n + 1 + i) % W) * d;
   };
-  const bool vec = (d & 7) == 0 && (reinterpret_cast<uintptr_t>(kb) & 15) == 0;
-  for (int c = tid; c < d; c += 256) qs[c] = to_f32(q[(size_t)bh * d + c]);
   if (APPEND && bh % KG == 0)
     for (int c = tid; c < d; c += 256) {
       const size_t from = (size_t)(bh / KG) * d + c;
@@ -1573,80 +1579,172 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
       ap.k_slot[to] = ap.k_new[from];
       ap.v_slot[to] = ap.v_new[from];
     }
-  __syncthreads();
   float mx = -1e30f;
   for (int j = 0; j < n_meta; ++j) mx = fmaxf(mx, meta(j));
-  // scores, key i = tid, tid + 256, ... (position pos - n + 1 + i)
-  for (int i = tid; i < n; i += 256) {
-    const bf16* kr = row(kb, ap.k_new, i);
-    float s = 0.f;
-    if (vec) {
-      for (int c = 0; c < d; c += 8) {
-        const bf16x8 k8 = *reinterpret_cast<const bf16x8*>(kr + c);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += qs[c + e] * to_f32(k8[e]);
-      }
-    } else {
-      for (int c = 0; c < d; ++c) s += qs[c] * to_f32(kr[c]);
-    }
-    s *= scale;
-    w[i] = s;
-    mx = fmaxf(mx, s);
-  }
-  const float m = decode_max256(sh, mx);
-  float l = 0.f;
-  for (int i = tid; i < n; i += 256) {
-    const float e = fexp(w[i] - m);
-    l += e;
-    w[i] = to_f32(to_bf16(e));
-  }
-  l = decode_sum256(sh, l);   // also orders the weight writes before the reads below
-  float ls = 0.f;
-  for (int j = 0; j < n_meta; ++j) ls += fexp(meta(j) - m);
-  const float inv = 1.f / (ls + l);
-  const int NG = 256 / d, g = tid / d, c = tid - g * d;   // d <= 256: NG >= 1
-  float acc = 0.f;
-  if (g < NG) {
-#pragma unroll 4
-    for (int i = g; i < n; i += NG)
-      acc += w[i] * to_f32(row(vb, ap.v_new, i)[c]);
-  }
-  part[tid] = acc;
-  __syncthreads();
-  if (tid < d) {
-    float t = part[tid];
-    for (int j = 1; j < NG; ++j) t += part[j * d + tid];
-    const size_t at = (size_t)bh * d + tid;
-    const bf16 ys = to_bf16(t * inv);
+  const size_t at0 = (size_t)bh * d;
+  // the row's column c of the output, from its weighted sum
+  auto put = [&](int c, float t) {
+    const bf16 ys = to_bf16(t);
     if constexpr (APPEND) {
 #pragma clang fp contract(off)
       const float al = mb ? to_f32(*static_cast<const bf16*>(ap.alpha))
                           : *static_cast<const float*>(ap.alpha);
-      const float o = to_f32(ap.yg[at]) + al * to_f32(ys);
+      const float o = to_f32(ap.yg[at0 + c]) + al * to_f32(ys);
       if (ap.out_bf16)
-        static_cast<bf16*>(y)[at] = to_bf16(o);
+        static_cast<bf16*>(y)[at0 + c] = to_bf16(o);
       else
-        static_cast<float*>(y)[at] = o;
+        static_cast<float*>(y)[at0 + c] = o;
     } else {
-      static_cast<bf16*>(y)[at] = ys;
+      static_cast<bf16*>(y)[at0 + c] = ys;
+    }
+  };
+
+  if constexpr (CG > 0) {
+    // CG lanes per key, 8 columns each: KP keys per pass, PASS passes' rows in
+    // flight, the first values' rows alongside the keys'
+    constexpr int KP = 256 / CG, PASS = 4;
+    const int cg = tid % CG, kg = tid / CG, lane = tid & 63, wave = tid >> 6;
+    auto rows = [&](bf16x8 (&x)[PASS], const bf16* cache, const bf16* fresh, int i0) {
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        const int i = min(i0 + KP * p + kg, n - 1);   // a valid row; unused past n
+        x[p] = *reinterpret_cast<const bf16x8*>(row(cache, fresh, i) + 8 * cg);
+      }
+    };
+    const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(q + at0 + 8 * cg);
+    bf16x8 v8[PASS];
+    for (int i0 = 0; i0 < n; i0 += KP * PASS) {
+      bf16x8 k8[PASS];
+      rows(k8, kb, ap.k_new, i0);
+      if (i0 == 0) rows(v8, vb, ap.v_new, 0);
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        float s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += to_f32(q8[e]) * to_f32(k8[p][e]);
+#pragma unroll
+        for (int off = 1; off < CG; off <<= 1) s += __shfl_xor(s, off);
+        s *= scale;
+        const int i = i0 + KP * p + kg;
+        if (i < n) {
+          mx = fmaxf(mx, s);
+          if (cg == 0) w[i] = s;
+        }
+      }
+    }
+    const float m = decode_max256(sh, mx);   // also orders the score writes
+    float l = 0.f;
+    for (int i = tid; i < n; i += 256) {
+      const float e = fexp(w[i] - m);
+      l += e;
+      w[i] = to_f32(to_bf16(e));
+    }
+    l = decode_sum256(sh, l);   // also orders the weight writes before the reads below
+    float ls = 0.f;
+    for (int j = 0; j < n_meta; ++j) ls += fexp(meta(j) - m);
+    const float inv = 1.f / (ls + l);
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n; i0 += KP * PASS) {
+      if (i0 > 0) rows(v8, vb, ap.v_new, i0);
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        const int i = i0 + KP * p + kg;
+        if (i < n) {
+          const float wi = w[i];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += wi * to_f32(v8[p][e]);
+        }
+      }
+    }
+    // over the keys of a wave, then over the waves in order
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+      for (int off = CG; off < 64; off <<= 1) acc[e] += __shfl_xor(acc[e], off);
+      if (lane < CG) part[wave * 8 * CG + 8 * lane + e] = acc[e];
+    }
+    __syncthreads();
+    if (tid < d) put(tid, ((part[tid] + part[8 * CG + tid]) +
+                           (part[16 * CG + tid] + part[24 * CG + tid])) * inv);
+  } else {
+    for (int c = tid; c < d; c += 256) qs[c] = to_f32(q[at0 + c]);
+    __syncthreads();
+    // scores, key i = tid, tid + 256, ... (position pos - n + 1 + i)
+    for (int i = tid; i < n; i += 256) {
+      const bf16* kr = row(kb, ap.k_new, i);
+      float s = 0.f;
+      for (int c = 0; c < d; ++c) s += qs[c] * to_f32(kr[c]);
+      s *= scale;
+      w[i] = s;
+      mx = fmaxf(mx, s);
+    }
+    const float m = decode_max256(sh, mx);
+    float l = 0.f;
+    for (int i = tid; i < n; i += 256) {
+      const float e = fexp(w[i] - m);
+      l += e;
+      w[i] = to_f32(to_bf16(e));
+    }
+    l = decode_sum256(sh, l);   // also orders the weight writes before the reads below
+    float ls = 0.f;
+    for (int j = 0; j < n_meta; ++j) ls += fexp(meta(j) - m);
+    const float inv = 1.f / (ls + l);
+    const int NG = 256 / d, g = tid / d, c = tid - g * d;   // d <= 256: NG >= 1
+    float acc = 0.f;
+    if (g < NG) {
+#pragma unroll 4
+      for (int i = g; i < n; i += NG) acc += w[i] * to_f32(row(vb, ap.v_new, i)[c]);
+    }
+    part[tid] = acc;
+    __syncthreads();
+    if (tid < d) {
+      float t = part[tid];
+      for (int j = 1; j < NG; ++j) t += part[j * d + tid];
+      put(tid, t * inv);
     }
   }
 }
 
 size_t swa_decode_lds(int W, int d) {
-  return ((size_t)W + ((d + 3) & ~3) + 256 + 4) * sizeof(float);
+  return ((size_t)W + ((d + 3) & ~3) + SWA_DEC_PART + 4) * sizeof(float);
+}
+
+// q, the caches and (APPEND) the new rows as 16-byte pieces
+static int swa_decode_lanes(int d, std::initializer_list<const void*> rows) {
+  if (d != 32 && d != 64 && d != 128 && d != 256) return 0;
+  for (const void* p : rows)
+    if (reinterpret_cast<uintptr_t>(p) & 15) return 0;
+  return d / 8;
+}
+
+template <bool APPEND>
+static hipError_t launch_decode(int lanes, const void* q, const void* k_cache, const void* v_cache,
+                                const void* meta, int n_meta, void* y, int BH, int W, int d,
+                                int pos, float scale, int KG, const SwaAppend& ap,
+                                hipStream_t st) {
+  auto launch = [&](auto tag) {
+    constexpr auto kern = decltype(tag)::value;
+    if (hipError_t e = ensure_lds<kern>((int)swa_decode_lds(SWA_DEC_MAX_W, 256)); e != hipSuccess)
+      return e;
+    hipLaunchKernelGGL(kern, dim3(BH), dim3(256), swa_decode_lds(W, d), st, (const bf16*)q,
+                       (const bf16*)k_cache, (const bf16*)v_cache, meta, n_meta, y, W, d, pos,
+                       scale, KG, ap);
+    return hipGetLastError();
+  };
+  switch (lanes) {
+    case 4: return launch(KernTag<swa_decode_kernel<4, APPEND>>{});
+    case 8: return launch(KernTag<swa_decode_kernel<8, APPEND>>{});
+    case 16: return launch(KernTag<swa_decode_kernel<16, APPEND>>{});
+    case 32: return launch(KernTag<swa_decode_kernel<32, APPEND>>{});
+    default: return launch(KernTag<swa_decode_kernel<0, APPEND>>{});
+  }
 }
 
 hipError_t launch_swa_decode(const void* q, const void* k_cache, const void* v_cache,
                              const float* meta, int n_meta, void* y, int BH, int W, int d,
                              int pos, float scale, int KG, hipStream_t st) {
-  const size_t lds = swa_decode_lds(W, d);
-  hipError_t e = ensure_lds<swa_decode_kernel<false>>((int)swa_decode_lds(SWA_DEC_MAX_W, 256));
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(swa_decode_kernel<false>, dim3(BH), dim3(256), lds, st, (const bf16*)q,
-                     (const bf16*)k_cache, (const bf16*)v_cache, (const void*)meta, n_meta, y, W,
-                     d, pos, scale, KG, SwaAppend{});
-  return hipGetLastError();
+  return launch_decode<false>(swa_decode_lanes(d, {q, k_cache, v_cache}), q, k_cache, v_cache,
+                              meta, n_meta, y, BH, W, d, pos, scale, KG, SwaAppend{}, st);
 }
 
 hipError_t launch_layer_decode_swa(const void* q, const void* k_new, const void* v_new,
@@ -1654,15 +1752,10 @@ hipError_t launch_layer_decode_swa(const void* q, const void* k_new, const void*
                                    const void* alpha, bool params_bf16, const void* yg, void* out,
                                    bool out_bf16, int BH, int W, int d, int pos, float scale,
                                    int KG, hipStream_t st) {
-  const size_t lds = swa_decode_lds(W, d);
-  hipError_t e = ensure_lds<swa_decode_kernel<true>>((int)swa_decode_lds(SWA_DEC_MAX_W, 256));
-  if (e != hipSuccess) return e;
   const SwaAppend ap = {(const bf16*)k_new, (const bf16*)v_new, (const bf16*)yg, alpha,
                         (bf16*)k_cache, (bf16*)v_cache, params_bf16, out_bf16};
-  hipLaunchKernelGGL(swa_decode_kernel<true>, dim3(BH), dim3(256), lds, st, (const bf16*)q,
-                     (const bf16*)k_cache, (const bf16*)v_cache, meta, n_meta, out, W, d, pos,
-                     scale, KG, ap);
-  return hipGetLastError();
+  return launch_decode<true>(swa_decode_lanes(d, {q, k_cache, v_cache, k_new, v_new}), q, k_cache,
+                             v_cache, meta, n_meta, out, BH, W, d, pos, scale, KG, ap, st);
 }
 
 }  // namespace lz

@@ -209,3 +209,28 @@ def test_layer_prefill_and_steps_continue_the_forward(dtype, prefix, steps):
         assert errs["forward_max"] <= OUT_TOL and errs["oracle_max"] <= OUT_TOL, errs
     else:
         assert errs["forward_norm"] < 1e-2 and errs["oracle_norm"] < 2e-2, errs
+
+
+# A lane group's pass covers 256 / (d / 8) keys and four passes' rows are in
+# flight: windows on both sides of one pass and of four, a cache still filling,
+# one that has wrapped, and head dims with and without whole lane groups
+@pytest.mark.parametrize("dim, window, pos", [
+    (64, 1, 0), (64, 31, 90), (64, 32, 40), (64, 33, 20), (64, 128, 127), (64, 129, 300),
+    (32, 64, 70), (32, 257, 600), (128, 64, 64), (128, 65, 30), (256, 33, 50), (256, 8, 3),
+    (96, 40, 77), (20, 300, 310)])
+def test_swa_decode_step_row_equals_the_forward_row(dim, window, pos):
+    b, h, kv = 2, 4, 2
+    g = torch.Generator(device="cuda").manual_seed(dim + window)
+    q = torch.randn(b, h, pos + 1, dim, device="cuda", generator=g).bfloat16()
+    k, v = (torch.randn(b, kv, pos + 1, dim, device="cuda", generator=g).bfloat16()
+            for _ in range(2))
+    meta = torch.randn(3, device="cuda", generator=g)
+    kc, vc = (torch.full((b, kv, window, dim), 7.0, device="cuda", dtype=torch.bfloat16)
+              for _ in range(2))
+    at = torch.arange(max(0, pos + 1 - window), pos + 1, device="cuda")
+    kc[:, :, at % window], vc[:, :, at % window] = k[:, :, at], v[:, :, at]
+    ours = kernels.swa_decode_step(q[:, :, pos].contiguous(), kc, vc, meta, pos)
+    theirs, _ = kernels.swa_forward(q, k, v, meta, window)
+    # both round their weights to bf16 (2^-9) before they meet v, about a common
+    # or a running maximum: outputs 2^-8 of the largest apart, and their own rounding
+    assert max_rel(ours, theirs[:, :, pos]) <= 2.0 ** -7
