@@ -63,6 +63,10 @@ extern "C" {
 /* Most sink logits (n_meta) the SWA entry points take. */
 #define LZ_SWA_MAX_META 65536
 
+/* Most rows and matrices lz_rows_linear takes. */
+#define LZ_ROWS_MAX 16
+#define LZ_ROWS_MATS 4
+
 /* ABI version of the loaded library (LZ_ABI_VERSION). */
 int lz_abi_version(void);
 
@@ -273,6 +277,18 @@ int lz_layer_decode_swa(const void* q, const void* k_new, const void* v_new, voi
                         int params_bf16, const void* y_gla, void* out, int out_bf16, int batch,
                         int heads, int kv_heads, int window, int dim, int pos, float scale,
                         void* stream);
+
+/*
+ * Products of a few rows with up to LZ_ROWS_MATS weight matrices, y_i = x w_i^T
+ * (a decode step's projections, src/lizard_attention.py:73-76,97):
+ *   x  bf16 [rows, cols], rows at most LZ_ROWS_MAX, cols a multiple of 8
+ *   w  host array of `mats` device pointers, w_i bf16 [n_i, cols]
+ *   y  host array, y_i [rows, n_i]: bf16, or with y_f32[i] the bf16 value as f32
+ *   n, y_f32  host arrays
+ * x and w_i 16-byte aligned and contiguous.  fp32 sums.
+ */
+int lz_rows_linear(const void* x, int rows, int cols, int mats, const void* const* w,
+                   void* const* y, const int* n, const int* y_f32, void* stream);
 
 /* Workspace bytes lz_swa_bwd needs for these sizes. */
 size_t lz_swa_bwd_workspace_bytes(int batch, int heads, int length, int dim, int n_meta);

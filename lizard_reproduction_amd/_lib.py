@@ -33,6 +33,7 @@ SIGNATURES = {
                         _I, _I, _I, _I, _I, _I, _I, _I, _P, _S, _P, _S, _P]),
     "lz_swa_fwd": (_I, [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
     "lz_swa_decode_step": (_I, [_P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "lz_rows_linear": (_I, [_P, _I, _I, _I, _P, _P, _P, _P, _P]),
     "lz_layer_decode_swa": (_I, [_P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I,
                                  _I, _I, _F, _P]),
     "lz_swa_bwd_workspace_bytes": (_S, [_I, _I, _I, _I, _I]),

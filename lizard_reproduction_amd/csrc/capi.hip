@@ -60,6 +60,8 @@ hipError_t launch_swa_bwd(const void* q, const void* k, const void* v, const flo
                           float* dmeta, int BH, int L, int d, int W, float scale, int KG,
                           hipStream_t st);
 constexpr int MAX_META = LZ_SWA_MAX_META;
+hipError_t launch_rows_linear(const void* x, int M, int K, int mats, const void* const* w,
+                              void* const* y, const int* n, const int* f32, hipStream_t st);
 bool prologue_dims_supported(int hd, int f, bool bf16_in);
 size_t prologue_bwd_workspace(int B, int L, int H, int Hkv, int hd, int f);
 hipError_t launch_prologue_fwd(const void* q, const void* k, const void* v, const void* wq,
@@ -437,6 +439,27 @@ extern "C" int lz_layer_decode_swa(const void* q, const void* k_new, const void*
                                   params_bf16 != 0, y_gla, out, out_bf16 != 0, batch * heads,
                                   window, dim, pos, scale, heads / kv_heads, (hipStream_t)stream),
       "layer_decode_swa");
+}
+
+extern "C" int lz_rows_linear(const void* x, int rows, int cols, int mats, const void* const* w,
+                              void* const* y, const int* n, const int* y_f32, void* stream) {
+  if (!x || !w || !y || !n || !y_f32) return fail(1, "rows_linear: null pointer");
+  if (rows <= 0 || rows > LZ_ROWS_MAX || mats <= 0 || mats > LZ_ROWS_MATS)
+    return fail(1, "rows_linear: rows must be in [1, %d] and matrices in [1, %d], got %d and %d",
+                LZ_ROWS_MAX, LZ_ROWS_MATS, rows, mats);
+  if (cols <= 0 || cols % 8) return fail(1, "rows_linear: cols %% 8 must be 0, got %d", cols);
+  uintptr_t bits = reinterpret_cast<uintptr_t>(x);
+  for (int i = 0; i < mats; ++i) {
+    if (!w[i] || !y[i]) return fail(1, "rows_linear: null pointer");
+    // one buffer resource per matrix, the last tile's rows past the end included
+    if (n[i] <= 0 || ((size_t)n[i] + 16) * cols * 2 >= (size_t(1) << 31))
+      return fail(1, "rows_linear: matrix of %d x %d outside (0, 2 GiB)", n[i], cols);
+    bits |= reinterpret_cast<uintptr_t>(w[i]);
+  }
+  if (bits & 15) return fail(1, "rows_linear: x and w must be 16-byte aligned");
+  return hip_status(lz::launch_rows_linear(x, rows, cols, mats, w, y, n, y_f32,
+                                           (hipStream_t)stream),
+                    "rows_linear");
 }
 
 extern "C" size_t lz_swa_bwd_workspace_bytes(int batch, int heads, int length, int dim,

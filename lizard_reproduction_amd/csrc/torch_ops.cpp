@@ -9,7 +9,7 @@
 // Python.  Measured for a forward and backward of one sequence (H = 32, L = 2048,
 // d = 64), where the kernels take 75 and 35 us: gla 138 -> 87 us, swa 120 -> 75 us;
 // a short forward (H = 4, L = 256) 17.5 -> 12.8 us; a decode step of the layer (B =
-// 4, hidden 2048) 201 -> 132 us, of which this function takes 21 us of host time.
+// 4, hidden 2048) 201 -> 132 us with torch's projections, 48 us with rows.hip's.
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
@@ -266,6 +266,44 @@ Tensor layer_step(Tensor qp, Tensor kp, Tensor vp, const Tensor& z, Tensor wq, T
   return out;
 }
 
+// y_i = x w_i^T for the rows of x [.., K]; outputs [.., n_i], the ones in `wide`
+// as fp32
+std::vector<Tensor> rows_linear(const Tensor& x, const std::vector<Tensor>& w,
+                                const std::vector<bool>& wide) {
+  const int rows = i32(x.numel() / x.size(-1)), cols = i32(x.size(-1)), mats = i32(w.size());
+  const void* wp[LZ_ROWS_MATS];
+  void* yp[LZ_ROWS_MATS];
+  int n[LZ_ROWS_MATS], f32out[LZ_ROWS_MATS];
+  TORCH_CHECK(mats <= LZ_ROWS_MATS, "rows_linear: at most ", LZ_ROWS_MATS, " matrices");
+  std::vector<Tensor> y;
+  for (int i = 0; i < mats; ++i) {
+    auto sizes = x.sizes().vec();
+    sizes.back() = w[i].size(0);
+    y.push_back(at::empty(sizes, x.options().dtype(wide[i] ? at::kFloat : at::kBFloat16)));
+    wp[i] = ptr(w[i]);
+    yp[i] = ptr(y[i]);
+    n[i] = i32(w[i].size(0));
+    f32out[i] = wide[i];
+  }
+  check(lz_rows_linear(ptr(x), rows, cols, mats, wp, yp, n, f32out, stream_of(x)),
+        "lz_rows_linear");
+  return y;
+}
+
+// The whole step of a bf16 layer whose projections are plain matrices, for x
+// [B, 1, hidden], B <= LZ_ROWS_MAX: the four projections of x in one launch
+// (the gate's logit as fp32, of its bf16 value), the step, and o_proj.
+Tensor layer_step_rows(const Tensor& x, const Tensor& q_proj, const Tensor& k_proj,
+                       const Tensor& v_proj, const Tensor& w_gamma, const Tensor& o_proj,
+                       const Tensor& wq, const Tensor& wk, const Tensor& cos, const Tensor& sin,
+                       const Tensor& meta, const Tensor& alpha, const Tensor& state,
+                       const Tensor& k_cache, const Tensor& v_cache, int64_t pos) {
+  const auto p = rows_linear(x, {q_proj, k_proj, v_proj, w_gamma}, {false, false, false, true});
+  const Tensor y = layer_step(p[0], p[1], p[2], p[3], wq, wk, cos, sin, meta, alpha, state, k_cache,
+                             v_cache, pos, true);
+  return rows_linear(y, {o_proj}, {false})[0];
+}
+
 }  // namespace
 
 PYBIND11_MODULE(lizard_torch, m) {
@@ -273,4 +311,7 @@ PYBIND11_MODULE(lizard_torch, m) {
   m.def("gla", &gla, nogil);
   m.def("swa", &swa, nogil);
   m.def("layer_step", &layer_step, nogil);
+  m.def("layer_step_rows", &layer_step_rows, nogil);
+  m.def("rows_linear", &rows_linear, nogil);
+  m.attr("ROWS_MAX") = LZ_ROWS_MAX;
 }

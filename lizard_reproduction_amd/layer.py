@@ -456,6 +456,31 @@ class LizardAttention(nn.Module):
         cache.pos = x.shape[1]
         return out, cache
 
+    def _projections(self):
+        return self.q_proj, self.k_proj, self.v_proj, self.W_gamma, self.o_proj
+
+    def _step_rows(self, x):
+        """Whether ``_ops.layer_step_rows`` may form the projections of x: few
+        enough rows of bf16, and plain nn.Linear modules that nothing hooks into,
+        patches or casts, with ordinary bf16 weights the kernel can read."""
+        if (x.dtype is not torch.bfloat16 or not 0 < x.shape[0] <= _ops.load().ROWS_MAX
+                or x.shape[2] % 8 or x.shape[2] != self.q_proj.in_features
+                or torch.is_autocast_enabled() or not _ops.plain()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or nn.modules.module._has_any_global_hook()):
+            return False
+        for m in self._projections():
+            if (type(m) is not nn.Linear or m.bias is not None or "forward" in m.__dict__
+                    or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                    or m._backward_pre_hooks):
+                return False
+            w = m.weight
+            if (type(w) is not nn.Parameter or w.dtype is not torch.bfloat16
+                    or not w.is_contiguous() or w.device != x.device or w.data_ptr() % 16
+                    or w.numel() * 2 >= 1 << 30):
+                return False
+        return x.data_ptr() % 16 == 0
+
     def _step_native(self, x, projections, cos, sin, cache):
         """Whether ``_ops.layer_step`` takes this step: the shapes the decode
         kernels take, and a cache as ``prefill`` and ``new_cache`` make it.  Any
@@ -489,6 +514,13 @@ class LizardAttention(nn.Module):
         if x.device.type != "cuda":
             raise ValueError("LizardAttention (hip backend) needs its input on a ROCm GPU")
         cos, sin = position_embeddings
+        if self._step_rows(x) and self._step_native(x, (x, x, x), cos, sin, cache):
+            out = _ops.load().layer_step_rows(
+                x.contiguous(), *(m.weight for m in self._projections()), self.phi_q.weight,
+                self.phi_k.weight, cos, sin, self.meta_tokens, self.alpha_blend, cache.state,
+                cache.k, cache.v, cache.pos)
+            cache.pos += 1
+            return out
         projections = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         if self._step_native(x, projections, cos, sin, cache):
             y = _ops.load().layer_step(*projections, self.W_gamma(x), self.phi_q.weight,

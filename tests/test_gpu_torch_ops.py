@@ -9,6 +9,7 @@ import torch.nn.functional as F
 
 from lizard_reproduction_amd import _ops, kernels
 from lizard_reproduction_amd.layer import LizardAttention
+from tests.helpers import max_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -162,3 +163,80 @@ def test_native_layer_step_equals_the_step_by_operators(monkeypatch, heads, kv, 
     theirs = _through_python(monkeypatch, run)
     for a, c in zip(ours, theirs):
         assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("rows, cols, sizes", [
+    (1, 8, [1]), (16, 64, [16, 17, 15, 1]), (3, 72, [33]), (5, 2048, [48, 16, 16, 1]),
+    (16, 2056, [100, 7]), (2, 4104, [16]), (7, 136, [512, 128, 128, 1])])
+def test_rows_linear_matches_the_product(rows, cols, sizes):
+    """Edges of the 16-row tiles, of the 64-column steps and of the waves' shares
+    of them (a share holds 4 steps of 64 columns in flight, 8 waves apart)."""
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(rows, 1, cols, device="cuda", generator=g).bfloat16()
+    w = [torch.randn(n, cols, device="cuda", generator=g).bfloat16() for n in sizes]
+    wide = [i % 2 == 1 for i in range(len(w))]
+    for y, m, f32 in zip(_ops.load().rows_linear(x, w, wide), w, wide):
+        exact = x.double() @ m.double().T
+        assert y.dtype == (torch.float32 if f32 else torch.bfloat16) and y.shape == exact.shape
+        assert torch.equal(y, y.bfloat16().to(y.dtype))
+        # half a bf16 unit, and fp32 sums of `cols` products of N(0, 1) values
+        bound = 2.0 ** -8 * exact.abs() + 2.0 ** -22 * cols
+        assert ((y.double() - exact).abs() <= bound).all()
+
+
+def _decode_layer(batch=3):
+    torch.manual_seed(5)
+    cfg = types.SimpleNamespace(hidden_size=256, num_attention_heads=4, num_key_value_heads=2)
+    layer = LizardAttention(cfg, 0, window=8, feature_dim=32).to("cuda", torch.bfloat16)
+    with torch.no_grad():
+        for n, p in layer.named_parameters():
+            p.normal_(0, 0.2 if n.startswith("phi") else 0.06)
+    x = torch.randn(batch, 20, 256, device="cuda").bfloat16()
+    angle = torch.rand(20, 64, device="cuda") * 6
+    return layer, x, (angle.cos().bfloat16(), angle.sin().bfloat16())
+
+
+def _decode(layer, x, tables):
+    _, cache = layer.prefill(x[:, :10], tuple(t[:10] for t in tables))
+    outs = [layer.step(x[:, t:t + 1], tuple(u[t:t + 1] for u in tables), cache)
+            for t in range(10, 20)]
+    return torch.cat(outs, 1), cache
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17])
+def test_step_with_its_projections_matches_the_forward(batch):
+    """Sixteen sequences are the most the skinny products take."""
+    layer, x, tables = _decode_layer(batch)
+    assert layer._step_rows(x[:, :1]) == (batch <= 16)
+    out, _ = _decode(layer, x, tables)
+    with torch.no_grad():
+        y = layer(x, tables)[0][:, 10:]
+    assert max_rel(out, y) <= 2e-2   # bf16 projections, outputs and o_proj, each rounded once
+
+
+def test_step_leaves_modules_that_do_more_to_their_forward():
+    """Hooked, patched, replaced, autocast and half-precision projections."""
+    layer, x, tables = _decode_layer()
+    plain, _ = _decode(layer, x, tables)
+    token = x[:, :1]
+    calls = []
+    handle = layer.k_proj.register_forward_hook(lambda *a: calls.append(1))
+    assert not layer._step_rows(token)
+    hooked, _ = _decode(layer, x, tables)
+    assert len(calls) == 11   # the prompt and ten steps
+    assert max_rel(hooked, plain) <= 2e-2
+    handle.remove()
+    assert layer._step_rows(token)
+    layer.q_proj.forward = lambda t, f=layer.q_proj.forward: 2 * f(t)
+    assert not layer._step_rows(token)
+    del layer.q_proj.forward
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not layer._step_rows(token)
+    o_proj = layer.o_proj
+    layer.o_proj = torch.nn.Sequential(o_proj)
+    assert not layer._step_rows(token)
+    layer.o_proj = torch.nn.Linear(256, 256, device="cuda", dtype=torch.bfloat16)   # a bias
+    assert not layer._step_rows(token)
+    layer.o_proj = o_proj
+    assert layer._step_rows(token) and not layer._step_rows(token.float())
+    assert not layer._step_rows(x.reshape(-1)[1:257].view(1, 1, 256))   # not 16-byte aligned
