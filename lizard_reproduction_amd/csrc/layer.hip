@@ -465,20 +465,25 @@ struct ProBwd {
   using C = Pro<T, FT, HT>;
   static constexpr int FP = C::FP, HP = C::HP, HK = C::HK, WP = C::WP, PARTS = C::PARTS;
   // feature groups: two where a row has two or more feature tiles and the
-  // per-group dx shares fit the LDS (head_dim <= 64)
-  static constexpr int NWF = FT >= 2 && HT <= 2 ? 2 : 1;
+  // per-group dx shares fit the LDS: each group's at head_dim <= 64, one at a
+  // time at head_dim 128 in bf16 (DX_TURNS; fp32's W and x tiles leave no room).
+  // With one group a wave held 465 registers there, one wave per SIMD: B=1
+  // L=4096, 32/8 heads, 128 features 208 -> 142 us, 64 features 116 -> 93 us
+  static constexpr bool DX_TURNS = HT == 4 && FT >= 2 && !C::SPLIT;
+  static constexpr int NWF = (FT >= 2 && HT <= 2) || DX_TURNS ? 2 : 1;
+  static constexpr int DXS = DX_TURNS ? 1 : NWF;         // dx shares held in LDS
   static constexpr int FTW = FT / NWF;                   // feature tiles per wave
   static constexpr int NW = PRO_WAVES * NWF, NT = 64 * NW;
   static constexpr int QP = lds_pitch(HP);    // x tiles [128][QP] bf16
   static constexpr int DP = lds_pitch(FP);    // dW tile [128][DP] bf16
   static constexpr int SP = 64 * NWF + 4;     // stage [128][SP] fp32: per group 32 dp, 32 dn
-  static constexpr int AP = HP + 4;           // dx shares [NWF][128][AP] fp32
+  static constexpr int AP = HP + 4;           // dx shares [DXS][128][AP] fp32
   static constexpr int BUF = imax(PRO_BLOCK * SP * 4, PRO_BLOCK * DP * 2);
   static constexpr int OFF_X = PARTS * FP * WP * 2;
   static constexpr int OFF_B = OFF_X + PARTS * PRO_BLOCK * QP * 2;
   // the dx shares take the buffer when they fit there, else they also span
   // the x tiles (then the next block waits for the epilogue before writing x)
-  static constexpr int DX = NWF * PRO_BLOCK * AP * 4;
+  static constexpr int DX = DXS * PRO_BLOCK * AP * 4;
   static constexpr bool DX_OVER_X = DX > BUF;
   static constexpr int OFF_DX = DX_OVER_X ? OFF_X : OFF_B;
   static constexpr int OFF_RED = imax(OFF_B + BUF, OFF_DX + DX);   // [NWF][4][128] row stats
@@ -500,9 +505,8 @@ struct ProBwd {
   // per SIMD has the registers for them, one in the split form with PRE (the
   // q blocks' only head: 1 % at config 5), none elsewhere (the two-workgroup
   // forms' second wave per SIMD hides the load latency instead, and held
-  // loads push them into spills; nor at FT = HT = 4, where a wave's own tiles
-  // already take every register)
-  static constexpr int GQ = OCC == 1 && NWF == 1 && FT * HT < 16 ? 4 : (PRE ? 1 : 0);
+  // loads push them into spills; at head_dim 128 they measured the same)
+  static constexpr int GQ = OCC == 1 && NWF == 1 ? 4 : (PRE ? 1 : 0);
   static constexpr int GQR = GQ > 0 ? GQ : 1;            // raw register sets held
 };
 
@@ -960,7 +964,26 @@ prologue_bwd_kernel(ProBwdArgs a) {
     }
 
     // ---- 6. dx = sum of the dx_phi shares + rope^T(drope) (+ dv sums) --------
-    {
+    if constexpr (K::DX_TURNS) {   // group 0's share, then group 1 adds its own to it
+      auto mine = [&](int ht, int q4) {
+        return reinterpret_cast<f32x4*>(dx_l + lrow * AP + 32 * ht + 8 * q4 + 4 * h);
+      };
+#pragma unroll
+      for (int turn = 0; turn < 2; ++turn) {
+        if (fh == turn) {
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              f32x4 v = {dacc[ht][4 * q4], dacc[ht][4 * q4 + 1], dacc[ht][4 * q4 + 2],
+                         dacc[ht][4 * q4 + 3]};
+              if (turn == 1) v += *mine(ht, q4);
+              *mine(ht, q4) = v;
+            }
+        }
+        if (turn == 0) __syncthreads();
+      }
+    } else {
       float* mine = dx_l + fh * PRO_BLOCK * AP;
 #pragma unroll
       for (int ht = 0; ht < HT; ++ht)
@@ -1008,7 +1031,7 @@ prologue_bwd_kernel(ProBwdArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = dr[e] * c[e] + sign * dr2[e] * s2[e];
 #pragma unroll
-        for (int g2 = 0; g2 < NWF; ++g2) {   // the shares in group order
+        for (int g2 = 0; g2 < K::DXS; ++g2) {   // the shares in group order
           const float* dxr = dx_l + (g2 * PRO_BLOCK + r) * AP + m0;
 #pragma unroll
           for (int e = 0; e < 8; ++e) out[e] += dxr[e];
@@ -1057,7 +1080,7 @@ prologue_bwd_kernel(ProBwdArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = dr[e] * c[e] + sign * dr2[e] * s2[e];
 #pragma unroll
-        for (int g2 = 0; g2 < NWF; ++g2) {   // the shares in group order
+        for (int g2 = 0; g2 < K::DXS; ++g2) {   // the shares in group order
           const float* dxr = dx_l + (g2 * PRO_BLOCK + r) * AP + m0;
 #pragma unroll
           for (int e = 0; e < 8; ++e) out[e] += dxr[e];
