@@ -313,3 +313,17 @@ def test_gla_value_tiles_in_place_match_oracle(features, dim, length, batch, hea
     grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(1))
     compare(gla_kernel(64), gla_reference, inputs, grad,
             label=f"value tiles F={features} D={dim} L={length} BH={batch * heads}")
+
+
+# records below 128 x 64 floats fold too: short sequences of few rows, every
+# segment one chunk, and enough rows for few segments of several chunks
+@pytest.mark.parametrize("batch, heads, length, features, dim, per_head", [
+    (1, 4, 256, 64, 64, False), (1, 2, 130, 32, 32, True), (3, 50, 330, 64, 32, True),
+    (2, 64, 450, 32, 64, False), (1, 128, 200, 64, 64, True)])
+def test_gla_walks_fold_few_small_records(batch, heads, length, features, dim, per_head):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=29)
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(2))
+    compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
+                                                      dtype=torch.float32),
+            inputs, grad, label=f"small folded F={features} D={dim} B*H={batch * heads} L={length}")
