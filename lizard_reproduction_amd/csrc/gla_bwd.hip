@@ -1380,6 +1380,15 @@ static hipError_t launch_gate_grad(const float* dG, const float* csum, const flo
   return hipGetLastError();
 }
 
+// Segments one walk workgroup takes in a row: two (G even) where one segment
+// each would be more workgroups than CUs, at one workgroup per CU.  Half as many
+// walks then take at most the rounds, and their entries, that the short ones
+// would (B=3 H=12 L=1777 F=D=96: 504 walks of two chunks in two rounds, dq 33 and dkv 39 us; 252 of four in
+// one, 26 and 32 us).
+static int gla_bwd_walk_segments(int BH, int G) {
+  return G % 2 == 0 && BH * G > device_geom().cus ? 2 : 1;
+}
+
 template <int FP, int DP, typename OutT, bool VEC>
 static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v, const float* lg,
                                    const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
@@ -1416,9 +1425,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
                               D, rows.ld, gate, G, cps, KG, fold, st);
     if (e != hipSuccess) return e;
   }
-  // the walks take two segments per workgroup while that still gives one
-  // workgroup per CU: fewer, longer walks
-  const int M = (G % 2 == 0 && BH * G / 2 >= device_geom().cus) ? 2 : 1;
+  const int M = gla_bwd_walk_segments(BH, G);
   const WalkGrid wg = walk_grid(BH * G / M, KG);
   const float* flam = fseg + (size_t)BH * G * SEG;
   // One segment per (b, h): the dq and dkv walks of a (b, h) run in one

@@ -327,3 +327,17 @@ def test_gla_walks_fold_few_small_records(batch, heads, length, features, dim, p
     compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
                                                       dtype=torch.float32),
             inputs, grad, label=f"small folded F={features} D={dim} B*H={batch * heads} L={length}")
+
+
+# between one and two times as many segments as CUs: the backward walks take two
+# segments each, over folded and over scanned records
+@pytest.mark.parametrize("batch, heads, length, features, dim, per_head", [
+    (10, 15, 100, 24, 40, False), (2, 25, 384, 64, 64, True), (1, 43, 450, 128, 96, False),
+    (1, 20, 1000, 256, 64, True)])
+def test_gla_backward_walks_of_two_segments(batch, heads, length, features, dim, per_head):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=31)
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(3))
+    compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
+                                                      dtype=torch.float32),
+            inputs, grad, label=f"two segments F={features} D={dim} B*H={batch * heads} L={length}")
