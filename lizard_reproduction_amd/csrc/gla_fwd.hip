@@ -1246,13 +1246,19 @@ bool gla_dims_supported(int F, int D) {
   return dp <= 128 && (fp <= 128 || dp <= 64);
 }
 
-// Segments per (b, h) so that B*H*G workgroups fill the GPU: two forward
-// workgroups per CU up to F = 128, one beyond (the LDS of a 256-wide chunk).
+// Segments per (b, h): as many as still run in one round of workgroups, two
+// forward workgroups per CU up to F = 128, one beyond (the LDS of a 256-wide
+// chunk).  One segment more would fill the round and leave a few walks of the
+// same length to a second one (forward + backward, us, against the split
+// rounded up: B*H = 40 L = 4096 F = D = 128 275 -> 240, G 13 -> 11; B*H = 160
+// L = 2048 458 -> 363, G 4 -> 3; B*H = 297 L = 1024 F = D = 64 252 -> 232 and
+// B*H = 250 L = 2048 F = 256 D = 64 743 -> 589, one segment; none of 35 shapes
+// slower, the same split where B*H divides the round).
 void gla_segments(int BH, int L, int F, int* G, int* cps) {
   const int NT = (L + GLA_C - 1) / GLA_C;
   const bool wide = gla_padded_dim(F) > 128;   // walks run one workgroup per CU
   const int target = wide ? gla_target_wg() / 2 : gla_target_wg();
-  int g = (target + BH - 1) / BH;
+  int g = target / BH;
   g = g < 1 ? 1 : (g > NT ? NT : g);
   // Wide walks: segments half as long as one walk, each walk taking two
   // (gla_walk_segments).  The segment state passes, which fit two workgroups

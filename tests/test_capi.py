@@ -262,6 +262,17 @@ def test_segment_split():
     assert segments(128, 4096, f=256) == (4, 16)   # config-5 layer shape: 2 segments per walk
 
 
+# B*H that does not divide the round of workgroups: the split that still runs in
+# one round (segments() above agrees with it where B*H divides)
+@pytest.mark.parametrize("b, h, length, f, split", [
+    (1, 40, 4096, 128, 11), (5, 32, 2048, 64, 3), (9, 33, 1024, 64, 1), (1, 40, 4096, 256, 11),
+    (1, 250, 2048, 256, 1), (3, 32, 64, 128, 1), (1, 7, 130, 32, 3)])
+def test_segments_stay_within_one_round(lib, b, h, length, f, split):
+    assert split == 1 or b * h * split <= 512
+    assert lib.lz_gla_fwd_workspace_bytes(b, h, length, f, 64, 0, 64) == \
+        4 * seg_floats(b * h, split, f, 64)
+
+
 def test_swa_workspace_sizes(lib):
     # delta [BH, L] plus dmeta partials [BH * ceil(L/128), n_meta]
     assert lib.lz_swa_bwd_workspace_bytes(1, 32, 2048, 64, 4) == 4 * (32 * 2048 + 32 * 16 * 4)

@@ -341,3 +341,17 @@ def test_gla_backward_walks_of_two_segments(batch, heads, length, features, dim,
     compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
                                                       dtype=torch.float32),
             inputs, grad, label=f"two segments F={features} D={dim} B*H={batch * heads} L={length}")
+
+
+# B*H that does not divide the round of workgroups: folded and scanned splits and one
+# segment, with a shorter last one
+@pytest.mark.parametrize("batch, heads, length, features, dim, per_head", [
+    (2, 40, 500, 64, 64, False), (5, 32, 321, 128, 64, True), (9, 33, 130, 64, 32, False),
+    (10, 15, 200, 256, 64, True)])
+def test_gla_split_within_one_round(batch, heads, length, features, dim, per_head):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=37)
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(4))
+    compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
+                                                      dtype=torch.float32),
+            inputs, grad, label=f"one round F={features} D={dim} B*H={batch * heads} L={length}")
