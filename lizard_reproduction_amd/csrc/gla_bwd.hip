@@ -238,8 +238,9 @@ __device__ __forceinline__ void gla_bwd_dq_body(
   float* zp = reinterpret_cast<float*>(smem + Cfg::OFF_ZP);
   float* rdec = reinterpret_cast<float*>(smem + Cfg::OFF_R);
 
-  // a workgroup walks M consecutive segments (seg .. seg + M - 1)
-  const int nwg = G / M;
+  // a workgroup walks M consecutive segments (seg .. seg + M - 1), the last of
+  // a row those that are left
+  const int nwg = (G + M - 1) / M;
   int blk;
   if (!walk_block(xper, nxcd, nblk, blk)) return;
   const int bh = blk / nwg, seg = (blk % nwg) * M;
@@ -909,12 +910,13 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
   float* gz = reinterpret_cast<float*>(smem + Cfg::OFF_GZ);
   float* rdec = reinterpret_cast<float*>(smem + Cfg::OFF_R);
 
-  // a workgroup walks M consecutive segments (seg0 .. seg0 + M - 1) in reverse,
+  // a workgroup walks M consecutive segments (seg0 .. seg0 + M - 1, or those
+  // that are left) in reverse,
   // entering with the state that flows into the last of them
-  const int nwg = G / M;
+  const int nwg = (G + M - 1) / M;
   int blk;
   if (!walk_block(xper, nxcd, nblk, blk, rev != 0)) return;
-  const int bh = blk / nwg, seg0 = (blk % nwg) * M, seg = seg0 + M - 1;
+  const int bh = blk / nwg, seg0 = (blk % nwg) * M, seg = min(seg0 + M, G) - 1;
   const int NT = (L + C - 1) / C;
   const int n0 = seg0 * cps, n1 = min(NT, n0 + M * cps);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -1380,13 +1382,18 @@ static hipError_t launch_gate_grad(const float* dG, const float* csum, const flo
   return hipGetLastError();
 }
 
-// Segments one walk workgroup takes in a row: two (G even) where one segment
-// each would be more workgroups than CUs, at one workgroup per CU.  Half as many
-// walks then take at most the rounds, and their entries, that the short ones
-// would (B=3 H=12 L=1777 F=D=96: 504 walks of two chunks in two rounds, dq 33 and dkv 39 us; 252 of four in
-// one, 26 and 32 us).
+// Segments one walk workgroup takes in a row: two where one segment each would
+// be more workgroups than CUs, at one workgroup per CU.  Half as many walks then
+// take at most the rounds, and their entries, that the short ones would (B=3
+// H=12 L=1777 F=D=96: 504 walks of two chunks in two rounds, dq 33 and dkv 39
+// us; 252 of four in one, 26 and 32 us).  With an odd G the last walk of a row
+// takes one, and two only where the walks then run in one round: three
+// segments in walks of two and one take as long as two rounds of one (B=1 L=4096,
+// backward, us: H=36 F=D=128 149 -> 135, F=D=64 90 -> 85, H=40 F=256 D=64 197 ->
+// 189).
 static int gla_bwd_walk_segments(int BH, int G) {
-  return G % 2 == 0 && BH * G > device_geom().cus ? 2 : 1;
+  const int cus = device_geom().cus;
+  return BH * G > cus && (G % 2 == 0 || (G > 1 && BH * (G / 2 + 1) <= cus)) ? 2 : 1;
 }
 
 template <int FP, int DP, typename OutT, bool VEC>
@@ -1426,7 +1433,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     if (e != hipSuccess) return e;
   }
   const int M = gla_bwd_walk_segments(BH, G);
-  const WalkGrid wg = walk_grid(BH * G / M, KG);
+  const WalkGrid wg = walk_grid(BH * ((G + M - 1) / M), KG);
   const float* flam = fseg + (size_t)BH * G * SEG;
   // One segment per (b, h): the dq and dkv walks of a (b, h) run in one
   // workgroup, one after the other (gla_bwd_fused_kernel): one launch, and

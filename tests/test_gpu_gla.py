@@ -355,3 +355,16 @@ def test_gla_split_within_one_round(batch, heads, length, features, dim, per_hea
     compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
                                                       dtype=torch.float32),
             inputs, grad, label=f"one round F={features} D={dim} B*H={batch * heads} L={length}")
+
+
+# an odd number of segments: the last backward walk of each row takes one (scanned and
+# folded records)
+@pytest.mark.parametrize("batch, heads, length, features, dim, per_head", [
+    (1, 40, 430, 64, 64, True), (2, 50, 192, 128, 64, False), (1, 20, 800, 256, 64, True)])
+def test_gla_backward_walks_of_odd_segments(batch, heads, length, features, dim, per_head):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=41)
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(5))
+    compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
+                                                      dtype=torch.float32),
+            inputs, grad, label=f"odd segments F={features} D={dim} B*H={batch * heads} L={length}")
