@@ -220,18 +220,70 @@ Tensor swa(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& meta
 // the layer's decode step between its projections and o_proj
 // ---------------------------------------------------------------------------
 
+bool is(const Tensor& t, at::IntArrayRef sizes, const Tensor& like) {
+  return t.defined() && t.sizes() == sizes && t.device() == like.device();
+}
+
+// Whether layer_step's launches, which take every size from the layer (heads, kv,
+// window, hd), fit these tensors: shapes, devices, and the layout and types of the
+// buffers that are written in place.  Projections that are formed later are left
+// out.  A step that does not fit goes operator by operator, which casts or refuses
+// what it is given.
+bool step_takes(const std::vector<Tensor>& projections, const Tensor& wq, const Tensor& wk,
+                const Tensor& cos, const Tensor& sin, const Tensor& state, const Tensor& k_cache,
+                const Tensor& v_cache, int64_t heads, int64_t kv, int64_t window, int64_t hd,
+                int64_t pos) {
+  if (state.dim() != 3 || wq.dim() != 2 || pos < 0) return false;
+  const int64_t b = state.size(0), f = wq.size(0), nf = 2 * f;
+  for (size_t i = 0; i < projections.size(); ++i)
+    if (!is(projections[i], {b, 1, (i ? kv : heads) * hd}, state)) return false;
+  const bool rope = cos.sizes() == sin.sizes() &&
+                    (is(cos, {1, hd}, state) || is(cos, {1, 1, hd}, state) ||
+                     is(cos, {b, 1, hd}, state));
+  if (b <= 0 || !rope || sin.device() != state.device() || !is(wq, {f, hd}, state) ||
+      !is(wk, {f, hd}, state) || !is(state, {b, heads, nf * hd + nf}, state) ||
+      state.scalar_type() != at::kFloat || !state.is_contiguous())
+    return false;
+  for (const Tensor* t : {&k_cache, &v_cache})
+    if (!is(*t, {b, kv, window, hd}, state) || t->scalar_type() != at::kBFloat16 ||
+        !t->is_contiguous())
+      return false;
+  return true;
+}
+
+// Whether rows_linear takes w [n, K] (any n < 1) for x's rows of K columns
+bool row_weight(const Tensor& w, int64_t n, int64_t cols, const Tensor& x) {
+  return w.dim() == 2 && (n < 1 || w.size(0) == n) && w.size(1) == cols &&
+         w.scalar_type() == at::kBFloat16 && w.is_contiguous() && w.device() == x.device() &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && w.numel() < (int64_t{1} << 29);
+}
+
+// Whether layer_step_rows can form the projections of x [B, 1, hidden] by weights
+// {q_proj, k_proj, v_proj, W_gamma, o_proj}: each [its outputs, its inputs]
+bool rows_take(const Tensor& x, const std::vector<Tensor>& w, int64_t q_width, int64_t kv_width) {
+  return x.dim() == 3 && x.size(1) == 1 && x.size(0) > 0 && x.size(0) <= LZ_ROWS_MAX &&
+         x.scalar_type() == at::kBFloat16 && x.size(2) > 0 && x.size(2) % 8 == 0 &&
+         reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && w.size() == 5 &&
+         row_weight(w[0], q_width, x.size(2), x) && row_weight(w[1], kv_width, x.size(2), x) &&
+         row_weight(w[2], kv_width, x.size(2), x) && row_weight(w[3], 0, x.size(2), x) &&
+         row_weight(w[4], 0, q_width, x);
+}
+
 // One token per sequence at position pos: the prologue on the projections' rows
 // (qp [B, 1, heads hd], kp, vp [B, 1, kv hd]), the GLA step on `state`, and the
 // window step that puts the token's key and value into their cache slot and
-// blends the two branches.  layer.py has checked the shapes; state, k_cache and
-// v_cache are contiguous, of their dtypes.  Returns [B, 1, heads hd] (bf16 when
-// out_bf16, else fp32).
+// blends the two branches.  For tensors that step_takes; others raise.  Returns
+// [B, 1, heads hd] (bf16 when out_bf16, else fp32).
 Tensor layer_step(Tensor qp, Tensor kp, Tensor vp, const Tensor& z, Tensor wq, Tensor wk,
                   Tensor cos, Tensor sin, const Tensor& meta, const Tensor& alpha,
-                  const Tensor& state, const Tensor& k_cache, const Tensor& v_cache, int64_t pos,
+                  const Tensor& state, const Tensor& k_cache, const Tensor& v_cache,
+                  int64_t heads_, int64_t kv_, int64_t window_, int64_t hd_, int64_t pos,
                   bool out_bf16) {
-  const int b = i32(k_cache.size(0)), kv = i32(k_cache.size(1)), window = i32(k_cache.size(2)),
-            hd = i32(k_cache.size(3)), heads = i32(state.size(1)), f = i32(wq.size(0));
+  TORCH_CHECK(step_takes({qp, kp, vp}, wq, wk, cos, sin, state, k_cache, v_cache, heads_, kv_,
+                         window_, hd_, pos),
+              "layer_step: tensors that do not fit the layer's sizes");
+  const int b = i32(state.size(0)), heads = i32(heads_), kv = i32(kv_), window = i32(window_),
+            hd = i32(hd_), f = i32(wq.size(0));
   bool all_bf16 = true;
   for (const Tensor* t : {&qp, &kp, &vp, &wq, &wk, &cos, &sin})
     all_bf16 = all_bf16 && t->scalar_type() == at::kBFloat16;
@@ -270,11 +322,17 @@ Tensor layer_step(Tensor qp, Tensor kp, Tensor vp, const Tensor& z, Tensor wq, T
 // as fp32
 std::vector<Tensor> rows_linear(const Tensor& x, const std::vector<Tensor>& w,
                                 const std::vector<bool>& wide) {
+  TORCH_CHECK(w.size() <= LZ_ROWS_MATS && w.size() == wide.size(), "rows_linear: at most ",
+              LZ_ROWS_MATS, " matrices");
+  TORCH_CHECK(x.dim() > 0 && x.numel() && x.scalar_type() == at::kBFloat16 && x.is_contiguous(),
+              "rows_linear: x must be contiguous bf16 rows");
   const int rows = i32(x.numel() / x.size(-1)), cols = i32(x.size(-1)), mats = i32(w.size());
   const void* wp[LZ_ROWS_MATS];
   void* yp[LZ_ROWS_MATS];
   int n[LZ_ROWS_MATS], f32out[LZ_ROWS_MATS];
-  TORCH_CHECK(mats <= LZ_ROWS_MATS, "rows_linear: at most ", LZ_ROWS_MATS, " matrices");
+  for (const Tensor& m : w)
+    TORCH_CHECK(row_weight(m, 0, cols, x), "rows_linear: matrices must be contiguous bf16 [n, ",
+                cols, "] on x's device, 16-byte aligned");
   std::vector<Tensor> y;
   for (int i = 0; i < mats; ++i) {
     auto sizes = x.sizes().vec();
@@ -290,18 +348,20 @@ std::vector<Tensor> rows_linear(const Tensor& x, const std::vector<Tensor>& w,
   return y;
 }
 
-// The whole step of a bf16 layer whose projections are plain matrices, for x
-// [B, 1, hidden], B <= LZ_ROWS_MAX: the four projections of x in one launch
+// The whole step of a bf16 layer whose projections are plain matrices (rows_take),
+// for x [B, 1, hidden], B <= LZ_ROWS_MAX: the four projections of x in one launch
 // (the gate's logit as fp32, of its bf16 value), the step, and o_proj.
-Tensor layer_step_rows(const Tensor& x, const Tensor& q_proj, const Tensor& k_proj,
-                       const Tensor& v_proj, const Tensor& w_gamma, const Tensor& o_proj,
-                       const Tensor& wq, const Tensor& wk, const Tensor& cos, const Tensor& sin,
-                       const Tensor& meta, const Tensor& alpha, const Tensor& state,
-                       const Tensor& k_cache, const Tensor& v_cache, int64_t pos) {
-  const auto p = rows_linear(x, {q_proj, k_proj, v_proj, w_gamma}, {false, false, false, true});
+Tensor layer_step_rows(const Tensor& x, const std::vector<Tensor>& w, const Tensor& wq,
+                       const Tensor& wk, const Tensor& cos, const Tensor& sin, const Tensor& meta,
+                       const Tensor& alpha, const Tensor& state, const Tensor& k_cache,
+                       const Tensor& v_cache, int64_t heads, int64_t kv, int64_t window,
+                       int64_t hd, int64_t pos) {
+  TORCH_CHECK(rows_take(x, w, heads * hd, kv * hd),
+              "layer_step_rows: projections that do not fit the layer's sizes");
+  const auto p = rows_linear(x.contiguous(), {w[0], w[1], w[2], w[3]}, {false, false, false, true});
   const Tensor y = layer_step(p[0], p[1], p[2], p[3], wq, wk, cos, sin, meta, alpha, state, k_cache,
-                             v_cache, pos, true);
-  return rows_linear(y, {o_proj}, {false})[0];
+                             v_cache, heads, kv, window, hd, pos, true);
+  return rows_linear(y, {w[4]}, {false})[0];
 }
 
 }  // namespace
@@ -310,6 +370,8 @@ PYBIND11_MODULE(lizard_torch, m) {
   const auto nogil = py::call_guard<py::gil_scoped_release>();
   m.def("gla", &gla, nogil);
   m.def("swa", &swa, nogil);
+  m.def("step_takes", &step_takes, nogil);
+  m.def("rows_take", &rows_take, nogil);
   m.def("layer_step", &layer_step, nogil);
   m.def("layer_step_rows", &layer_step_rows, nogil);
   m.def("rows_linear", &rows_linear, nogil);

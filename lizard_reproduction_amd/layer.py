@@ -462,44 +462,36 @@ class LizardAttention(nn.Module):
     def _step_rows(self, x):
         """Whether ``_ops.layer_step_rows`` may form the projections of x: few
         enough rows of bf16, and plain nn.Linear modules that nothing hooks into,
-        patches or casts, with ordinary bf16 weights the kernel can read."""
-        if (x.dtype is not torch.bfloat16 or not 0 < x.shape[0] <= _ops.load().ROWS_MAX
-                or x.shape[2] % 8 or x.shape[2] != self.q_proj.in_features
+        patches or casts, with ordinary bf16 weights of the layer's sizes."""
+        if (x.dtype is not torch.bfloat16 or x.shape[2] != self.q_proj.in_features
                 or torch.is_autocast_enabled() or not _ops.plain()
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or nn.modules.module._has_any_global_hook()):
             return False
+        weights = []
         for m in self._projections():
             if (type(m) is not nn.Linear or m.bias is not None or "forward" in m.__dict__
                     or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                    or m._backward_pre_hooks):
+                    or m._backward_pre_hooks or type(m.weight) is not nn.Parameter):
                 return False
-            w = m.weight
-            if (type(w) is not nn.Parameter or w.dtype is not torch.bfloat16
-                    or not w.is_contiguous() or w.device != x.device or w.data_ptr() % 16
-                    or w.numel() * 2 >= 1 << 30):
-                return False
-        return x.data_ptr() % 16 == 0
+            weights.append(m.weight)
+        return _ops.load().rows_take(x, weights, self.heads * self.head_dim,
+                                     self.kv_heads * self.head_dim)
 
     def _step_native(self, x, projections, cos, sin, cache):
-        """Whether ``_ops.layer_step`` takes this step: the shapes the decode
-        kernels take, and a cache as ``prefill`` and ``new_cache`` make it.  Any
-        other step goes operator by operator, which casts or refuses it."""
-        b, hd, nf = x.shape[0], self.head_dim, 2 * self.phi_q.weight.shape[0]
-        ring = (b, self.kv_heads, self.window, hd)
-        return (b > 0 and _ops.plain() and self._fused(*projections, cos, sin)
-                and kernels.gla_native(nf, hd)
-                and tuple(cos.shape) == tuple(sin.shape)
-                and tuple(cos.shape) in ((1, hd), (1, 1, hd), (b, 1, hd))
-                and type(cache.pos) is int and cache.pos >= 0
+        """Whether ``_ops.layer_step`` takes this step: projections (none: those
+        ``_step_rows`` allows), weights and tables of the layer's sizes, the shapes
+        the decode kernels take, and a cache as ``prefill`` and ``new_cache`` make
+        it.  Any other step goes operator by operator, which casts or refuses it."""
+        return (_ops.plain() and type(cache.pos) is int
                 and self.window <= kernels.SWA_DECODE_MAX_WINDOW
-                and tuple(cache.state.shape) == (b, self.heads, nf * hd + nf)
-                and cache.state.dtype is torch.float32 and cache.state.is_contiguous()
-                and all(tuple(t.shape) == ring and t.dtype is torch.bfloat16
-                        and t.is_contiguous() and t.device == x.device
-                        for t in (cache.k, cache.v))
+                and self._fused(*(projections or (x, x, x)), cos, sin)
+                and kernels.gla_native(2 * self.phi_q.weight.shape[0], self.head_dim)
+                and tuple(cache.state.shape[:1]) == tuple(x.shape[:1])
                 and cache.state.device == x.device
-                and all(t.device == x.device for t in (cos, sin)))
+                and _ops.load().step_takes(list(projections), self.phi_q.weight, self.phi_k.weight,
+                                           cos, sin, cache.state, cache.k, cache.v, self.heads,
+                                           self.kv_heads, self.window, self.head_dim, cache.pos))
 
     @torch.no_grad()
     def step(self, hidden_states, position_embeddings, cache):
@@ -514,19 +506,20 @@ class LizardAttention(nn.Module):
         if x.device.type != "cuda":
             raise ValueError("LizardAttention (hip backend) needs its input on a ROCm GPU")
         cos, sin = position_embeddings
-        if self._step_rows(x) and self._step_native(x, (x, x, x), cos, sin, cache):
+        sizes = self.heads, self.kv_heads, self.window, self.head_dim
+        if self._step_rows(x) and self._step_native(x, (), cos, sin, cache):
             out = _ops.load().layer_step_rows(
-                x.contiguous(), *(m.weight for m in self._projections()), self.phi_q.weight,
+                x, [m.weight for m in self._projections()], self.phi_q.weight,
                 self.phi_k.weight, cos, sin, self.meta_tokens, self.alpha_blend, cache.state,
-                cache.k, cache.v, cache.pos)
+                cache.k, cache.v, *sizes, cache.pos)
             cache.pos += 1
             return out
         projections = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         if self._step_native(x, projections, cos, sin, cache):
             y = _ops.load().layer_step(*projections, self.W_gamma(x), self.phi_q.weight,
                                        self.phi_k.weight, cos, sin, self.meta_tokens,
-                                       self.alpha_blend, cache.state, cache.k, cache.v, cache.pos,
-                                       x.dtype == torch.bfloat16)
+                                       self.alpha_blend, cache.state, cache.k, cache.v, *sizes,
+                                       cache.pos, x.dtype == torch.bfloat16)
             cache.pos += 1
             return self.o_proj(y.to(x.dtype))
         z, fq, fk, qr, kr, v = self._operands(x, position_embeddings, projections)

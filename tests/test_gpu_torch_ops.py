@@ -240,3 +240,23 @@ def test_step_leaves_modules_that_do_more_to_their_forward():
     layer.o_proj = o_proj
     assert layer._step_rows(token) and not layer._step_rows(token.float())
     assert not layer._step_rows(x.reshape(-1)[1:257].view(1, 1, 256))   # not 16-byte aligned
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name, inputs, outputs, error", [
+    ("phi_k", 64, 16, ValueError), ("k_proj", 256, 64, ValueError), ("v_proj", 256, 256, ValueError),
+    ("q_proj", 256, 128, ValueError), ("q_proj", 128, 256, RuntimeError),
+    ("k_proj", 128, 128, RuntimeError), ("o_proj", 128, 256, RuntimeError)])
+def test_step_refuses_modules_of_other_sizes(dtype, name, inputs, outputs, error):
+    """The errors of the operators' step (prologue_forward's and torch's), and the
+    layer decodes on once its own module is back."""
+    layer, x, tables = _decode_layer()
+    layer, x, tables = layer.to(dtype), x.to(dtype), tuple(t.to(dtype) for t in tables)
+    plain, _ = _decode(layer, x, tables)
+    _, cache = layer.prefill(x[:, :10], tuple(t[:10] for t in tables))
+    own = getattr(layer, name)
+    setattr(layer, name, torch.nn.Linear(inputs, outputs, bias=False, device="cuda", dtype=dtype))
+    with pytest.raises(error):
+        layer.step(x[:, 10:11], tuple(t[10:11] for t in tables), cache)
+    setattr(layer, name, own)
+    assert torch.equal(_decode(layer, x, tables)[0], plain)

@@ -8,6 +8,7 @@ import torch
 from transformers import LlamaConfig, LlamaForCausalLM
 from transformers.models.llama.modeling_llama import LlamaAttention, LlamaRotaryEmbedding
 
+from lizard_reproduction_amd import _ops
 from lizard_reproduction_amd import layer as hip_layer
 from oracle import lizard_oracle as lo
 
@@ -339,3 +340,104 @@ def test_rounded_oracle_layer_applies_its_rounding_points():
     lo.round_bf16(t).backward(up)
     assert torch.equal(lo.round_bf16(t).detach(), t.detach().bfloat16().double())
     assert torch.equal(t.grad, up.bfloat16().double())
+
+
+# -- the decode step's choice of path (no launch: the gates read shapes) --------
+
+def decode_layer(dtype=torch.bfloat16, feature_dim=32):
+    return hip_layer.LizardAttention(tiny_config(), 0, window=8,
+                                     feature_dim=feature_dim).to(dtype)
+
+
+def step_gates(layer, batch=2):
+    """(the projections formed natively, the step between them native) for one
+    token of each of `batch` sequences."""
+    dtype = layer.W_gamma.weight.dtype
+    x = torch.randn(batch, 1, 128).to(dtype)
+    cos, sin = (torch.randn(1, 32).to(dtype) for _ in range(2))
+    cache = layer.new_cache(batch, "cpu")
+    rows = layer._step_rows(x)
+    if rows:
+        return rows, layer._step_native(x, (), cos, sin, cache)
+    try:
+        projections = layer.q_proj(x), layer.k_proj(x), layer.v_proj(x)
+    except RuntimeError:   # torch refuses the product
+        return False, False
+    return rows, layer._step_native(x, projections, cos, sin, cache)
+
+
+def linear(inputs, outputs, dtype):
+    return torch.nn.Linear(inputs, outputs, bias=False, dtype=dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name, inputs, outputs, native", [
+    ("phi_k", 32, 16, False), ("phi_k", 32, 40, False), ("phi_k", 16, 32, False),
+    ("phi_q", 32, 16, False),              # the state holds 32 features
+    ("q_proj", 128, 96, False), ("q_proj", 120, 128, False), ("k_proj", 128, 32, False),
+    ("k_proj", 64, 64, False), ("v_proj", 64, 64, False), ("v_proj", 128, 128, False),
+    ("o_proj", 64, 128, True)])            # the step is native, o_proj's product torch's
+def test_native_step_leaves_modules_of_other_sizes(dtype, name, inputs, outputs, native):
+    """The native step takes its sizes from the layer, so it must not run on a
+    weight of another size: the operators refuse or cast that."""
+    layer = decode_layer(dtype)
+    assert step_gates(layer) == (dtype is torch.bfloat16, True)
+    setattr(layer, name, linear(inputs, outputs, dtype))
+    rows, step = step_gates(layer)
+    if name.startswith("phi"):
+        assert not step
+    else:
+        assert (rows, step) == (False, native)
+
+
+def test_native_step_leaves_caches_and_tables_of_other_sizes():
+    layer = decode_layer()
+    x = torch.randn(2, 1, 128).bfloat16()
+    table = torch.randn(1, 32).bfloat16()
+
+    def native(cos=table, sin=table, **changes):
+        cache = layer.new_cache(2, "cpu")
+        for name, value in changes.items():
+            setattr(cache, name, value(getattr(cache, name)))
+        return layer._step_native(x, (), cos, sin, cache)
+    assert native() and native(table[None], table[None])
+    assert native(table.expand(2, 1, 32), table.expand(2, 1, 32))
+    assert not native(table[:, :16], table[:, :16]) and not native(table, table[:, :16])
+    assert not native(table.expand(3, 1, 32), table.expand(3, 1, 32))
+    for name in ("k", "v"):
+        assert not native(**{name: lambda t: t[:, :1]})
+        assert not native(**{name: lambda t: t[:, :, :4]})
+        assert not native(**{name: lambda t: t.float()})
+        assert not native(**{name: lambda t: t.transpose(1, 2).contiguous().transpose(1, 2)})
+    for change in (lambda t: t[:1], lambda t: t[:, :2], lambda t: t[..., :-1], torch.Tensor.double):
+        assert not native(state=change)
+    assert not native(pos=lambda p: -1) and not native(pos=float)
+
+
+def test_products_of_rows_refuse_matrices_of_other_sizes():
+    """Refused before any launch: a narrower matrix would be read past its end."""
+    rows_linear = _ops.load().rows_linear
+    x = torch.zeros(2, 1, 64, dtype=torch.bfloat16)
+    for w in (linear(56, 16, torch.bfloat16), linear(64, 16, torch.float32)):
+        with pytest.raises(RuntimeError, match="matrices must be"):
+            rows_linear(x, [w.weight.detach()], [False])
+    with pytest.raises(RuntimeError, match="matrices must be"):
+        rows_linear(x, [torch.zeros(64, 16, dtype=torch.bfloat16).T], [False])
+    with pytest.raises(RuntimeError, match="x must be"):
+        rows_linear(x.float(), [torch.zeros(16, 64, dtype=torch.bfloat16)], [False])
+
+
+def test_native_step_itself_refuses_what_does_not_fit():
+    """Called past the gates, the module's entries raise before any launch."""
+    layer, ops = decode_layer(), _ops.load()
+    cache = layer.new_cache(2, "cpu")
+    x, table = torch.zeros(2, 1, 128).bfloat16(), torch.zeros(1, 32).bfloat16()
+    kv = torch.zeros(2, 1, 64).bfloat16()
+    rest = (layer.phi_q.weight, linear(32, 16, torch.bfloat16).weight, table, table,
+            layer.meta_tokens, layer.alpha_blend, cache.state, cache.k, cache.v, 4, 2, 8, 32, 0)
+    with pytest.raises(RuntimeError, match="layer's sizes"):
+        ops.layer_step(x, kv, kv, x[..., :1], *rest, True)
+    weights = [m.weight for m in layer._projections()]
+    weights[1] = linear(128, 32, torch.bfloat16).weight
+    with pytest.raises(RuntimeError, match="layer's sizes"):
+        ops.layer_step_rows(x, weights, *rest)
