@@ -265,12 +265,13 @@ bool rows_take(const Tensor& x, const std::vector<Tensor>& w, int64_t q_width, i
          x.scalar_type() == at::kBFloat16 && x.size(2) > 0 && x.size(2) % 8 == 0 &&
          reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && w.size() == 5 &&
          row_weight(w[0], q_width, x.size(2), x) && row_weight(w[1], kv_width, x.size(2), x) &&
-         row_weight(w[2], kv_width, x.size(2), x) && row_weight(w[3], 0, x.size(2), x) &&
+         row_weight(w[2], kv_width, x.size(2), x) && row_weight(w[3], 1, x.size(2), x) &&
          row_weight(w[4], 0, q_width, x);
 }
 
 // One token per sequence at position pos: the prologue on the projections' rows
-// (qp [B, 1, heads hd], kp, vp [B, 1, kv hd]), the GLA step on `state`, and the
+// (qp [B, 1, heads hd], kp, vp [B, 1, kv hd]), the GLA step on `state` with the
+// token's gate logit z [B, 1, 1] (a logit per head goes by operators), and the
 // window step that puts the token's key and value into their cache slot and
 // blends the two branches.  For tensors that step_takes; others raise.  Returns
 // [B, 1, heads hd] (bf16 when out_bf16, else fp32).
@@ -282,6 +283,7 @@ Tensor layer_step(Tensor qp, Tensor kp, Tensor vp, const Tensor& z, Tensor wq, T
   TORCH_CHECK(step_takes({qp, kp, vp}, wq, wk, cos, sin, state, k_cache, v_cache, heads_, kv_,
                          window_, hd_, pos),
               "layer_step: tensors that do not fit the layer's sizes");
+  TORCH_CHECK(is(z, {qp.size(0), 1, 1}, state), "layer_step: one gate logit per token expected");
   const int b = i32(state.size(0)), heads = i32(heads_), kv = i32(kv_), window = i32(window_),
             hd = i32(hd_), f = i32(wq.size(0));
   bool all_bf16 = true;

@@ -405,7 +405,7 @@ class LizardAttention(nn.Module):
         k = torch.zeros(shape, device=device, dtype=torch.bfloat16)
         return LizardCache(state, k, torch.zeros_like(k), 0)
 
-    def _operands(self, x, position_embeddings, projections=None):
+    def _operands(self, x, position_embeddings, projections=None, gate=None):
         kernels._refuse_capture("LizardAttention")
         if x.device.type != "cuda":
             raise ValueError("LizardAttention (hip backend) needs its input on a ROCm GPU")
@@ -418,7 +418,7 @@ class LizardAttention(nn.Module):
                              f"{self.head_dim} is not one: F <= 256, D <= 128, D <= 64 when "
                              "F > 128)")
         # the gate logit: the GLA kernels take logsigmoid of it themselves
-        z = self.W_gamma(x).float().squeeze(-1).contiguous()
+        z = (self.W_gamma(x) if gate is None else gate).float().squeeze(-1).contiguous()
         fq, fk, qr, kr, v, _ = prologue_forward(qp, kp, vp, self.phi_q.weight,
                                                 self.phi_k.weight, cos, sin, self.heads,
                                                 self.kv_heads)
@@ -514,15 +514,17 @@ class LizardAttention(nn.Module):
                 cache.k, cache.v, *sizes, cache.pos)
             cache.pos += 1
             return out
-        projections = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        projections, gate = (self.q_proj(x), self.k_proj(x), self.v_proj(x)), None
         if self._step_native(x, projections, cos, sin, cache):
-            y = _ops.load().layer_step(*projections, self.W_gamma(x), self.phi_q.weight,
-                                       self.phi_k.weight, cos, sin, self.meta_tokens,
-                                       self.alpha_blend, cache.state, cache.k, cache.v, *sizes,
-                                       cache.pos, x.dtype == torch.bfloat16)
-            cache.pos += 1
-            return self.o_proj(y.to(x.dtype))
-        z, fq, fk, qr, kr, v = self._operands(x, position_embeddings, projections)
+            gate = self.W_gamma(x)
+            if tuple(gate.shape) == (x.shape[0], 1, 1):   # not a logit per head
+                y = _ops.load().layer_step(*projections, gate, self.phi_q.weight,
+                                           self.phi_k.weight, cos, sin, self.meta_tokens,
+                                           self.alpha_blend, cache.state, cache.k, cache.v, *sizes,
+                                           cache.pos, x.dtype == torch.bfloat16)
+                cache.pos += 1
+                return self.o_proj(y.to(x.dtype))
+        z, fq, fk, qr, kr, v = self._operands(x, position_embeddings, projections, gate)
         cache.put(kr, v, cache.pos)
         y_gla = kernels.gla_decode_step(fq[:, :, 0], fk[:, :, 0], v[:, :, 0], z[:, 0].contiguous(),
                                         cache.state, gate_logit=True)

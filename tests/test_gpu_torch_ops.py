@@ -8,6 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from lizard_reproduction_amd import _ops, kernels
+from lizard_reproduction_amd import layer as hip_layer
 from lizard_reproduction_amd.layer import LizardAttention
 from tests.helpers import max_rel
 
@@ -260,3 +261,33 @@ def test_step_refuses_modules_of_other_sizes(dtype, name, inputs, outputs, error
         layer.step(x[:, 10:11], tuple(t[10:11] for t in tables), cache)
     setattr(layer, name, own)
     assert torch.equal(_decode(layer, x, tables)[0], plain)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_step_takes_a_gate_logit_per_head(monkeypatch, dtype):
+    """W_gamma with an output per head: the operators' step, each head decaying by
+    its own gate."""
+    layer, x, tables = _decode_layer()
+    layer, x, tables = layer.to(dtype), x.to(dtype), tuple(t.to(dtype) for t in tables)
+    layer.W_gamma = torch.nn.Linear(256, 4, bias=False, device="cuda", dtype=dtype)
+    calls = []
+    layer.W_gamma.register_forward_hook(lambda *a: calls.append(1))
+
+    def run():
+        cache = layer.new_cache(3)
+        return torch.cat([layer.step(x[:, t:t + 1], tuple(u[t:t + 1] for u in tables), cache)
+                          for t in range(9)], 1), cache.state
+    y, state = run()
+    assert len(calls) == 9
+    for a, b in zip((y, state), _through_python(monkeypatch, run)):
+        assert torch.equal(a, b)
+    # the normaliser state of the keys and gates that the steps saw, 9 fp32 sums
+    z = torch.zeros(3, 4, 64, device="cuda", dtype=torch.float64)
+    for t in range(9):
+        row = x[:, t:t + 1]
+        fk = hip_layer.prologue_forward(layer.q_proj(row), layer.k_proj(row), layer.v_proj(row),
+                                        layer.phi_q.weight, layer.phi_k.weight,
+                                        *(u[t:t + 1] for u in tables), 4, 2)[1]
+        gate = torch.sigmoid(layer.W_gamma(row).double())[:, 0, :, None]
+        z = gate * z + fk[:, :, 0].double().repeat_interleave(2, 1)
+    assert max_rel(kernels.split_state(state, 64, 64)[1], z) <= 1e-5

@@ -441,3 +441,17 @@ def test_native_step_itself_refuses_what_does_not_fit():
     weights[1] = linear(128, 32, torch.bfloat16).weight
     with pytest.raises(RuntimeError, match="layer's sizes"):
         ops.layer_step_rows(x, weights, *rest)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_native_step_leaves_a_gate_logit_per_head(dtype):
+    layer = decode_layer(dtype)
+    layer.W_gamma = linear(128, 4, dtype)
+    assert not layer._step_rows(torch.randn(2, 1, 128).to(dtype))
+    cache, x = layer.new_cache(2, "cpu"), torch.zeros(2, 1, 128).to(dtype)
+    table = torch.zeros(1, 32, dtype=dtype)
+    with pytest.raises(RuntimeError, match="one gate logit"):
+        _ops.load().layer_step(layer.q_proj(x), layer.k_proj(x), layer.v_proj(x), layer.W_gamma(x),
+                               layer.phi_q.weight, layer.phi_k.weight, table, table,
+                               layer.meta_tokens, layer.alpha_blend, cache.state, cache.k, cache.v,
+                               4, 2, 8, 32, 0, True)
