@@ -230,9 +230,9 @@ bool is(const Tensor& t, at::IntArrayRef sizes, const Tensor& like) {
 // out.  A step that does not fit goes operator by operator, which casts or refuses
 // what it is given.
 bool step_takes(const std::vector<Tensor>& projections, const Tensor& wq, const Tensor& wk,
-                const Tensor& cos, const Tensor& sin, const Tensor& state, const Tensor& k_cache,
-                const Tensor& v_cache, int64_t heads, int64_t kv, int64_t window, int64_t hd,
-                int64_t pos) {
+                const Tensor& cos, const Tensor& sin, const Tensor& meta, const Tensor& alpha,
+                const Tensor& state, const Tensor& k_cache, const Tensor& v_cache, int64_t heads,
+                int64_t kv, int64_t window, int64_t hd, int64_t pos) {
   if (state.dim() != 3 || wq.dim() != 2 || pos < 0) return false;
   const int64_t b = state.size(0), f = wq.size(0), nf = 2 * f;
   for (size_t i = 0; i < projections.size(); ++i)
@@ -242,7 +242,8 @@ bool step_takes(const std::vector<Tensor>& projections, const Tensor& wq, const 
                      is(cos, {b, 1, hd}, state));
   if (b <= 0 || !rope || sin.device() != state.device() || !is(wq, {f, hd}, state) ||
       !is(wk, {f, hd}, state) || !is(state, {b, heads, nf * hd + nf}, state) ||
-      state.scalar_type() != at::kFloat || !state.is_contiguous())
+      state.scalar_type() != at::kFloat || !state.is_contiguous() || meta.dim() != 1 ||
+      meta.device() != state.device() || alpha.numel() != 1 || alpha.device() != state.device())
     return false;
   for (const Tensor* t : {&k_cache, &v_cache})
     if (!is(*t, {b, kv, window, hd}, state) || t->scalar_type() != at::kBFloat16 ||
@@ -280,8 +281,8 @@ Tensor layer_step(Tensor qp, Tensor kp, Tensor vp, const Tensor& z, Tensor wq, T
                   const Tensor& state, const Tensor& k_cache, const Tensor& v_cache,
                   int64_t heads_, int64_t kv_, int64_t window_, int64_t hd_, int64_t pos,
                   bool out_bf16) {
-  TORCH_CHECK(step_takes({qp, kp, vp}, wq, wk, cos, sin, state, k_cache, v_cache, heads_, kv_,
-                         window_, hd_, pos),
+  TORCH_CHECK(step_takes({qp, kp, vp}, wq, wk, cos, sin, meta, alpha, state, k_cache, v_cache,
+                         heads_, kv_, window_, hd_, pos),
               "layer_step: tensors that do not fit the layer's sizes");
   TORCH_CHECK(is(z, {qp.size(0), 1, 1}, state), "layer_step: one gate logit per token expected");
   const int b = i32(state.size(0)), heads = i32(heads_), kv = i32(kv_), window = i32(window_),

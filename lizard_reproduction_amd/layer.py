@@ -490,7 +490,8 @@ class LizardAttention(nn.Module):
                 and tuple(cache.state.shape[:1]) == tuple(x.shape[:1])
                 and cache.state.device == x.device
                 and _ops.load().step_takes(list(projections), self.phi_q.weight, self.phi_k.weight,
-                                           cos, sin, cache.state, cache.k, cache.v, self.heads,
+                                           cos, sin, self.meta_tokens, self.alpha_blend,
+                                           cache.state, cache.k, cache.v, self.heads,
                                            self.kv_heads, self.window, self.head_dim, cache.pos))
 
     @torch.no_grad()

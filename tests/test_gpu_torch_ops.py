@@ -291,3 +291,15 @@ def test_step_takes_a_gate_logit_per_head(monkeypatch, dtype):
         gate = torch.sigmoid(layer.W_gamma(row).double())[:, 0, :, None]
         z = gate * z + fk[:, :, 0].double().repeat_interleave(2, 1)
     assert max_rel(kernels.split_state(state, 64, 64)[1], z) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name, shape, error", [
+    ("alpha_blend", (3,), RuntimeError), ("meta_tokens", (2, 2), ValueError),
+    ("meta_tokens", (), ValueError)])
+def test_step_refuses_blends_and_sinks_of_other_shapes(dtype, name, shape, error):
+    layer, x, tables = _decode_layer()
+    layer, x, tables = layer.to(dtype), x.to(dtype), tuple(t.to(dtype) for t in tables)
+    setattr(layer, name, torch.nn.Parameter(torch.ones(shape, device="cuda", dtype=dtype)))
+    with pytest.raises(error):
+        layer.step(x[:, :1], tuple(t[:1] for t in tables), layer.new_cache(3))

@@ -455,3 +455,18 @@ def test_native_step_leaves_a_gate_logit_per_head(dtype):
                                layer.phi_q.weight, layer.phi_k.weight, table, table,
                                layer.meta_tokens, layer.alpha_blend, cache.state, cache.k, cache.v,
                                4, 2, 8, 32, 0, True)
+
+
+def test_native_step_leaves_blends_and_sinks_of_other_shapes():
+    """alpha has one element, the sinks one dimension; the operators refuse others."""
+    layer = decode_layer()
+    assert step_gates(layer) == (True, True)
+    for name, value, native in (("alpha_blend", torch.ones(3), False),
+                                ("alpha_blend", torch.ones(1, 1), True),
+                                ("meta_tokens", torch.zeros(2, 2), False),
+                                ("meta_tokens", torch.zeros(()), False),
+                                ("meta_tokens", torch.zeros(0), True),
+                                ("meta_tokens", torch.zeros(9), True)):
+        layer = decode_layer()
+        setattr(layer, name, torch.nn.Parameter(value))
+        assert step_gates(layer) == (True, native)
