@@ -463,8 +463,7 @@ class LizardAttention(nn.Module):
         """Whether ``_ops.layer_step_rows`` may form the projections of x: few
         enough rows of bf16, and plain nn.Linear modules that nothing hooks into,
         patches or casts, with ordinary bf16 weights of the layer's sizes."""
-        if (x.dtype is not torch.bfloat16 or x.shape[2] != self.q_proj.in_features
-                or torch.is_autocast_enabled() or not _ops.plain()
+        if (x.dtype is not torch.bfloat16 or torch.is_autocast_enabled() or not _ops.plain()
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or nn.modules.module._has_any_global_hook()):
             return False

@@ -303,3 +303,11 @@ def test_step_refuses_blends_and_sinks_of_other_shapes(dtype, name, shape, error
     setattr(layer, name, torch.nn.Parameter(torch.ones(shape, device="cuda", dtype=dtype)))
     with pytest.raises(error):
         layer.step(x[:, :1], tuple(t[:1] for t in tables), layer.new_cache(3))
+
+
+@pytest.mark.parametrize("name", ["q_proj", "k_proj", "v_proj", "W_gamma", "o_proj"])
+def test_step_runs_replaced_modules(name):
+    layer, x, tables = _decode_layer()
+    plain, _ = _decode(layer, x, tables)
+    setattr(layer, name, torch.nn.Sequential(getattr(layer, name)))
+    assert max_rel(_decode(layer, x, tables)[0], plain) <= 2e-2   # the products rounded apart

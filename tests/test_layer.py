@@ -470,3 +470,16 @@ def test_native_step_leaves_blends_and_sinks_of_other_shapes():
         layer = decode_layer()
         setattr(layer, name, torch.nn.Parameter(value))
         assert step_gates(layer) == (True, native)
+
+
+@pytest.mark.parametrize("name", ["q_proj", "k_proj", "v_proj", "W_gamma", "o_proj"])
+def test_native_products_leave_replaced_modules(name):
+    """A module of another type (here without in_features or weight) forms its own
+    product; the step after it stays native."""
+    layer = decode_layer()
+    cache, x = layer.new_cache(2, "cpu"), torch.randn(2, 1, 128).bfloat16()
+    table = torch.randn(1, 32).bfloat16()
+    setattr(layer, name, torch.nn.Sequential(getattr(layer, name)))
+    assert not layer._step_rows(x)
+    assert layer._step_native(x, (layer.q_proj(x), layer.k_proj(x), layer.v_proj(x)), table, table,
+                              cache)
