@@ -39,6 +39,7 @@ import torch.nn.functional as F
 from . import _lib, _ops, kernels
 
 BACKENDS = ("hip",)
+LINEAR = (nn.Linear.forward, F.linear)   # what the native step's products stand in for
 MAX_HEAD_DIM = 256       # lz_swa_*: dim <= 256
 MAX_FEATURE_DIM = 2048   # lz_gla_*: F = 2 feature_dim <= LZ_GLA_MAX_DIM
 
@@ -464,6 +465,7 @@ class LizardAttention(nn.Module):
         enough rows of bf16, and plain nn.Linear modules that nothing hooks into,
         patches or casts, with ordinary bf16 weights of the layer's sizes."""
         if (x.dtype is not torch.bfloat16 or torch.is_autocast_enabled() or not _ops.plain()
+                or (nn.Linear.forward, F.linear) != LINEAR
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or nn.modules.module._has_any_global_hook()):
             return False

@@ -483,3 +483,15 @@ def test_native_products_leave_replaced_modules(name):
     assert not layer._step_rows(x)
     assert layer._step_native(x, (layer.q_proj(x), layer.k_proj(x), layer.v_proj(x)), table, table,
                               cache)
+
+
+def test_native_products_leave_a_patched_linear(monkeypatch):
+    """nn.Linear or F.linear replaced for the whole process (injected adapters,
+    counters): the modules' own calls see it."""
+    layer, x = decode_layer(), torch.randn(2, 1, 128).bfloat16()
+    for owner, name in ((torch.nn.Linear, "forward"), (torch.nn.functional, "linear")):
+        with monkeypatch.context() as m:
+            own = getattr(owner, name)
+            m.setattr(owner, name, lambda *a: own(*a))
+            assert not layer._step_rows(x)
+        assert layer._step_rows(x)
