@@ -44,6 +44,8 @@
 //     (V^T, K~^T, V) come from LDS transpose reads of the row-major tiles.
 //   * the prefetched chunk is written to LDS, the gate scan of the next chunk
 //     runs on wave 0, and z is updated.
+#include <algorithm>
+
 #include "gla_common.hpp"
 
 namespace lz {
@@ -1247,26 +1249,34 @@ bool gla_dims_supported(int F, int D) {
 }
 
 // Segments per (b, h): as many as still run in one round of workgroups, two
-// forward workgroups per CU up to F = 128, one beyond (the LDS of a 256-wide
-// chunk).  One segment more would fill the round and leave a few walks of the
-// same length to a second one (forward + backward, us, against the split
-// rounded up: B*H = 40 L = 4096 F = D = 128 275 -> 240, G 13 -> 11; B*H = 160
-// L = 2048 458 -> 363, G 4 -> 3; B*H = 297 L = 1024 F = D = 64 252 -> 232 and
-// B*H = 250 L = 2048 F = 256 D = 64 743 -> 589, one segment; none of 35 shapes
-// slower, the same split where B*H divides the round).
+// forward workgroups per CU up to F = 128.  One segment more would fill the round
+// and leave a few walks of the same length to a second one (forward + backward,
+// us, against the split rounded up: B*H = 40 L = 4096 F = D = 128 275 -> 240, G 13
+// -> 11; B*H = 160 L = 2048 458 -> 363, G 4 -> 3; B*H = 297 L = 1024 F = D = 64
+// 252 -> 232 and B*H = 250 L = 2048 F = 256 D = 64 743 -> 589, one segment).
+// Beyond F = 128 the walks run one per CU (the LDS of a 256-wide chunk), and the
+// split is doubled where B*H leaves room for two: segments half as long, which the
+// state passes, two workgroups per CU, run at once, and the walks in two rounds or
+// two in a row (gla_walk_segments, gla_bwd_walk_segments).  An odd number of
+// segments fits those two rounds where twice the rounded number leaves some of the
+// second empty; it is taken where that makes them shorter by an eleventh or more
+// (D = 64, forward and forward + backward, us: B*H = 44 L = 4096 G 10 -> 11 108 ->
+// 100 and 324 -> 309; B*H = 96 L = 4096 G 4 -> 5 215 -> 191 and 634 -> 584; B*H =
+// 72 L = 4096 G 6 -> 7 158 -> 152 and 468 -> 464; by less the backward loses:
+// B*H = 56 L = 8192, 16 -> 15 chunks, 228 -> 222 and 674 -> 695).
 void gla_segments(int BH, int L, int F, int* G, int* cps) {
   const int NT = (L + GLA_C - 1) / GLA_C;
-  const bool wide = gla_padded_dim(F) > 128;   // walks run one workgroup per CU
-  const int target = wide ? gla_target_wg() / 2 : gla_target_wg();
-  int g = target / BH;
-  g = g < 1 ? 1 : (g > NT ? NT : g);
-  // Wide walks: segments half as long as one walk, each walk taking two
-  // (gla_walk_segments).  The segment state passes, which fit two workgroups
-  // per CU, then run twice the workgroups at half the length.
-  if (wide && g > 1) g = 2 * g > NT ? NT : 2 * g;
-  const int c = (NT + g - 1) / g;
-  *cps = c;
-  *G = (NT + c - 1) / c;
+  const bool wide = gla_padded_dim(F) > 128;
+  const int round = gla_target_wg();           // two workgroups per CU
+  auto chunks = [NT](int g) { return (NT + g - 1) / g; };   // of a segment, g of them
+  int g = std::max(1, std::min(NT, wide ? round / 2 / BH : round / BH));
+  if (wide && g > 1) {
+    const int odd = std::min(NT, round / BH);
+    g = std::min(NT, 2 * g);
+    if (11 * chunks(odd) <= 10 * chunks(g)) g = odd;
+  }
+  *cps = chunks(g);
+  *G = (NT + *cps - 1) / *cps;
 }
 
 // Segments one walk workgroup takes in a row: two when each (b, h) has an

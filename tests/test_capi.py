@@ -273,6 +273,17 @@ def test_segments_stay_within_one_round(lib, b, h, length, f, split):
         4 * seg_floats(b * h, split, f, 64)
 
 
+# F > 128: two rounds of walks, an odd number of segments where it shortens them by
+# an eleventh or more (44: 7 -> 6 chunks; 72: 11 -> 10; 56: 16 -> 15 is too little)
+@pytest.mark.parametrize("b, h, length, split", [
+    (1, 44, 4096, 11), (3, 32, 4096, 5), (9, 8, 4096, 7), (7, 8, 8192, 8), (8, 16, 4096, 4),
+    (4, 32, 4096, 4), (1, 129, 4096, 1), (1, 44, 64, 1), (1, 1, 700, 11)])
+def test_wide_segments_run_in_two_rounds(lib, b, h, length, split):
+    assert split == 1 or b * h * split <= 512
+    assert lib.lz_gla_fwd_workspace_bytes(b, h, length, 256, 64, 0, 64) == \
+        4 * seg_floats(b * h, split, 256, 64)
+
+
 def test_swa_workspace_sizes(lib):
     # delta [BH, L] plus dmeta partials [BH * ceil(L/128), n_meta]
     assert lib.lz_swa_bwd_workspace_bytes(1, 32, 2048, 64, 4) == 4 * (32 * 2048 + 32 * 16 * 4)
