@@ -221,7 +221,8 @@ size_t lz_gla_bwd_workspace_bytes(int batch, int heads, int length, int nf, int 
  *                 kept it (it then holds the segment state records, scanned
  *                 into the state entering each segment or, for at most 4
  *                 segments, left for the walks to combine, and the backward
- *                 skips recomputing them); may be NULL
+ *                 skips recomputing them, unless it takes the rows whole that
+ *                 the forward split); may be NULL
  * The other arguments are those of lz_gla_fwd, with its sizes.
  */
 int lz_gla_bwd(const void* fq, const void* fk, const void* v, const float* log_gamma,

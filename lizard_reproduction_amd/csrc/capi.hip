@@ -23,6 +23,7 @@ hipError_t launch_gla_decode(const void* fq, const void* fk, const void* v, cons
                              float* state, void* y, int B, int H, int F, int D,
                              int gate_per_head, int KG, hipStream_t st);
 size_t gla_fwd_workspace(int B, int H, int L, int F, int D);
+size_t gla_kept_records(int B, int H, int L, int F, int D);
 hipError_t gla_fwd_prepare();
 bool gla_dims_supported(int F, int D);
 struct GlaTiles {
@@ -280,7 +281,7 @@ extern "C" int lz_gla_bwd(const void* fq, const void* fk, const void* v, const f
   // entering each segment; otherwise the backward recomputes it (always for
   // sizes past the walks', whose forward workspace holds tiles instead)
   const bool native = lz::gla_dims_supported(nf, nd);
-  const size_t fneed = native ? lz::gla_fwd_workspace(batch, heads, length, nf, nd) : 0;
+  const size_t fneed = native ? lz::gla_kept_records(batch, heads, length, nf, nd) : 0;
   const float* fws = nullptr;
   if (fwd_workspace && fneed) {
     if (fwd_workspace_bytes < fneed)

@@ -48,6 +48,8 @@ struct GlaPart {
 // The native walks (F, D within gla_dims_supported).  raw_den: see
 // gla_fwd_kernel's RAW; ext_den / ext_delta: see gla_bwd_dq_kernel's EXT.
 size_t gla_fwd_workspace(int B, int H, int L, int F, int D);
+// bytes of the forward's records that a backward takes (0: it splits the rows otherwise)
+size_t gla_kept_records(int B, int H, int L, int F, int D);
 size_t gla_bwd_workspace(int B, int H, int L, int F, int D, int gate);
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
                           int B, int H, int L, int F, int D, GlaRows rows, int gate, int KG,
@@ -71,7 +73,8 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
 // Sets, on the current device, the LDS limit of every kernel launch_gla_fwd
 // (without raw_den) and launch_gla_fwd_states can launch.
 hipError_t gla_fwd_prepare();
-void gla_segments(int BH, int L, int F, int* G, int* cps);
+void gla_segments(int BH, int L, int F, int D, int* G, int* cps);
+void gla_fwd_segments(int BH, int L, int F, int D, int* G, int* cps);
 int gla_walk_segments(int BH, int G, int F);
 size_t gla_segment_floats(int BH, int G, int F, int D);
 

@@ -1248,6 +1248,25 @@ bool gla_dims_supported(int F, int D) {
   return dp <= 128 && (fp <= 128 || dp <= 64);
 }
 
+// Narrow forward walks (F, D <= 64) leave room for a third workgroup on a CU:
+// whether the split above the rounded one, two or three segments, still runs in one
+// round of three.  At F = D = 64, where three slow each other more, it may
+// fill half of the third places.  For rows of at least 24 chunks (32): below, the
+// state pass takes what the shorter walks give, above they give, in us, forward
+// and forward + backward: B*H = 200 L = 4096 F = D = 32 121 -> 97 and 522 -> 498 (G
+// 2 -> 3), F = D = 64 141 -> 124 and 542 -> 534; B*H = 300 L = 2048 F = D = 32 83 ->
+// 73 and 420 -> 412 (G 1 -> 2, the forward's only), B*H = 257 F = D = 64 99 -> 88 and
+// 452 -> 443.  Least in its favour: B*H = 255 L = 1500 F = 64 D = 32 54 -> 46 and 216
+// -> 219.  Four segments for three would speed a forward up as well (B*H = 150 L =
+// 4096 F = D = 32 88 -> 74) but slow the backward down by more (370 -> 447).
+static bool rounds_up(int BH, int NT, int F, int D) {
+  const int fp = gla_padded_dim(F), dp = gla_padded_dim(D), round = gla_target_wg();
+  const int g = round / BH + 1;
+  const bool square = fp == 64 && dp == 64;
+  return round % BH && fp <= 64 && dp <= 64 && NT >= (square ? 32 : 24) && (g == 2 || g == 3) &&
+         BH * g <= (square ? 5 * round / 4 : 3 * round / 2);
+}
+
 // Segments per (b, h): as many as still run in one round of workgroups, two
 // forward workgroups per CU up to F = 128.  One segment more would fill the round
 // and leave a few walks of the same length to a second one (forward + backward,
@@ -1264,7 +1283,7 @@ bool gla_dims_supported(int F, int D) {
 // 100 and 324 -> 309; B*H = 96 L = 4096 G 4 -> 5 215 -> 191 and 634 -> 584; B*H =
 // 72 L = 4096 G 6 -> 7 158 -> 152 and 468 -> 464; by less the backward loses:
 // B*H = 56 L = 8192, 16 -> 15 chunks, 228 -> 222 and 674 -> 695).
-void gla_segments(int BH, int L, int F, int* G, int* cps) {
+void gla_segments(int BH, int L, int F, int D, int* G, int* cps) {
   const int NT = (L + GLA_C - 1) / GLA_C;
   const bool wide = gla_padded_dim(F) > 128;
   const int round = gla_target_wg();           // two workgroups per CU
@@ -1275,8 +1294,21 @@ void gla_segments(int BH, int L, int F, int* G, int* cps) {
     g = std::min(NT, 2 * g);
     if (11 * chunks(odd) <= 10 * chunks(g)) g = odd;
   }
+  if (g == 2 && rounds_up(BH, NT, F, D)) g = 3;
   *cps = chunks(g);
   *G = (NT + *cps - 1) / *cps;
+}
+
+// The forward's split: two segments in some rows that the backward, whose walks
+// run one per CU, takes whole and so without the forward's records (a backward of
+// another number of segments would have to form its own: 4 % of the pair).
+void gla_fwd_segments(int BH, int L, int F, int D, int* G, int* cps) {
+  gla_segments(BH, L, F, D, G, cps);
+  const int NT = (L + GLA_C - 1) / GLA_C;
+  if (*G == 1 && rounds_up(BH, NT, F, D)) {
+    *cps = (NT + 1) / 2;
+    *G = 2;
+  }
 }
 
 // Segments one walk workgroup takes in a row: two when each (b, h) has an
@@ -1295,8 +1327,15 @@ size_t gla_segment_floats(int BH, int G, int F, int D) {
 
 size_t gla_fwd_workspace(int B, int H, int L, int F, int D) {
   int G, cps;
-  gla_segments(B * H, L, F, &G, &cps);
+  gla_fwd_segments(B * H, L, F, D, &G, &cps);
   return gla_segment_floats(B * H, G, F, D) * sizeof(float);
+}
+
+size_t gla_kept_records(int B, int H, int L, int F, int D) {
+  int G, cps, Gf, cf;
+  gla_segments(B * H, L, F, D, &G, &cps);
+  gla_fwd_segments(B * H, L, F, D, &Gf, &cf);
+  return G == Gf && cps == cf ? gla_fwd_workspace(B, H, L, F, D) : 0;
 }
 
 hipError_t launch_gla_segment_scan(float* seg_state, const float* seg_logdecay, int BH, int G,
@@ -1413,7 +1452,7 @@ static hipError_t launch_gla_fwd_t(const void* fq, const void* fk, const void* v
   using Cfg = GlaFwd<FP, DP>;
   const int BH = B * H;
   int G, cps;
-  gla_segments(BH, L, F, &G, &cps);
+  gla_fwd_segments(BH, L, F, D, &G, &cps);
   constexpr bool CAN_FOLD = gla_can_fold<FP, DP, VEC>() && !RAW;
   const bool fold = CAN_FOLD && gla_fold_segments(G);
   float* seg_state = ws;
@@ -1558,7 +1597,7 @@ hipError_t launch_gla_fwd_phi(const void* q, const void* wq, const void* fk, con
   constexpr int FP = 256, DP = 64;
   const int F = FP, D = DP, BH = B * H;
   int G, cps;
-  gla_segments(BH, L, F, &G, &cps);
+  gla_fwd_segments(BH, L, F, D, &G, &cps);
   float* seg_lam = ws + (size_t)BH * G * GlaFwd<FP, DP>::SEG;
   const bool fold = gla_fold_segments(G);   // the walk with phi has a folding variant
   static_assert(gla_can_fold<FP, DP, true>(), "folding variant of the phi walk");

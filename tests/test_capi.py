@@ -284,6 +284,24 @@ def test_wide_segments_run_in_two_rounds(lib, b, h, length, split):
         4 * seg_floats(b * h, split, 256, 64)
 
 
+# F, D <= 64: three segments for two (both directions), two for one (the forward's
+# only), in rows of at least 24 chunks (32 at F = D = 64) and up to three workgroups a
+# CU (half as many third ones at F = D = 64)
+@pytest.mark.parametrize("bh, length, f, d, forward, backward", [
+    (257, 1472, 32, 32, 1, 1), (257, 1473, 32, 32, 2, 1), (384, 4096, 32, 64, 2, 1),
+    (385, 4096, 32, 64, 1, 1), (257, 1984, 64, 64, 1, 1), (320, 1985, 64, 64, 2, 1),
+    (321, 4096, 64, 64, 1, 1), (300, 4096, 64, 65, 1, 1), (300, 4096, 65, 64, 1, 1),
+    (256, 4096, 32, 32, 2, 2), (255, 1473, 64, 32, 3, 3), (255, 1472, 64, 32, 2, 2),
+    (171, 1473, 24, 20, 3, 3), (170, 4096, 32, 32, 3, 3), (213, 1985, 64, 64, 3, 3),
+    (214, 4096, 64, 64, 2, 2), (512, 4096, 32, 32, 1, 1), (1, 4096, 32, 32, 64, 64)])
+def test_narrow_segments_take_a_third_place(lib, bh, length, f, d, forward, backward):
+    for b, h in ((1, bh), (bh, 1)):
+        assert lib.lz_gla_fwd_workspace_bytes(b, h, length, f, d, 0, 64) == \
+            4 * seg_floats(bh, forward, f, d)
+        assert lib.lz_gla_bwd_workspace_bytes(b, h, length, f, d, 0, 64) == \
+            4 * (4 * bh * length + 2 * seg_floats(bh, backward, f, d) + bh * -(-length // 64))
+
+
 def test_swa_workspace_sizes(lib):
     # delta [BH, L] plus dmeta partials [BH * ceil(L/128), n_meta]
     assert lib.lz_swa_bwd_workspace_bytes(1, 32, 2048, 64, 4) == 4 * (32 * 2048 + 32 * 16 * 4)

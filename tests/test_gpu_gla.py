@@ -368,3 +368,31 @@ def test_gla_backward_walks_of_odd_segments(batch, heads, length, features, dim,
     compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
                                                       dtype=torch.float32),
             inputs, grad, label=f"odd segments F={features} D={dim} B*H={batch * heads} L={length}")
+
+
+# narrow walks, three to a CU: three segments in both directions, and two of the
+# forward's only, the backward's rows whole; a shorter last segment in each
+@pytest.mark.parametrize("batch, heads, length, features, dim, per_head", [
+    (1, 171, 1473, 32, 32, True), (3, 67, 1985, 64, 64, False), (1, 257, 1473, 32, 64, False),
+    (2, 160, 2049, 64, 64, True), (17, 16, 1500, 24, 20, False)])
+def test_gla_narrow_rows_of_two_and_three_segments(batch, heads, length, features, dim, per_head):
+    inputs = gla_inputs(length, gates=(heads,) if per_head else (), batch=batch, heads=heads,
+                        features=features, dim=dim, seed=43)
+    grad = torch.randn(inputs[2].shape, generator=torch.Generator().manual_seed(6))
+    compare(gla_kernel(64), lambda *a: lo.gla_chunked(*a[:3], F.logsigmoid(a[3]), chunk=64,
+                                                      dtype=torch.float32),
+            inputs, grad, label=f"narrow F={features} D={dim} B*H={batch * heads} L={length}")
+
+
+def test_gla_backward_of_whole_rows_leaves_the_forwards_records():
+    """B*H = 300: two segments forward, whose records the backward has no use for,
+    and the forward without a graph gives the same bits."""
+    fq, fk, v, z = gla_inputs(1600, gates=(300,), batch=1, heads=300, features=32, dim=32, seed=47)
+    fq, fk, v, lg = fq.cuda(), fk.cuda(), v.cuda(), F.logsigmoid(z.cuda())
+    dy = torch.randn(v.shape, device="cuda").bfloat16()
+    y, state = kernels.gla_forward(fq, fk, v, lg, keep_state=True)
+    assert state is not None
+    assert torch.equal(y, kernels.gla_forward(fq, fk, v, lg, keep_state=False)[0])
+    kept = kernels.gla_backward(fq, fk, v, lg, dy, state, torch.bfloat16)
+    for a, b in zip(kept, kernels.gla_backward(fq, fk, v, lg, dy, None, torch.bfloat16)):
+        assert torch.equal(a, b)
