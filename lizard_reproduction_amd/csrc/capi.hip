@@ -10,11 +10,8 @@
 #include "common.hpp"
 
 namespace lz {
-struct GlaRows {
-  int ld, ldy, hsy;
-};
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
-                          int B, int H, int L, int F, int D, GlaRows rows, int gate_per_head, int KG,
+                          int B, int H, int L, int F, int D, int ld, int gate_per_head, int KG,
                           float* ws, float* final_state, float* raw_den, hipStream_t st);
 hipError_t launch_gla_fwd_phi(const void* q, const void* wq, const void* fk, const void* v,
                               const float* lg, void* y, int B, int H, int L, int gate, int KG,
@@ -206,7 +203,7 @@ extern "C" int lz_gla_prefill(const void* fq, const void* fk, const void* v,
     return fail(1, "gla_prefill: workspace of %zu bytes given, %zu needed", workspace_bytes,
                 need);
   return hip_status(lz::launch_gla_fwd(fq, fk, v, log_gamma, y, batch, heads, length, nf, nd,
-                                       lz::GlaRows{nd, nd, length * nd}, gate_mode,
+                                       nd, gate_mode,
                                        heads / kv_heads, (float*)workspace,
                                        state, nullptr, (hipStream_t)stream),
                     "gla_prefill");
@@ -374,7 +371,7 @@ extern "C" int lz_gla_fwd_noalloc(const void* fq, const void* fk, const void* v,
   if (int rc = noalloc_setup(&ws)) return rc;
   if (!need) ws = nullptr;
   return hip_status(lz::launch_gla_fwd(fq, fk, v, log_gamma, y, batch, heads, length, nf, nd,
-                                       lz::GlaRows{nd, nd, length * nd}, gate_mode,
+                                       nd, gate_mode,
                                        heads / kv_heads, ws, nullptr,
                                        nullptr, (hipStream_t)stream),
                     "gla_fwd_noalloc");

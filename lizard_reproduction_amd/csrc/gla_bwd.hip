@@ -135,22 +135,13 @@ struct BwdA : BwdCommon<FP, DP> {
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
 
-// dy of (b, h)
-__device__ __forceinline__ size_t dy_offset(const GlaRows& rows, int bh, int H, int L) {
-  if (rows.ldy == rows.ld && rows.hsy == L * rows.ld) return (size_t)bh * L * rows.ld;
-  return (size_t)(bh / H) * H * L * rows.ld + (size_t)(bh % H) * rows.hsy;
-}
-
-// The rows as the walk of FP features takes them: only the widest is launched on
-// columns of wider rows (GlaPart); for the others they follow each other, known
-// when compiled (as arguments, the pitches spilled 15 more scalar registers of
-// the F = D = 128 backward: 871 -> 874 us for the headline's fwd+bwd).
+// The pitch of v, dy and dv rows as the walk of FP features takes it: only the
+// widest is launched on columns of wider rows (GlaPart); for the others they follow
+// each other, known when compiled (as an argument, the pitch spilled 15 more scalar
+// registers of the F = D = 128 backward: 871 -> 874 us for the headline's fwd+bwd).
 template <int FP>
-__device__ __forceinline__ GlaRows walk_rows(const GlaRows& given, int L, int D) {
-  if constexpr (FP == 256)
-    return given;
-  else
-    return GlaRows{D, D, L * D};
+__device__ __forceinline__ int walk_pitch(int given, int D) {
+  return FP == 256 ? given : D;
 }
 
 // Columns [f, f + 4) of row `tok` of the fp32 [L, F] sums of (b, h) (at `off`)
@@ -203,10 +194,10 @@ __device__ __forceinline__ void gla_bwd_dq_body(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy, OutT* __restrict__ dfq,
     float* __restrict__ den_out, float* __restrict__ delta_out, float* __restrict__ p_out,
-    const float* __restrict__ seg_state, int H, int L, int F, int D, GlaRows given, int gate, int G,
+    const float* __restrict__ seg_state, int H, int L, int F, int D, int given, int gate, int G,
     int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam,
     GlaPart part) {
-  const GlaRows rows = walk_rows<FP>(given, L, D);
+  const int ld = walk_pitch<FP>(given, D);
   using Cfg = BwdA<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT;
@@ -249,9 +240,9 @@ __device__ __forceinline__ void gla_bwd_dq_body(
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
   const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
-  const size_t offDy = dy_offset(rows, bh, H, L);
+  const size_t offDy = (size_t)bh * L * ld;
   // fk and v of the kv head of this query head (KG query heads share one)
-  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * rows.ld;
+  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the forward state entering segment seg: its scanned record, or (FOLD) the
   // local records of segments 0 .. seg - 1 folded here (their total log
@@ -355,8 +346,8 @@ __device__ __forceinline__ void gla_bwd_dq_body(
     if (n < n1) {
       load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF, F);
       load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF, F);
-      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, rows.ld);
-      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, rows.ldy);
+      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, ld);
+      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, ld);
       if (wave == GW) {
         rg[S] = gate_at(lgb, n * C + lane, L);
         rgok[S] = n * C + lane < L;
@@ -614,11 +605,11 @@ __global__ __launch_bounds__(B_THREADS, 1) void gla_bwd_dq_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ fk, const bf16* __restrict__ v,
     const float* __restrict__ log_gamma, const bf16* __restrict__ dy, OutT* __restrict__ dfq,
     float* __restrict__ den_out, float* __restrict__ delta_out, float* __restrict__ p_out,
-    const float* __restrict__ seg_state, int H, int L, int F, int D, GlaRows rows, int gate, int G,
+    const float* __restrict__ seg_state, int H, int L, int F, int D, int ld, int gate, int G,
     int cps, int M, int KG, int xper, int nxcd, int nblk, const float* __restrict__ seg_lam,
     GlaPart part) {
   gla_bwd_dq_body<FP, DP, OutT, VEC, EXT, FOLD, PART>(
-      fq, fk, v, log_gamma, dy, dfq, den_out, delta_out, p_out, seg_state, H, L, F, D, rows, gate, G,
+      fq, fk, v, log_gamma, dy, dfq, den_out, delta_out, p_out, seg_state, H, L, F, D, ld, gate, G,
       cps, M, KG, xper, nxcd, nblk, seg_lam, part);
 }
 
@@ -709,8 +700,8 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
     const bf16* __restrict__ fq, const bf16* __restrict__ dy, const float* __restrict__ log_gamma,
     const float* __restrict__ den_in, const float* __restrict__ delta_in,
     float* __restrict__ seg_state, float* __restrict__ seg_logdecay, int H, int L, int F, int D,
-    GlaRows given, int gate, int G, int cps) {
-  const GlaRows rows = walk_rows<FP>(given, L, D);
+    int given, int gate, int G, int cps) {
+  const int ld = walk_pitch<FP>(given, D);
   using Cfg = BwdS<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT, NTILE = NFT * NDT, TPW = (NTILE + 3) / 4;
@@ -735,7 +726,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
   const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
-  const size_t offDy = dy_offset(rows, bh, H, L);
+  const size_t offDy = (size_t)bh * L * ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
 
   f32x16 dS[TPW];
@@ -747,7 +738,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
   uint4 rq[Cfg::NLF], rd[Cfg::NLD];
   TokScalars sc;
   load_chunk<FP>(rq, fq + offF, (n1 - 1) * C, L, F, vecF, F);
-  load_chunk<DP>(rd, dy + offDy, (n1 - 1) * C, L, D, vecD, rows.ldy);
+  load_chunk<DP>(rd, dy + offDy, (n1 - 1) * C, L, D, vecD, ld);
   sc = load_scalars(lgb, den_in, delta_in, nullptr, offL, (n1 - 1) * C + lane, L);
   store_chunk<FP>(rq, fq_l, PF);
   store_chunk<DP>(rd, dy_l, PD);
@@ -759,7 +750,7 @@ __global__ __launch_bounds__(256, 2) void gla_bwd_state_kernel(
     const bool more = n - 1 >= n0;
     if (more) {
       load_chunk<FP>(rq, fq + offF, (n - 1) * C, L, F, vecF, F);
-      load_chunk<DP>(rd, dy + offDy, (n - 1) * C, L, D, vecD, rows.ldy);
+      load_chunk<DP>(rd, dy + offDy, (n - 1) * C, L, D, vecD, ld);
       sc = load_scalars(lgb, den_in, delta_in, nullptr, offL, (n - 1) * C + lane, L);
     }
     // dz partials sum_i fq_i (qh_i delta_i)
@@ -882,9 +873,9 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
     const float* __restrict__ p_in, OutT* __restrict__ dfk, OutT* __restrict__ dv,
     float* __restrict__ dG, float* __restrict__ csum, float* __restrict__ dlg_direct,
     const float* __restrict__ seg_state, int H,
-    int L, int F, int D, GlaRows given, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
+    int L, int F, int D, int given, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
     int nblk, const float* __restrict__ seg_lam, int rev, GlaPart part) {
-  const GlaRows rows = walk_rows<FP>(given, L, D);
+  const int ld = walk_pitch<FP>(given, D);
   using Cfg = BwdB<FP, DP>;
   constexpr int C = Cfg::C, PF = Cfg::PF, PD = Cfg::PD;
   constexpr int NFT = Cfg::NFT, NDT = Cfg::NDT, ZP = Cfg::ZP;
@@ -923,9 +914,9 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
   const int col = lane & 31, h = lane >> 5;
   const bool vecF = VEC || (F & 7) == 0, vecD = VEC || (D & 7) == 0;
   const size_t offF = (size_t)bh * L * F, offL = (size_t)bh * L;
-  const size_t offDy = dy_offset(rows, bh, H, L);
+  const size_t offDy = (size_t)bh * L * ld;
   // fk and v of the kv head of this query head (KG query heads share one)
-  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * rows.ld;
+  const size_t offFk = (size_t)(bh / KG) * L * F, offDv = (size_t)(bh / KG) * L * ld;
   const float* lgb = log_gamma + (size_t)((gate & GATE_PER_HEAD) ? bh : bh / H) * L;
   // the gradient state entering segment seg from the right: its scanned
   // record, or (FOLD) the local records of segments G - 1 .. seg + 1 folded
@@ -1004,8 +995,8 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
     if (n >= n0) {
       load_tile8<FP>(rq[S], fq + offF, n * C, L, F, vecF, F);
       load_tile8<FP>(rk[S], fk + offFk, n * C, L, F, vecF, F);
-      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, rows.ld);
-      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, rows.ldy);
+      load_tile8<DP>(rv[S], v + offDv, n * C, L, D, vecD, ld);
+      load_tile8<DP>(rd[S], dy + offDy, n * C, L, D, vecD, ld);
       if (wave == SCW) sc[S] = load_scalars(lgb, den_in, delta_in, p_in, offL, n * C + lane, L);
     }
   };
@@ -1141,7 +1132,7 @@ __device__ __forceinline__ void gla_bwd_dkv_body(
         for (int qb = 0; qb < 4; ++qb)   // keys 32-63 have no queries in blocks 0, 1
           if (hk == 0 || qb >= 2)
             g = mfma(tr_operand(dy_l, PD, 16 * qb, dt * 32, lane), fa[(hk * 4 + qb) * 64 + lane], g);
-        store_acc_row_pitched<OutT>(dv + (size_t)bh * L * rows.ld, t0 + key, dt * 32, L, D, rows.ld,
+        store_acc_row_pitched<OutT>(dv + (size_t)bh * L * ld, t0 + key, dt * 32, L, D, ld,
                                     vecD, g, 1.f, h);
       }
     }
@@ -1258,11 +1249,11 @@ __global__ __launch_bounds__(B_THREADS, (BwdB<FP, DP>::LB)) void gla_bwd_dkv_ker
     const float* __restrict__ p_in, OutT* __restrict__ dfk, OutT* __restrict__ dv,
     float* __restrict__ dG, float* __restrict__ csum, float* __restrict__ dlg_direct,
     const float* __restrict__ seg_state, int H,
-    int L, int F, int D, GlaRows rows, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
+    int L, int F, int D, int ld, int gate, int G, int cps, int M, int KG, int xper, int nxcd,
     int nblk, const float* __restrict__ seg_lam, int rev, GlaPart part) {
   gla_bwd_dkv_body<FP, DP, OutT, VEC, FOLD, PART>(
       fq, fk, v, log_gamma, dy, den_in, delta_in, p_in, dfk, dv, dG, csum, dlg_direct, seg_state, H,
-      L, F, D, rows, gate, G, cps, M, KG, xper, nxcd, nblk, seg_lam, rev, part);
+      L, F, D, ld, gate, G, cps, M, KG, xper, nxcd, nblk, seg_lam, rev, part);
 }
 
 // One segment per (b, h): the dq walk and then the dkv walk of the same
@@ -1276,15 +1267,15 @@ __global__ __launch_bounds__(B_THREADS, 1) void gla_bwd_fused_kernel(
     OutT* __restrict__ dfk, OutT* __restrict__ dv, float* __restrict__ den,
     float* __restrict__ delta, float* __restrict__ p, float* __restrict__ dG,
     float* __restrict__ csum, float* __restrict__ dlg_direct, int H, int L, int F, int D,
-    GlaRows rows, int gate, int cps, int KG, int xper, int nxcd, int nblk, GlaPart part) {
+    int ld, int gate, int cps, int KG, int xper, int nxcd, int nblk, GlaPart part) {
   gla_bwd_dq_body<FP, DP, OutT, VEC, false, false, PART>(
-      fq, fk, v, log_gamma, dy, dfq, den, delta, p, nullptr, H, L, F, D, rows, gate, 1, cps, 1, KG,
+      fq, fk, v, log_gamma, dy, dfq, den, delta, p, nullptr, H, L, F, D, ld, gate, 1, cps, 1, KG,
       xper, nxcd, nblk, nullptr, part);
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   __syncthreads();
   gla_bwd_dkv_body<FP, DP, OutT, VEC, false, PART>(
       fq, fk, v, log_gamma, dy, den, delta, p, dfk, dv, dG, csum, dlg_direct, nullptr, H, L, F, D,
-      rows, gate, 1, cps, 1, KG, xper, nxcd, nblk, nullptr, 0, part);
+      ld, gate, 1, cps, 1, KG, xper, nxcd, nblk, nullptr, 0, part);
 }
 
 // ============================================================================
@@ -1399,7 +1390,7 @@ static int gla_bwd_walk_segments(int BH, int G) {
 template <int FP, int DP, typename OutT, bool VEC>
 static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v, const float* lg,
                                    const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                                   int B, int H, int L, int F, int D, GlaRows rows, int gate,
+                                   int B, int H, int L, int F, int D, int ld, int gate,
                                    int KG, const float* fwd_ws, float* ws, const float* ext_den,
                                    const float* ext_delta, const GlaPart* part, hipStream_t st) {
   const int BH = B * H;
@@ -1429,7 +1420,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
   hipError_t e;
   if (G > 1 && !fwd_ws) {
     e = launch_gla_fwd_states(fk, v, lg, own_fseg, own_fseg + (size_t)BH * G * SEG, BH, H, L, F,
-                              D, rows.ld, gate, G, cps, KG, fold, st);
+                              D, ld, gate, G, cps, KG, fold, st);
     if (e != hipSuccess) return e;
   }
   const int M = gla_bwd_walk_segments(BH, G);
@@ -1458,7 +1449,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
       hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_F, st, (const bf16*)fq,
                          (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (OutT*)dfq,
                          (OutT*)dfk, (OutT*)dv, den, delta, p, dG, csum,
-                         direct_dlg ? dlg : nullptr, H, L, F, D, rows, gate, cps, KG, wg.per, wg.nx,
+                         direct_dlg ? dlg : nullptr, H, L, F, D, ld, gate, cps, KG, wg.per, wg.nx,
                          wg.nblk, pt);
       return hipGetLastError();
     };
@@ -1473,7 +1464,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     if (hipError_t e2 = ensure_lds<kern>(LDS_A); e2 != hipSuccess) return e2;
     hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_A, st, (const bf16*)fq,
                        (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (OutT*)dfq, den,
-                       delta, p, fseg, H, L, F, D, rows, gate, G, cps, M, KG, wg.per, wg.nx,
+                       delta, p, fseg, H, L, F, D, ld, gate, G, cps, M, KG, wg.per, wg.nx,
                        wg.nblk, flam, pt);
     return hipGetLastError();
   };
@@ -1494,7 +1485,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     if ((e = ensure_lds<gla_bwd_state_kernel<FP, DP, VEC>>(LDS_S)) != hipSuccess) return e;
     hipLaunchKernelGGL(ks, dim3(BH * (G - 1)), dim3(256), LDS_S, st,
                        (const bf16*)fq, (const bf16*)dy, lg, (const float*)den,
-                       (const float*)delta, rseg, rlam, H, L, F, D, rows, gate, G, cps);
+                       (const float*)delta, rseg, rlam, H, L, F, D, ld, gate, G, cps);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!fold && (e = launch_gla_segment_scan(rseg, rlam, BH, G, SEG, true, st)) != hipSuccess)
       return e;
@@ -1511,7 +1502,7 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
     hipLaunchKernelGGL(kern, dim3(wg.grid), dim3(B_THREADS), LDS_B, st, (const bf16*)fq,
                        (const bf16*)fk, (const bf16*)v, lg, (const bf16*)dy, (const float*)den,
                        (const float*)delta, (const float*)p, (OutT*)dfk, (OutT*)dv, dG, csum,
-                       direct_dlg ? dlg : nullptr, (const float*)rseg, H, L, F, D, rows, gate, G,
+                       direct_dlg ? dlg : nullptr, (const float*)rseg, H, L, F, D, ld, gate, G,
                        cps, M, KG, wg.per, wg.nx, wg.nblk, (const float*)rlam, rev, pt);
     return hipGetLastError();
   };
@@ -1530,16 +1521,15 @@ static hipError_t launch_gla_bwd_t(const void* fq, const void* fk, const void* v
 // dimension) den and delta [BH, L] of the whole feature dimension
 hipError_t launch_gla_bwd(const void* fq, const void* fk, const void* v, const float* lg,
                           const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                          bool grad_bf16, int B, int H, int L, int F, int D, GlaRows rows,
+                          bool grad_bf16, int B, int H, int L, int F, int D, int ld,
                           int gate, int KG, const float* fwd_ws, float* ws, const float* ext_den,
                           const float* ext_delta, const GlaPart* part, hipStream_t st) {
   const int fp = gla_padded_dim(F), dp = gla_padded_dim(D);
-  if (fp < 256 && (rows.ld != D || rows.ldy != D || rows.hsy != L * D)) return hipErrorInvalidValue;
-  const bool vec = F % 8 == 0 && D % 8 == 0 && rows.ld % 8 == 0 && rows.ldy % 8 == 0 &&
-                   rows.hsy % 8 == 0;
+  if (fp < 256 && ld != D) return hipErrorInvalidValue;
+  const bool vec = F % 8 == 0 && D % 8 == 0 && ld % 8 == 0;
 #define LZ_GLA_BWD_V(FPV, DPV, OUT, V)                                                          \
   launch_gla_bwd_t<FPV, DPV, OUT, V>(fq, fk, v, lg, dy, dfq, dfk, dv, dlg, B, H, L, F, D,      \
-                                     rows, gate, KG, fwd_ws, ws, ext_den, ext_delta, part, st)
+                                     ld, gate, KG, fwd_ws, ws, ext_den, ext_delta, part, st)
 #define LZ_GLA_BWD(FPV, DPV)                                                                    \
   if (fp == FPV && dp == DPV)                                                                   \
     return grad_bf16 ? (vec ? LZ_GLA_BWD_V(FPV, DPV, bf16, true)                                \

@@ -27,15 +27,6 @@ struct GlaTiles {
 };
 GlaTiles gla_tiles(int F, int D);
 
-// Where the D-side rows of a walk lie, in elements: v, y and dv rows are `ld`
-// apart ([.., L, ld] slabs per head, the walk on D <= ld columns of them from
-// the pointers it is given: one D tile), dy rows `ldy` apart with heads `hsy`
-// apart.  Every batch entry spans H * L * ld elements.
-struct GlaRows {
-  int ld, ldy, hsy;
-};
-inline GlaRows gla_rows(int L, int ld) { return GlaRows{ld, ld, L * ld}; }
-
 // One of several D tiles' backward: dfq and dfk are sums over the tiles, kept
 // in fp32 [BH, L, F].  `in`: the sums so far to add (nullptr: the first tile);
 // `out`: where to leave them (nullptr: the last tile writes dfq, dfk and the
@@ -47,16 +38,19 @@ struct GlaPart {
 
 // The native walks (F, D within gla_dims_supported).  raw_den: see
 // gla_fwd_kernel's RAW; ext_den / ext_delta: see gla_bwd_dq_kernel's EXT.
+// ld: elements from one row of v, y, dy and dv to the next ([.., L, ld] slabs per
+// head); the walk is on D <= ld columns of them from the pointers it is given (one
+// D tile).
 size_t gla_fwd_workspace(int B, int H, int L, int F, int D);
 // bytes of the forward's records that a backward takes (0: it splits the rows otherwise)
 size_t gla_kept_records(int B, int H, int L, int F, int D);
 size_t gla_bwd_workspace(int B, int H, int L, int F, int D, int gate);
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
-                          int B, int H, int L, int F, int D, GlaRows rows, int gate, int KG,
+                          int B, int H, int L, int F, int D, int ld, int gate, int KG,
                           float* ws, float* final_state, float* raw_den, hipStream_t st);
 hipError_t launch_gla_bwd(const void* fq, const void* fk, const void* v, const float* lg,
                           const void* dy, void* dfq, void* dfk, void* dv, float* dlg,
-                          bool grad_bf16, int B, int H, int L, int F, int D, GlaRows rows,
+                          bool grad_bf16, int B, int H, int L, int F, int D, int ld,
                           int gate, int KG, const float* fwd_ws, float* ws, const float* ext_den,
                           const float* ext_delta, const GlaPart* part, hipStream_t st);
 // Any F and D: the native walks, or tiles of them (gla_tiled.hip).

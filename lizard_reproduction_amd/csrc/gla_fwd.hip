@@ -1564,9 +1564,9 @@ hipError_t gla_fwd_prepare() {
 // feature dimension) y is the fp32 numerator [BH, L, D] and raw_den the fp32
 // denominator [BH, L] of this tile (see gla_fwd_kernel's RAW).
 hipError_t launch_gla_fwd(const void* fq, const void* fk, const void* v, const float* lg, void* y,
-                          int B, int H, int L, int F, int D, GlaRows rows, int gate, int KG,
+                          int B, int H, int L, int F, int D, int ld, int gate, int KG,
                           float* ws, float* final_state, float* raw_den, hipStream_t st) {
-  const int fp = gla_padded_dim(F), dp = gla_padded_dim(D), ld = rows.ld;
+  const int fp = gla_padded_dim(F), dp = gla_padded_dim(D);
   const bool vec = F % 8 == 0 && D % 8 == 0 && ld % 8 == 0;
 #define LZ_GLA_FWD_R(FPV, DPV, V)                                                               \
   (raw_den ? launch_gla_fwd_t<FPV, DPV, V, true>(fq, fk, v, lg, y, B, H, L, F, D, ld,           \

@@ -23,7 +23,7 @@
 //   tile f are its columns, dv and d log_gamma sums over the tiles.
 //
 // D tiles alone (F <= 256) need no copies: the walks read and write their
-// columns of v, y, dy and dv where they lie (GlaRows), and at F > 128 the
+// columns of v, y, dy and dv where they lie (at the pitch of the whole rows), and at F > 128 the
 // backward's walks add dfq and dfk over the tiles themselves (GlaPart: fp32
 // sums left by one tile's walk, added by the next, written by the last).  That
 // needs rows of whole 16-byte pieces (D % 8 == 0).  At F = 256 D = 128 (B=1 H=32
@@ -224,7 +224,7 @@ hipError_t raw_forward(const GlaTiles& t, const FwdBufs& b, const void* fq, cons
         if ((e = copy_bf16(b.vt, dw, 0, (const bf16*)v, D, d * t.Dt, dw, BHLk, st))) return e;
         vt = b.vt;
       }
-      if ((e = launch_gla_fwd(b.fqt, b.fkt, vt, lg, b.numt, B, H, L, fw, dw, gla_rows(L, dw), gph,
+      if ((e = launch_gla_fwd(b.fqt, b.fkt, vt, lg, b.numt, B, H, L, fw, dw, dw, gph,
                               KG, b.inner,
                               nullptr, b.dent, st)))
         return e;
@@ -250,7 +250,7 @@ hipError_t launch_gla_fwd_any(const void* fq, const void* fk, const void* v, con
                               void* ws, hipStream_t st) {
   const GlaTiles t = gla_tiles(F, D);
   if (t.native())
-    return launch_gla_fwd(fq, fk, v, lg, y, B, H, L, F, D, gla_rows(L, D), gph, KG, (float*)ws,
+    return launch_gla_fwd(fq, fk, v, lg, y, B, H, L, F, D, D, gph, KG, (float*)ws,
                           nullptr, nullptr, st);
   Carve c{(char*)ws};
   const FwdBufs b = carve_fwd(c, t, B, H, L, F, D);
@@ -264,12 +264,12 @@ hipError_t launch_gla_fwd_any(const void* fq, const void* fk, const void* v, con
       const int gd = d + 1 < t.nD ? gph & ~GATE_NO_REUSE : gph;
       if (tiles_in_place(t, D)) {
         if ((e = launch_gla_fwd(fq, fk, (const bf16*)v + d * t.Dt, lg, (bf16*)y + d * t.Dt, B, H, L,
-                                F, dw, gla_rows(L, D), gd, KG, b.inner, nullptr, nullptr, st)))
+                                F, dw, D, gd, KG, b.inner, nullptr, nullptr, st)))
           return e;
         continue;
       }
       if ((e = copy_bf16(b.vt, dw, 0, (const bf16*)v, D, d * t.Dt, dw, BHLk, st))) return e;
-      if ((e = launch_gla_fwd(fq, fk, b.vt, lg, b.yt, B, H, L, F, dw, gla_rows(L, dw), gd, KG,
+      if ((e = launch_gla_fwd(fq, fk, b.vt, lg, b.yt, B, H, L, F, dw, dw, gd, KG,
                               b.inner, nullptr, nullptr, st)))
         return e;
       if ((e = copy_bf16((bf16*)y, D, d * t.Dt, b.yt, dw, 0, dw, BHL, st))) return e;
@@ -342,7 +342,7 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
   const GlaTiles t = gla_tiles(F, D);
   if (t.native())
     return launch_gla_bwd(fq, fk, v, lg, dy, dfq, dfk, dv, dlg, grad_bf16, B, H, L, F, D,
-                          gla_rows(L, D), gph, KG, fwd_ws, (float*)ws, nullptr, nullptr, nullptr,
+                          D, gph, KG, fwd_ws, (float*)ws, nullptr, nullptr, nullptr,
                           st);
   Carve c{(char*)ws};
   const BwdBufs b = carve_bwd(c, t, B, H, L, F, D, gph);
@@ -357,7 +357,7 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
                             last ? nullptr : b.dfq_a, last ? nullptr : b.dfk_a};
       if ((e = launch_gla_bwd(fq, fk, (const bf16*)v + c0, lg, (const bf16*)dy + c0, dfq, dfk,
                               (char*)dv + c0 * es, last ? dlg : nullptr, grad_bf16, B, H, L, F,
-                              width_of(d, t.nD, t.Dt, D), gla_rows(L, D), gph, KG, nullptr, b.inner,
+                              width_of(d, t.nD, t.Dt, D), D, gph, KG, nullptr, b.inner,
                               nullptr, nullptr, &part, st)))
         return e;
     }
@@ -395,7 +395,7 @@ hipError_t launch_gla_bwd_any(const void* fq, const void* fk, const void* v, con
       const float* eden = t.nF > 1 ? b.fwd.den : nullptr;
       const float* edel = t.nF > 1 ? b.delta + (size_t)d * BHL : nullptr;
       if ((e = launch_gla_bwd(fqt, fkt, vt, lg, dyt, b.dfq_t, b.dfk_t, b.dv_t, b.dlg_t, false, B,
-                              H, L, fw, dw, gla_rows(L, dw), gph, KG, nullptr, b.inner, eden, edel,
+                              H, L, fw, dw, dw, gph, KG, nullptr, b.inner, eden, edel,
                               nullptr, st)))
         return e;
       // dfq, dfk: this F tile's columns, summed over the D tiles
