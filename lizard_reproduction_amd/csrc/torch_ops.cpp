@@ -74,8 +74,8 @@ at::ScalarType grad_dtype(const std::vector<int64_t>& dtypes) {
 
 int padded(int64_t n) { return n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 256 ? 256 : 0; }
 
-// whether the walks take (F, D) directly: the forward's workspace then holds
-// segment records that the backward reuses
+// whether the walks take (F, D) directly (gla_fwd.hip's gla_dims_supported): the
+// forward's workspace then holds segment records that the backward reuses
 bool gla_native(int64_t nf, int64_t nd) {
   const int fp = padded(nf), dp = padded(nd);
   return fp && dp && dp <= 128 && (fp <= 128 || dp <= 64);
@@ -371,6 +371,7 @@ Tensor layer_step_rows(const Tensor& x, const std::vector<Tensor>& w, const Tens
 
 PYBIND11_MODULE(lizard_torch, m) {
   const auto nogil = py::call_guard<py::gil_scoped_release>();
+  m.def("gla_native", &gla_native);
   m.def("gla", &gla, nogil);
   m.def("swa", &swa, nogil);
   m.def("step_takes", &step_takes, nogil);

@@ -150,16 +150,11 @@ def _check_gate(what, fq, lg):
                          f"got {tuple(lg.shape)}")
 
 
-def _padded(n):
-    return next((p for p in (32, 64, 128, 256) if n <= p), None)
-
-
 def gla_native(nf, nd):
     """Whether the GLA walks take (F, D) directly (F <= 256, D <= 128, D <= 64
     when F > 128); past that the library runs them on tiles, and the
     forward's workspace holds tiles rather than segment states."""
-    fp, dp = _padded(nf), _padded(nd)
-    return fp is not None and dp is not None and dp <= 128 and (fp <= 128 or dp <= 64)
+    return _ops.load().gla_native(nf, nd)
 
 
 # gate_mode bits of the C ABI (include/lizard_hip.h)
