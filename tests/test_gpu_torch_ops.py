@@ -1,6 +1,7 @@
 """The C++ autograd nodes and decode step (csrc/torch_ops.cpp) against the Python
 ones they stand in for: the same bits over the forms the operators accept, and
-the same behaviour under the features that act on an autograd node."""
+the same behaviour under the features that act on an autograd node.  The products
+of few rows, summed in another order than torch's, within a tolerance."""
 import types
 
 import pytest
@@ -127,23 +128,30 @@ def test_changed_operands_second_backward_and_transforms_are_refused():
         kernels.gla(fq, fk, torch.autograd.forward_ad.make_dual(v, torch.ones_like(v)), lg)
 
 
-@pytest.mark.parametrize("heads, kv, dtype, rope_batched, window, prompt", [
-    (4, 2, torch.bfloat16, False, 16, 40), (4, 4, torch.float32, True, 64, 10),
-    (2, 1, torch.bfloat16, True, 5, 0)])
-def test_native_layer_step_equals_the_step_by_operators(monkeypatch, heads, kv, dtype, rope_batched,
-                                                        window, prompt):
+@pytest.mark.parametrize("heads, kv, dim, dtype, rope_batched, window, prompt", [
+    (4, 2, 64, torch.bfloat16, False, 16, 40), (4, 4, 64, torch.float32, True, 64, 10),
+    (2, 1, 64, torch.bfloat16, True, 5, 0), (4, 2, 128, torch.bfloat16, False, 16, 40),
+    (2, 2, 32, torch.float32, False, 7, 3)])
+def test_native_layer_step_equals_the_step_by_operators(monkeypatch, heads, kv, dim, dtype,
+                                                        rope_batched, window, prompt):
     """Prompt (none, shorter and longer than the window), then steps through the
-    ring's wrap: outputs, state and caches bit for bit."""
+    ring's wrap: outputs, state and caches bit for bit, the projections formed by
+    the modules on both sides."""
     torch.manual_seed(heads)
-    cfg = types.SimpleNamespace(hidden_size=64 * heads, num_attention_heads=heads,
+    monkeypatch.setattr(LizardAttention, "_step_rows", lambda *a: False)
+    native = []
+    step_native = LizardAttention._step_native
+    monkeypatch.setattr(LizardAttention, "_step_native",
+                        lambda *a: native.append(step_native(*a)) or native[-1])
+    cfg = types.SimpleNamespace(hidden_size=dim * heads, num_attention_heads=heads,
                                 num_key_value_heads=kv)
     layer = LizardAttention(cfg, 0, window=window, feature_dim=32).to("cuda", dtype)
     with torch.no_grad():
         for p in layer.parameters():
             p.normal_(0, 0.2)
     b, steps = 3, 9
-    x = torch.randn(b, prompt + steps, 64 * heads, device="cuda").to(dtype)
-    angle = torch.rand(prompt + steps, 64, device="cuda") * 6
+    x = torch.randn(b, prompt + steps, dim * heads, device="cuda").to(dtype)
+    angle = torch.rand(prompt + steps, dim, device="cuda") * 6
     cos, sin = angle.cos().to(dtype), angle.sin().to(dtype)
 
     def tables(lo, hi):
@@ -162,6 +170,7 @@ def test_native_layer_step_equals_the_step_by_operators(monkeypatch, heads, kv, 
         return outs + [cache.state, cache.k, cache.v]
     ours = run()
     theirs = _through_python(monkeypatch, run)
+    assert native == [True] * steps + [False] * steps
     for a, c in zip(ours, theirs):
         assert torch.equal(a, c)
 
@@ -185,15 +194,16 @@ def test_rows_linear_matches_the_product(rows, cols, sizes):
         assert ((y.double() - exact).abs() <= bound).all()
 
 
-def _decode_layer(batch=3):
+def _decode_layer(batch=3, heads=4):
     torch.manual_seed(5)
-    cfg = types.SimpleNamespace(hidden_size=256, num_attention_heads=4, num_key_value_heads=2)
+    cfg = types.SimpleNamespace(hidden_size=256, num_attention_heads=heads,
+                                num_key_value_heads=heads // 2)
     layer = LizardAttention(cfg, 0, window=8, feature_dim=32).to("cuda", torch.bfloat16)
     with torch.no_grad():
         for n, p in layer.named_parameters():
             p.normal_(0, 0.2 if n.startswith("phi") else 0.06)
     x = torch.randn(batch, 20, 256, device="cuda").bfloat16()
-    angle = torch.rand(20, 64, device="cuda") * 6
+    angle = torch.rand(20, 256 // heads, device="cuda") * 6
     return layer, x, (angle.cos().bfloat16(), angle.sin().bfloat16())
 
 
@@ -204,10 +214,10 @@ def _decode(layer, x, tables):
     return torch.cat(outs, 1), cache
 
 
-@pytest.mark.parametrize("batch", [1, 16, 17])
-def test_step_with_its_projections_matches_the_forward(batch):
-    """Sixteen sequences are the most the skinny products take."""
-    layer, x, tables = _decode_layer(batch)
+@pytest.mark.parametrize("batch, heads", [(1, 4), (16, 4), (17, 4), (3, 2)])
+def test_step_with_its_projections_matches_the_forward(batch, heads):
+    """Sixteen sequences are the most the skinny products take; head_dim 64 and 128."""
+    layer, x, tables = _decode_layer(batch, heads)
     assert layer._step_rows(x[:, :1]) == (batch <= 16)
     out, _ = _decode(layer, x, tables)
     with torch.no_grad():
