@@ -1363,6 +1363,28 @@ static int swa_ring_blocks(int BH, int L, int NS) {
   return best;
 }
 
+// Whether the ring is the faster form at 32 < d <= 64 (at 64 < d <= 128 it is
+// everywhere, 1.1 to 2.8 times), from 400 calls timed in both; B*H = 1 to 1000, L =
+// 128 to 8192, W = 70 to 289, d = 36, 48 and 64 (us, the ring and the two kernels):
+// * one round of workgroups: the eight waves (NS <= 6) always.  A step of twelve
+//   takes 2.5 to 3.1 us, so a segment has to be long beside its halo of NS - 1
+//   blocks (B*H = 32 L = 2048 W = 289, NB = 8, 62 against 49; B*H = 64 L = 2000 W =
+//   250, NB = 16, 78 against 88), or a whole row, or the row end soon after the halo
+//   (B*H = 128 L = 256 26 against 28);
+// * several rounds: where enough of the workgroups' steps, one for their start
+//   included, are blocks of their own and not halos or a last round's empty places
+//   (B*H = 300 L = 700 W = 289 157 against 142, half of them; B*H = 512 L = 300 73
+//   against 91), and not for rows of up to 128 tokens (B*H = 512 L = 128 32 and,
+//   with eight waves, 28 against 26).
+static bool swa_ring_pays(int BH, int L, int NS) {
+  const int nsub = (L + 31) / 32, cus = device_geom().cus, NB = swa_ring_blocks(BH, L, NS);
+  const long long wgs = (long long)BH * ((nsub + NB - 1) / NB), rounds = (wgs + cus - 1) / cus;
+  const bool eight = NS <= swa_ring_max_ns(8);
+  if (rounds == 1) return eight || NB == nsub || 5 * NB >= 7 * NS || nsub <= NS + 2;
+  const int steps = NB + NS - 1 < nsub ? NB + NS - 1 : nsub;
+  return nsub > 4 && 100LL * BH * nsub >= (eight ? 52 : 57) * rounds * cus * (steps + 1);
+}
+
 template <int DP, int R, typename OutT, bool VEC>
 static hipError_t launch_swa_bwd_ring(const void* q, const void* k, const void* v,
                                       const float* meta, int n_meta, const float* lse,
@@ -1400,17 +1422,18 @@ static hipError_t launch_swa_bwd_t(const void* q, const void* k, const void* v, 
   }
   // wider windows at 32 < d <= 64 and all windows at 64 < d <= 128: the ring
   // walk, where its waves cover the window's key blocks (W <= 161, and W <= 289
-  // at d <= 64).  Against the two kernels below (B=4 H=32 L=4096, us): d = 64
-  // W = 96 152 against 225, W = 289 290 against 351; d = 128 W = 1 214 against
-  // 378, W = 161 276 against 713.  At d <= 32 they stay the faster ones: W = 16
-  // 102 against 86, W = 64 115 against 107.
+  // at d <= 64) and it is the faster form (swa_ring_pays).  Against the two
+  // kernels below (B=4 H=32 L=4096, us): d = 64 W = 96 152 against 225, W = 289 290
+  // against 351; d = 128 W = 1 214 against 378, W = 161 276 against 713.  At d <= 32
+  // they stay the faster ones: W = 16 102 against 86, W = 64 115 against 107.
   if constexpr (DP == 64 || DP == 128) {
     const int NS = swa_ring_ns(W);
-    if (NS <= swa_ring_max_ns(8))
+    const bool ring = DP == 128 || (NS <= swa_ring_max_ns(12) && swa_ring_pays(BH, L, NS));
+    if (ring && NS <= swa_ring_max_ns(8))
       return launch_swa_bwd_ring<DP, 8, OutT, VEC>(q, k, v, meta, n_meta, lse, dy, dq, dk, dv,
                                                    dmeta_part, dmeta, BH, L, d, W, scale, KG, st);
     if constexpr (DP <= 64) {
-      if (NS <= swa_ring_max_ns(12))
+      if (ring)
         return launch_swa_bwd_ring<DP, 12, OutT, VEC>(q, k, v, meta, n_meta, lse, dy, dq, dk, dv,
                                                       dmeta_part, dmeta, BH, L, d, W, scale, KG,
                                                       st);

@@ -129,7 +129,13 @@ def test_swa_many_sinks_match_oracle(sinks, dim):
     (640, 161, 128, 2, False), (640, 162, 128, 2, False), (641, 162, 64, 2, False),
     (450, 289, 40, 2, False), (450, 290, 64, 2, False), (300, 64, 128, 2, True),
     (31, 128, 128, 2, False), (130, 1, 96, 2, False), (290, 128, 30, 3, False),
-    (300, 200, 20, 2, True), (1100, 128, 100, 64, False)])
+    (300, 200, 20, 2, True), (1100, 128, 100, 64, False),
+    # twelve waves where the row ends within the halo (nine and twelve blocks), the
+    # two kernels a block longer; long segments; whole rows in full rounds of
+    # workgroups, and two thirds empty last rounds; eight waves above 128 tokens
+    (288, 162, 64, 2, False), (289, 162, 64, 2, True), (384, 289, 40, 2, True),
+    (385, 289, 64, 2, False), (450, 162, 64, 230, False), (300, 250, 64, 500, False),
+    (300, 250, 64, 270, False), (128, 100, 64, 300, False), (129, 100, 36, 500, False)])
 def test_swa_wide_window_backward_matches_oracle(length, window, dim, heads, fp32):
     inputs = swa_inputs(length, batch=1, heads=heads, dim=dim, seed=window)
     if fp32:
