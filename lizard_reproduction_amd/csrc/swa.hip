@@ -27,6 +27,7 @@
 // straight from the accumulator registers.  Consecutive workgroups of one
 // (b, h) are mapped to one XCD so that the tiles they share hit one L2.
 #include <initializer_list>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -1627,21 +1628,21 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
     // flight, the first values' rows alongside the keys'
     constexpr int KP = 256 / CG, PASS = 4;
     const int cg = tid % CG, kg = tid / CG, lane = tid & 63, wave = tid >> 6;
-    auto rows = [&](bf16x8 (&x)[PASS], const bf16* cache, const bf16* fresh, int i0) {
+    auto rows = [&](auto passes, bf16x8 (&x)[PASS], const bf16* cache, const bf16* fresh, int i0) {
 #pragma unroll
-      for (int p = 0; p < PASS; ++p) {
+      for (int p = 0; p < decltype(passes)::value; ++p) {
         const int i = min(i0 + KP * p + kg, n - 1);   // a valid row; unused past n
         x[p] = *reinterpret_cast<const bf16x8*>(row(cache, fresh, i) + 8 * cg);
       }
     };
     const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(q + at0 + 8 * cg);
     bf16x8 v8[PASS];
-    for (int i0 = 0; i0 < n; i0 += KP * PASS) {
+    auto scores = [&](auto passes, int i0) {
       bf16x8 k8[PASS];
-      rows(k8, kb, ap.k_new, i0);
-      if (i0 == 0) rows(v8, vb, ap.v_new, 0);
+      rows(passes, k8, kb, ap.k_new, i0);
+      if (i0 == 0) rows(passes, v8, vb, ap.v_new, 0);
 #pragma unroll
-      for (int p = 0; p < PASS; ++p) {
+      for (int p = 0; p < decltype(passes)::value; ++p) {
         float s = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) s += to_f32(q8[e]) * to_f32(k8[p][e]);
@@ -1654,7 +1655,13 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
           if (cg == 0) w[i] = s;
         }
       }
-    }
+    };
+    // keys of one pass (a sequence's first positions, small windows): no loads of
+    // the other three, which B*H = 8192, d = 32 paid with 24.0 for 21.8 us at position 0
+    if (n <= KP)
+      scores(std::integral_constant<int, 1>{}, 0);
+    else
+      for (int i0 = 0; i0 < n; i0 += KP * PASS) scores(std::integral_constant<int, PASS>{}, i0);
     const float m = decode_max256(sh, mx);   // also orders the score writes
     float l = 0.f;
     for (int i = tid; i < n; i += 256) {
@@ -1668,7 +1675,7 @@ __global__ __launch_bounds__(256) void swa_decode_kernel(
     const float inv = 1.f / (ls + l);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int i0 = 0; i0 < n; i0 += KP * PASS) {
-      if (i0 > 0) rows(v8, vb, ap.v_new, i0);
+      if (i0 > 0) rows(std::integral_constant<int, PASS>{}, v8, vb, ap.v_new, i0);
 #pragma unroll
       for (int p = 0; p < PASS; ++p) {
         const int i = i0 + KP * p + kg;
