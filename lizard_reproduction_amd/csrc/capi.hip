@@ -298,8 +298,8 @@ extern "C" int lz_gla_bwd(const void* fq, const void* fk, const void* v, const f
 // ---------------------------------------------------------------------------
 // `scratch` holds the state records of lz_gla_fwd_noalloc's segment split
 // (the only device memory the forward needs beyond its inputs and output).
-// Its size covers every split the forward makes on a whole MI355X: the
-// largest, 64.75 MiB, is F = 256, D = 64 at B*H = 255.  Every GPU the library
+// Its size covers every split the forward makes on a whole MI355X, twice over:
+// the largest, 32.5 MiB, is F = 256, D = 64 at B*H = 128.  Every GPU the library
 // runs on holds its own copy until the process ends.
 static_assert(LZ_GLA_FWD_NOALLOC_MAX_BYTES % 256 == 0, "scratch size");
 static __device__ __align__(256) float scratch[LZ_GLA_FWD_NOALLOC_MAX_BYTES / sizeof(float)];

@@ -456,8 +456,8 @@ __device__ __forceinline__ void fold_records(float* __restrict__ out,
 // for at most 4 segments per row, in the walks that have a folding variant
 // (whole 16-byte rows).  Measured: with 4 segments (F = D = 128, B = 4, L =
 // 2048) and 3 (F = 256, D = 64, the config-5 layer) the fold took 6-11 us off a
-// fwd+bwd; at F = D = 64 with 4, 12.7 -> 10.4 us of a short forward (H = 4, L =
-// 256), 23.9 -> 20.1 us (B = 8, H = 16, L = 512), 49.3 -> 45.7 us (B = 4, H = 32,
+// fwd+bwd; at F = D = 64 with 4, 11.4 -> 10.0 us of a short forward (H = 4, L =
+// 256), 23.7 -> 19.9 us (B = 8, H = 16, L = 512), 49.0 -> 45.3 us (B = 4, H = 32,
 // L = 2048) and 2 us of each backward.  With 8 (B = 2, H = 32) it measured 1 us
 // slower; with 16 (B = 1, L = 2048) its passes over 15 records of each walk cost
 // more than the scan launch.  The state passes leave the records unscanned

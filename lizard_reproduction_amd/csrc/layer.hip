@@ -467,7 +467,7 @@ struct ProBwd {
   // feature groups: two where a row has two or more feature tiles and the
   // per-group dx shares fit the LDS: each group's at head_dim <= 64, one at a
   // time at head_dim 128 in bf16 (DX_TURNS; fp32's W and x tiles leave no room).
-  // With one group a wave held 465 registers there, one wave per SIMD: B=1
+  // With one group a wave held 471 to 507 registers there, one wave per SIMD: B=1
   // L=4096, 32/8 heads, 128 features 208 -> 142 us, 64 features 116 -> 93 us
   static constexpr bool DX_TURNS = HT == 4 && FT >= 2 && !C::SPLIT;
   static constexpr int NWF = (FT >= 2 && HT <= 2) || DX_TURNS ? 2 : 1;

@@ -8,10 +8,11 @@
 // stream, and the graph node.  The nodes and layer_step make the launches that
 // Python made on the same operands, with the same bits; layer_step_rows forms the
 // projections with rows.hip's products, whose sums run in another order than the
-// library's (each rounded to bf16 once, as there).  Measured for a forward and backward of one sequence (H = 32, L = 2048,
-// d = 64), where the kernels take 75 and 35 us: gla 138 -> 87 us, swa 120 -> 75 us;
-// a short forward (H = 4, L = 256) 17.5 -> 12.8 us; a decode step of the layer (B =
-// 4, hidden 2048) 201 -> 132 us with torch's projections, 48 us with rows.hip's.
+// library's (each rounded to bf16 once, as there).  Measured for a forward and
+// backward of one sequence (H = 32, L = 2048, d = 64), where the kernels take 75 and
+// 35 us: gla 138 -> 87 us, swa 120 -> 75 us; a short forward (H = 4, L = 256) 17.6 ->
+// 11.4 us (10.0 since its walks fold the segment records); a decode step of the layer
+// (B = 4, hidden 2048) 201 -> 132 us with torch's projections, 48 us with rows.hip's.
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 

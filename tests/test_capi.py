@@ -220,10 +220,10 @@ def test_layer_prologue_workspace_sizes(lib, b, length, heads, kv, hd, f):
 
 
 def segments(bh, length, f=64, chunk=64):
-    """The library's split of each (b, h) sequence into segments (so that
-    B*H*segments fills the GPU: 512 workgroups up to F = 128, 256 beyond,
-    where the split is then doubled and each walk takes two segments):
-    returns (segments, chunks per segment)."""
+    """The library's split of each (b, h) sequence into segments where B*H divides
+    the GPU's workgroups or the sequence is short (so that B*H*segments fills the
+    GPU: 512 workgroups up to F = 128, 256 beyond, where the split is then doubled
+    and each walk takes two segments): returns (segments, chunks per segment)."""
     wide = padded(f) > 128
     target = 256 if wide else 512
     nt = -(-length // chunk)
