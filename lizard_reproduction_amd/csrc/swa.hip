@@ -1365,7 +1365,7 @@ static int swa_ring_blocks(int BH, int L, int NS) {
 }
 
 // Whether the ring is the faster form at 32 < d <= 64 (at 64 < d <= 128 it is
-// everywhere, 1.1 to 2.8 times), from 400 calls timed in both; B*H = 1 to 1000, L =
+// everywhere, 1.1 to 2.8 times), from 300 calls timed in both; B*H = 1 to 1000, L =
 // 128 to 8192, W = 70 to 289, d = 36, 48 and 64 (us, the ring and the two kernels):
 // * one round of workgroups: the eight waves (NS <= 6) always.  A step of twelve
 //   takes 2.5 to 3.1 us, so a segment has to be long beside its halo of NS - 1
